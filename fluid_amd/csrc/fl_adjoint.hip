@@ -1144,6 +1144,7 @@ static int adj_step(Vjp* J, const float* tp, int K, float dt) {
     hipLaunchKernelGGL(k_mirror_in, gr, bl, 0, st, g, c->S, L[L_OU], L[L_OV], m->U, m->V, m->p);
     FL_HIP(hipGetLastError());
     m->prm.pressure_damping = P.pressure_damping;
+    m->prm.relaxation = P.relaxation;
     m->prm.block_sweeps = P.block_sweeps;
     m->prm.handoff_lag = P.handoff_lag;
     m->prm.block_cols = P.block_cols;

@@ -34,9 +34,9 @@ static void batch_free(Batch* B) {
   for (Ctx* c : B->members) free_ctx(c);
   for (float* p : B->pool)
     if (p) (void)hipFree(p);
-  for (void* p : {(void*)B->flags_pool, (void*)B->diag_pool, (void*)B->keep_pool, (void*)B->ctrl_pool, (void*)B->maxdiv_pool,
+  for (void* p : {(void*)B->flags_pool, (void*)B->mask_pool, (void*)B->keep_pool, (void*)B->ctrl_pool, (void*)B->maxdiv_pool,
                   (void*)B->d_sims, (void*)B->d_cells, (void*)B->d_rings, (void*)B->d_tiles, (void*)B->kout,
-                  (void*)B->gout, (void*)B->prog, (void*)B->ticket, (void*)B->d_omega, (void*)B->d_src,
+                  (void*)B->gout, (void*)B->kinit, (void*)B->d_skews, (void*)B->ticket, (void*)B->d_omega, (void*)B->d_src,
                   (void*)B->d_src_seg, (void*)B->d_src_sim, (void*)B->d_ekeys, (void*)B->d_evals,
                   (void*)B->d_eseg, (void*)B->d_esim})
     if (p) (void)hipFree(p);
@@ -294,9 +294,7 @@ static int batch_update(Batch* B, float dt) {
 }
 
 // ---- autotuning of the Gauss-Seidel tile depth ---------------------------------------------
-// Tile shapes the autotuners time: sweeps per tile (2, 4, 8, 16), columns per block (4, 8,
-// 16) and handoff publication (1 on time, 2 a block late, 3 halfway), ordered so that the
-// layout changes only with the first two.
+// Tile shapes the autotuners time: sweeps per tile (2, 4, 8, 16) and columns per block (4, 8).
 // Shallow tiles multiply the handoff traffic and the tile count, so 2-deep tiles are tried
 // only where the 8-deep tiling has at most two tiles per CU (the critical path, not the CUs'
 // throughput, bounds such solves).
@@ -307,8 +305,7 @@ static std::vector<TuneShape> tune_shapes(long long tiles8, int cus) {
   std::vector<TuneShape> v;
   for (int tk : {2, 4, 8, 16}) {
     if (tk == 2 && tiles8 > 2LL * cus) continue;
-    for (int blk : {4, 8, 16})
-      for (int lag : {1, 2, 3}) v.push_back(TuneShape{tk, blk, lag});
+    for (int blk : {4, 8}) v.push_back(TuneShape{tk, blk, 1});
   }
   return v;
 }
@@ -393,13 +390,13 @@ int fl_batch_create(int n, const int* widths, const int* heights, float density,
     batch_free(B);
     return berr(code, m);
   };
-  size_t ncells = 0, ndiag = 0, nkeep = 0;
+  size_t ncells = 0, nmask = 0, nkeep = 0;
   for (int e = 0; e < n; e++) {
     if (widths[e] < 1 || heights[e] < 1) return fail(FL_ERR_INVALID_ARG, "member sizes must be >= 1");
     if ((int64_t)(widths[e] + 2) * (heights[e] + 2) > (int64_t)1 << 28)
       return fail(FL_ERR_INVALID_ARG, "member grid too large (more than 2^28 cells)");
     ncells += (size_t)(widths[e] + 2) * (heights[e] + 2);
-    ndiag += (size_t)(widths[e] + heights[e] + 3) * (widths[e] + 2);
+    nmask += mask_bytes(widths[e] + 2, heights[e] + 2);
     nkeep += (size_t)(widths[e] + 2) * ((heights[e] + 2 + 63) / 64);
   }
   if (ncells * NBUF > ((size_t)1 << 31) * 8) return fail(FL_ERR_INVALID_ARG, "batch too large");
@@ -410,19 +407,19 @@ int fl_batch_create(int n, const int* widths, const int* heights, float density,
     if (hipMalloc(&B->pool[k], sizeof(float) * ncells) != hipSuccess) return fail(FL_ERR_HIP, "hipMalloc pool");
     (void)hipMemsetAsync(B->pool[k], 0, sizeof(float) * ncells, B->stream);
   }
-  if (hipMalloc(&B->flags_pool, ncells) != hipSuccess || hipMalloc(&B->diag_pool, ndiag) != hipSuccess ||
+  if (hipMalloc(&B->flags_pool, ncells) != hipSuccess || hipMalloc(&B->mask_pool, nmask) != hipSuccess ||
       hipMalloc(&B->keep_pool, sizeof(uint32_t) * nkeep) != hipSuccess ||
       hipMalloc(&B->ctrl_pool, sizeof(int32_t) * 4 * n) != hipSuccess ||
       hipMalloc(&B->maxdiv_pool, sizeof(uint32_t) * 2 * MEMBER_NMAX * n) != hipSuccess ||
       hipMalloc(&B->d_sims, sizeof(SimDesc) * n) != hipSuccess ||
       hipMalloc(&B->d_omega, sizeof(float) * MEMBER_NMAX) != hipSuccess)
     return fail(FL_ERR_HIP, "hipMalloc batch");
-  (void)hipMemsetAsync(B->diag_pool, 0, ndiag, B->stream);
+  (void)hipMemsetAsync(B->mask_pool, 0, nmask, B->stream);
   (void)hipMemsetAsync(B->ctrl_pool, 0, sizeof(int32_t) * 4 * n, B->stream);
   (void)hipMemsetAsync(B->maxdiv_pool, 0, sizeof(uint32_t) * 2 * MEMBER_NMAX * n, B->stream);
   std::vector<CellItem> cells;
   std::vector<RingItem> rings;
-  size_t off = 0, doff = 0, koff = 0;
+  size_t off = 0, moff = 0, koff = 0;
   for (int e = 0; e < n; e++) {
     Ctx* c = new Ctx();
     c->batch = B;
@@ -441,7 +438,7 @@ int fl_batch_create(int n, const int* widths, const int* heights, float density,
                             &c->U2, &c->V2, &c->M2, &c->T0, &c->T1, &c->T2, &c->T3};
     for (int k = 0; k < NBUF; k++) *fields[k] = B->pool[k] + off;
     c->flags = B->flags_pool + off;
-    c->flags_diag = B->diag_pool + doff;
+    c->masks = B->mask_pool + moff;
     c->keep = B->keep_pool + koff;
     c->d_ctrl = B->ctrl_pool + 4 * e;
     c->d_maxdiv = B->maxdiv_pool + (size_t)2 * MEMBER_NMAX * e;
@@ -455,7 +452,7 @@ int fl_batch_create(int n, const int* widths, const int* heights, float density,
     const int m = std::max(c->NX, c->NY);
     for (int blk = 0; blk < (m + 255) / 256; blk++) rings.push_back(RingItem{e, blk});
     off += c->N;
-    doff += (size_t)(c->NX + c->NY - 1) * c->NX;
+    moff += mask_bytes(c->NX, c->NY);
     koff += (size_t)c->NX * ((c->NY + 63) / 64);
   }
   {  // item k runs on XCD k % 8: give each XCD a contiguous run of the list

@@ -371,9 +371,8 @@ void free_ctx(Ctx* c) {
     for (auto** b : bufs)
       if (*b) (void)hipFree(*b);
     if (c->flags) (void)hipFree(c->flags);
-    if (c->flags_diag) (void)hipFree(c->flags_diag);
+    if (c->masks) (void)hipFree(c->masks);
     if (c->keep) (void)hipFree(c->keep);
-    if (c->snap_hint) (void)hipHostFree(c->snap_hint);
     if (c->d_ctrl) (void)hipFree(c->d_ctrl);
     if (c->d_maxdiv) (void)hipFree(c->d_maxdiv);
   }
@@ -558,14 +557,10 @@ int fl_create(float density, int width, int height, float h, fl_ctx** out) {
   if ((e = hipMalloc(&c->flags, c->N)) != hipSuccess) return fail(e, "hipMalloc flags");
   if ((e = hipMalloc(&c->keep, sizeof(uint32_t) * c->NX * ((c->NY + 63) / 64))) != hipSuccess)
     return fail(e, "hipMalloc keep");
-  if ((e = hipHostMalloc((void**)&c->snap_hint, 64, hipHostMallocCoherent)) != hipSuccess)
-    return fail(e, "hipHostMalloc hint");
-  *c->snap_hint = 0;
-  if ((e = hipMalloc(&c->flags_diag, (size_t)(c->NX + c->NY - 1) * c->NX)) != hipSuccess)
-    return fail(e, "hipMalloc flags_diag");
+  if ((e = hipMalloc(&c->masks, mask_bytes(c->NX, c->NY))) != hipSuccess) return fail(e, "hipMalloc masks");
   // entries off the grid stay zero for the context's lifetime
-  if ((e = hipMemsetAsync(c->flags_diag, 0, (size_t)(c->NX + c->NY - 1) * c->NX, c->stream)) != hipSuccess)
-    return fail(e, "hipMemset flags_diag");
+  if ((e = hipMemsetAsync(c->masks, 0, mask_bytes(c->NX, c->NY), c->stream)) != hipSuccess)
+    return fail(e, "hipMemset masks");
   if ((e = hipMalloc(&c->d_ctrl, 64)) != hipSuccess) return fail(e, "hipMalloc ctrl");
   if ((e = hipMemsetAsync(c->d_ctrl, 0, 64, c->stream)) != hipSuccess) return fail(e, "hipMemset ctrl");
   if ((e = hipMalloc(&c->d_red, 64)) != hipSuccess) return fail(e, "hipMalloc red");
@@ -764,11 +759,11 @@ int fl_get_gs_layout(fl_ctx* ctx, fl_gs_layout* out) {
   CTX_CHECK(ctx);
   if (!out) return err(FL_ERR_INVALID_ARG, "null argument");
   const GsWork& W = C_OF(ctx)->gs;
-  if (W.defer < 0) return err(FL_ERR_INVALID_ARG, "no temporal-blocked solve has run on this context");
+  if (W.lag == 0) return err(FL_ERR_INVALID_ARG, "no temporal-blocked solve has run on this context");
   *out = fl_gs_layout{};
   out->sweeps_per_tile = W.tk;
   out->cols_per_block = W.blk;
-  out->handoff_lag = W.defer + 1;
+  out->handoff_lag = W.lag;
   out->row_tiles = W.G;
   out->sweep_blocks = W.KB;
   out->steps_per_tile = W.rows;

@@ -3,25 +3,41 @@
 //
 // Cell (i,j) of sweep k needs (i-1,j,k), (i,j-1,k), (i+1,j,k-1), (i,j+1,k-1) and (i,j,k-1).
 // With skewed rows i' = i + k these become forward dependences in (i', k), plus a
-// j-lag of at most one column. A workgroup owns a tile of 64 skewed rows (the lanes a)
-// by TK sweeps (the waves b) and marches along j: at step s, thread (a,b) updates cell
-// (i = i0 + a - b, j = s - a - b) of sweep k0 + b. Every face then travels between
-// neighbouring threads:
+// j-lag of at most one column. A tile is 64 skewed rows (the lanes a) by TK = W x S sweeps;
+// a wave holds S of them in registers and marches along j: at step s it updates, for each of
+// its sweeps b, the cells (i = i0 + a - b, j = s - a - b) of sweep k0 + b. Every face then
+// travels as follows:
 //   U right face, after the update, -> (a+1, b)   at s+1   (DPP wave_shr:1)
-//   U left face                     -> (a, b+1)   at s+1   (LDS)
-//   V bottom face and p             -> (a+1, b+1) at s+1   (LDS; p is used at s+2)
+//   U left face                     -> (a, b+1)   at s+1   (register; LDS to the next wave)
+//   V bottom face and p             -> (a+1, b+1) at s+1   (DPP wave_shr:1; p is used at s+2)
 //   V top face                      -> (a, b) itself       (register)
-// so the state of a tile lives in registers and LDS for all its TK sweeps; HBM sees the
-// initial U,V once, the final U,V,p once, and per tile and column the boundary faces
-// handed to the next tile along i' (G stream) and the next block of sweeps (K stream).
-// Tiles run as a persistent kernel in ticket order (a topological order of the tile
-// graph); a consumer waits on its producers' published progress, in blocks of 8 columns.
-// Handoff data and progress counters are accessed only with agent-scope relaxed atomic
-// loads and stores (device-coherent accesses, global_load/store sc1), so neither side
-// needs an L2 writeback or invalidate; the producer waits for its data stores to
-// complete before it stores the new progress value (publish_rows: a full wait at the next
-// block, or a counted wait one block later), and consumers issue their data loads only after
-// observing it.
+// Within a step the sweeps run from the last to the first, so each takes what its predecessor
+// left in registers at the step before, and the S updates of a step are independent: a wave
+// needs no barrier and no LDS round trip between its sweeps. Only a wave's first sweep (from the
+// wave before it) and its lane 0 (from the tile one row-tile up) read LDS, two steps ahead.
+//
+// The solve is a wavefront over a chain of dependent steps, so its time is steps times the time
+// of a step, not memory or arithmetic rate; and a step is the issue of one wave's instructions: a
+// lone wave issues an independent vector instruction every 4.7 cycles, a dependent one after 8,
+// a 16-byte LDS write takes 28 and a 4-byte one 16 (measured). So a step is about 15 vector
+// instructions per sweep and the few LDS accesses around them: 280 cycles for one sweep to a
+// wave, 340 for two, 530 for four, where one sweep a wave with a barrier a step took 640.
+//
+// The waves of a workgroup run one block of B steps apart, with one barrier per block: wave
+// w runs block n while wave w-1 runs block n+1 into the other half of their LDS buffer. Between
+// tiles the boundary goes through global memory: per step the three faces and p of lane 63 of
+// each sweep (the G stream, for the tile one row-tile up) and the last wave's 64 lanes (the K
+// stream, for the next TK sweeps). Each cell's values are one 16-byte word with a tag, the number
+// of the solve, in each half, and the consumer loads the words until they carry the tag of this
+// solve. So a handoff costs one trip of the data: no wait for stores, no progress counters, no
+// polls beside the loads themselves. A block's words are loaded while the block before it runs.
+// Tiles run as a persistent kernel in ticket order (a topological order of the tile graph), so
+// whatever a workgroup waits for was taken earlier by a workgroup that runs. k_gs_skew lays the
+// initial state out as K-stream words and k_gs_unskew takes the last sweep's back, so tiles
+// read and write nothing but words, whole lines at a time.
+//
+// Solves, start of the change to this form -> now: 256^2 40 sweeps 0.49 -> 0.21 ms, 300x251 8
+// sweeps 0.42 -> 0.14, 512^2 200 sweeps 1.32 -> 0.64, 4096^2 200 sweeps 10.5 -> 5.7.
 //
 // Cells outside the interior or solid pass their faces through unchanged, exactly like
 // the skipped cells of the serial loop. Faces no interior cell touches keep their input
@@ -31,6 +47,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -40,7 +57,7 @@
 namespace fl {
 
 static constexpr int LANES = 64;
-static constexpr int SPIN_LIMIT = 1 << 22;     // bounded wait (about a second); then error and continue
+static constexpr int SPIN_LIMIT = 1 << 20;     // bounded wait (about a second); then error and continue
 
 // One launch of the solve (main run or early-exit re-run).
 struct GsRun {
@@ -50,11 +67,9 @@ struct GsRun {
   int K;
   int32_t* ticket;
   const int32_t* rerun;  // re-run launch only: nonzero when some simulation asked for one
+  const int32_t* solve;  // the number of this solve, from which its tags are made
   const float* omega;
   float damping;
-  int rPin, rPout;    // roles of the initial p (read; < 0: p starts at zero) and of the solve's p
-  int defer;          // when handoff rows are published (publish_rows below): 0 at the next
-                      // block's start, 1 one block later, 2 halfway through the next block
 };
 
 __device__ __forceinline__ bool tile_empty(int g, int kb, int K, int TK, int NX) {
@@ -65,459 +80,653 @@ __device__ __forceinline__ bool tile_empty(int g, int kb, int K, int TK, int NX)
   return rmax < 0 || rmin > NX - 1;
 }
 
-// Device-coherent (agent scope) accesses of the handoff buffers.
-__device__ __forceinline__ float ld_dev(const float* p) {
-  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A handoff word: a left or right U face, a bottom V face and p with the solve's tag, 16 bytes.
+// Each 8-byte half carries the tag's 16 bits (and half of V), so a consumer that loads the word
+// while it is being written sees for each half whether it is this solve's; only the 8-byte halves
+// have to arrive whole. Words are written once per solve, so the tag they hold before is that of one of the
+// last solves. Device-coherent accesses (sc1), so that neither side needs a cache writeback or
+// invalidate.
+typedef uint32_t word4 __attribute__((ext_vector_type(4)));
+static constexpr int SC1 = 16, VOLATILE_OP = (int)0x80000000;  // cache policy of the buffer intrinsics
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t word_buffer(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffff, 0x00027000);
 }
-__device__ __forceinline__ void st_dev(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ word4 ld_word(__amdgpu_buffer_rsrc_t b, uint32_t byte) {
+  return __builtin_amdgcn_raw_buffer_load_b128(b, byte, 0, SC1 | VOLATILE_OP);
 }
-// One handoff entry (U, V, p) stored as three planes of `stride` floats.
-__device__ __forceinline__ float4 ld_dev3(const float* p, int stride) {
-  return make_float4(ld_dev(p), ld_dev(p + stride), ld_dev(p + 2 * stride), 0.0f);
+__device__ __forceinline__ void st_word(__amdgpu_buffer_rsrc_t b, uint32_t byte, float u, float v, float p, uint32_t tag) {
+  word4 w;
+  w.x = __float_as_uint(u);
+  w.y = (__float_as_uint(v) & 0xffffu) | (tag << 16);
+  w.z = __float_as_uint(p);
+  w.w = __builtin_amdgcn_alignbit(tag, __float_as_uint(v), 16);
+  __builtin_amdgcn_raw_buffer_store_b128(w, b, byte, 0, SC1);
 }
-// Wait until every store this wave issued has been acknowledged by the memory system.
-__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Wait until at most N of this wave's vector memory operations are in flight. The wave's
-// stores retire in issue order, so when at least N stores were issued after a given store,
-// that store is complete once this returns (loads issued in between only lengthen the wait).
-template <int N> __device__ __forceinline__ void wait_stores_but() {
-  static_assert(N >= 0 && N <= 63, "vmcnt is a 6-bit count");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ int ld_prog(const int32_t* p) {
+// Zero in the upper 16 bits when both halves carry the tag.
+__device__ __forceinline__ uint32_t word_tag(word4 w, uint32_t tag) { return (w.y ^ (tag << 16)) | (w.w ^ (tag << 16)); }
+__device__ __forceinline__ float word_u(word4 w) { return __uint_as_float(w.x); }
+__device__ __forceinline__ float word_v(word4 w) { return __uint_as_float(__builtin_amdgcn_perm(w.w, w.y, 0x05040100u)); }
+__device__ __forceinline__ float word_p(word4 w) { return __uint_as_float(w.z); }
+__device__ __forceinline__ int ld_err(const int32_t* p) {
   return __hip_atomic_load(const_cast<int32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Wait until producer progress reaches what a block needs: seen[x] >= need[x] for the G and K
-// producers (need 0: nothing to wait for). The counters still short are loaded together, so a
-// block whose producers have both published costs one round trip. The wait is bounded: after
-// SPIN_LIMIT polls, or as soon as another wait of this simulation has expired (err set), it
-// sets err and gives up, so a solve whose producers stall ends within about a second with
-// FL_ERR_INTERNAL instead of every later wait running out its own limit.
-__device__ __forceinline__ void wait_producers(const int32_t* pg, int needG, const int32_t* pk, int needK, int& seenG,
-                                               int& seenK, int32_t* err) {
-  for (int it = 0;; it++) {
-    const bool wG = seenG < needG, wK = seenK < needK;
-    if (!wG && !wK) return;
-    if (it > SPIN_LIMIT || ((it & 255) == 255 && ld_prog(err) != 0)) {
-      atomicOr(err, 1);
-      seenG = max(seenG, needG);
-      seenK = max(seenK, needK);
-      return;
-    }
-    if (it) __builtin_amdgcn_s_sleep(2);
-    int vG = 0, vK = 0;
-    if (wG) vG = ld_prog(pg);
-    if (wK) vK = ld_prog(pk);
-    if (wG) seenG = vG;
-    if (wK) seenK = vK;
-  }
 }
 
 __device__ __forceinline__ const SimDesc& sim_desc(const OneSim& m, int) { return m.d; }
 __device__ __forceinline__ const SimDesc& sim_desc(const ManySims& m, int e) { return m.sims[e]; }
 
-// TK sweeps per tile (one wave each), BLK columns per staging and publish block (BLK divides 64).
-// SNAP: the main run also writes the first sweep's U, V, p to T0, T1, T2, so that an early exit
-// after sweep 0 needs no re-run (k_gs_take_first); a separate instantiation, so the usual kernel
-// carries none of its code or registers.
-// 8-sweep tiles of up to 8 columns per block are held to 128 VGPRs (at least 4 waves per SIMD),
-// so two workgroups share a CU: the batched kernel needs 137 otherwise and fits without spills.
-template <int TK, int BLK, class M, bool SNAP = false>
-__global__ __launch_bounds__(TK * LANES, (TK == 8 && BLK <= 8) ? 4 : 1) void k_gs_wave(M m, GsRun R) {
-  static_assert(LANES % BLK == 0, "progress is published in whole blocks that divide the tile height");
+// Lane a takes lane a-1's v; lane 0 takes its own `first`.
+__device__ __forceinline__ float from_lane_below(float first, float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138, 0xF, 0xF, false));
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(uniform(__float_as_int(v))); }
+
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // four floats at any word address
+
+// S sweeps of a wave, in registers. What each sweep left at the step before: UrO the right U
+// face, UlO, VbO, pO the left U face, bottom V face and p; Vt the top V face (the next column's
+// bottom face); pn the p of the next column.
+template <int S> struct Sweeps {
+  float UrO[S], UlO[S], VbO[S], pO[S], Vt[S], pn[S], md[S], om[S];
+};
+
+// The weights of a cell by the mask of its fluid neighbours (the index, 0 for a cell that no
+// sweep updates), in LDS: what the update multiplies its faces by, 1/s, s, and a mask for div.
+// An inactive cell has q = -0 and weights +0, and x + (+0 * -0) is x to the bit.
+struct CellW {
+  float4 w;  // -sx0, sx1, -sy0, sy1
+  float4 d;  // 1/s, s, bits: all ones where updated, unused
+};
+__device__ __forceinline__ CellW cell_weights(int mask) {
+  const float x0 = (mask & 1) ? 1.0f : 0.0f, x1 = (mask & 2) ? 1.0f : 0.0f, y0 = (mask & 4) ? 1.0f : 0.0f,
+              y1 = (mask & 8) ? 1.0f : 0.0f;
+  const float s = x0 + x1 + y0 + y1;
+  CellW c;
+  c.w = mask ? make_float4(-x0, x1, -y0, y1) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  c.d = make_float4(mask ? 1.0f / s : 1.0f, mask ? s : 1.0f, __uint_as_float(mask ? 0xffffffffu : 0u), 0.0f);
+  return c;
+}
+
+// One step's cells of a wave's S sweeps: their faces, p and cells before and after the update. The
+// operations are written sweep by sweep inside each line of the update, so that consecutive
+// instructions are independent (a dependent one issues 8 cycles after its source, an independent
+// one after 4 to 5).
+template <int S> struct Cells {
+  float Ul[S], Ur[S], Vb[S], Vt[S], p[S];
+};
+#define FL_EACH _Pragma("unroll") for (int c = 0; c < S; c++)
+
+// The reference cell update (fluid.go:196-229) where every cell of the wave is a fluid interior
+// cell with four fluid neighbours: s = 4 and all weights are 1, so (-div)/4 is the exact product
+// with 0.25 and the face updates are plain adds. Damping is 1 (q * 1 is q).
+template <int S>
+__device__ __forceinline__ void update_plain(Cells<S>& x, float (&md)[S], const float (&om)[S], float cp) {
+  float d[S], q[S], t[S];
+  FL_EACH d[c] = x.Ur[c] - x.Ul[c];
+  FL_EACH d[c] += x.Vt[c];
+  FL_EACH d[c] -= x.Vb[c];
+  FL_EACH q[c] = -d[c] * 0.25f;
+  FL_EACH md[c] = fmaxf(md[c], fabsf(d[c]));
+  FL_EACH q[c] *= om[c];
+  FL_EACH t[c] = cp * q[c];
+  FL_EACH x.Ur[c] += q[c];
+  FL_EACH x.Vb[c] -= q[c];
+  FL_EACH x.Vt[c] += q[c];
+  FL_EACH x.Ul[c] -= q[c];
+  FL_EACH x.p[c] += t[c];
+}
+// The update of any cell. The weights are 0 or 1, so each fma rounds once what the reference's
+// multiply (exact) and add round. -div / s: the product with the rounded 1/s and one correction
+// step is the correctly rounded quotient for every float and s in 1..4 (compared with the
+// division over all 2^32 floats); v_div_fixup gives infinities and NaN the division's results.
+// FULL: any damping, relaxation and cp (also negative or not finite): the inactive cells' faces
+// are selected instead of left to the signs of their zeros.
+template <int S, bool FULL>
+__device__ __forceinline__ void update_any(Cells<S>& x, float (&md)[S], const float (&om)[S], float damping, float cp,
+                                           const CellW (&w)[S]) {
+  float d[S], q[S], e[S], t[S];
+  FL_EACH d[c] = x.Ur[c] - x.Ul[c];
+  FL_EACH d[c] += x.Vt[c];
+  FL_EACH d[c] -= x.Vb[c];
+  FL_EACH d[c] = __uint_as_float(__float_as_uint(d[c]) & __float_as_uint(w[c].d.z));
+  FL_EACH q[c] = -d[c] * w[c].d.x;
+  FL_EACH md[c] = fmaxf(md[c], fabsf(d[c]));
+  FL_EACH e[c] = __builtin_fmaf(q[c], w[c].d.y, d[c]);
+  FL_EACH q[c] = __builtin_fmaf(e[c], -w[c].d.x, q[c]);
+  FL_EACH q[c] = __builtin_amdgcn_div_fixupf(q[c], w[c].d.y, -d[c]);
+  FL_EACH q[c] *= om[c];
+  if constexpr (FULL) {
+    FL_EACH q[c] *= damping;
+    FL_EACH {
+      const bool on = __float_as_uint(w[c].d.z) != 0u;
+      const float p = x.p[c] + cp * q[c], ul = __builtin_fmaf(w[c].w.x, q[c], x.Ul[c]),
+                  ur = __builtin_fmaf(w[c].w.y, q[c], x.Ur[c]), vb = __builtin_fmaf(w[c].w.z, q[c], x.Vb[c]),
+                  vt = __builtin_fmaf(w[c].w.w, q[c], x.Vt[c]);
+      x.p[c] = on ? p : x.p[c];
+      x.Ul[c] = on ? ul : x.Ul[c];
+      x.Ur[c] = on ? ur : x.Ur[c];
+      x.Vb[c] = on ? vb : x.Vb[c];
+      x.Vt[c] = on ? vt : x.Vt[c];
+    }
+  } else {
+    FL_EACH t[c] = cp * q[c];
+    FL_EACH x.Ur[c] = __builtin_fmaf(w[c].w.y, q[c], x.Ur[c]);
+    FL_EACH x.Vb[c] = __builtin_fmaf(w[c].w.z, q[c], x.Vb[c]);
+    FL_EACH x.Vt[c] = __builtin_fmaf(w[c].w.w, q[c], x.Vt[c]);
+    FL_EACH x.Ul[c] = __builtin_fmaf(w[c].w.x, q[c], x.Ul[c]);
+    FL_EACH x.p[c] += t[c];
+  }
+}
+
+// The masks of a sweep's cells in a row, four bits each, eight steps to a word; loaded sixteen
+// steps at a time, at any byte.
+typedef uint32_t word2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t word4_any __attribute__((ext_vector_type(4), aligned(1)));
+static constexpr int MASK_STEPS = 16;
+
+template <int S, int W, int B> struct GsShared {
+  static constexpr int GP = (3 * S + 3 + 3) / 4 * 4;  // pitch of a Gi row, one float before and two after it
+  float4 K[W][2][B][LANES];    // K[w]: the rows (U, V, p) wave w's first sweep reads
+  float Gi[W][B + 1][GP];      // boundary below lane 0: V, p of the sweep before, U of this one
+  float4 Go[W][B][S];          // lane 63's U, V, p of each sweep
+  float4 tabw[16], tabd[16];   // CellW by mask
+  int tile;
+};
+
+// How a block's cells are updated: all plain; with weights looked up once (along a wall, say: every
+// lane's cells of a sweep have the same mask); or with weights looked up per cell.
+enum { BLOCK_PLAIN, BLOCK_SAME, BLOCK_ANY };
+// Where a wave's rows go: to the next wave's LDS rows, or to memory as handoff words.
+enum { OUT_LDS, OUT_WORDS };
+
+// Lane 63's U, V, p of S sweeps to LDS words off.. (four per sweep) of `at`. One change of the exec
+// mask and back for all of them: a branch would cut the block's straight code in pieces, and a
+// store by every lane would take the LDS bandwidth that the waves' rows need.
+template <int S>
+__device__ __forceinline__ void store_lane63(uint32_t at, int off, const float (&U)[S], const float (&V)[S],
+                                             const float (&p)[S]) {
+  if constexpr (S == 1) {
+    asm volatile(
+        "s_mov_b64 exec, %0\n\t"
+        "ds_write2_b32 %1, %2, %3 offset0:%5 offset1:%6\n\t"
+        "ds_write_b32 %1, %4 offset:%7\n\t"
+        "s_mov_b64 exec, -1" ::"s"(1ull << 63),
+        "v"(at), "v"(U[0]), "v"(V[0]), "v"(p[0]), "n"(off), "n"(off + 1), "n"(4 * (off + 2)));
+  } else {
+    static_assert(S == 2, "one or two sweeps per wave");
+    asm volatile(
+        "s_mov_b64 exec, %0\n\t"
+        "ds_write2_b32 %1, %2, %3 offset0:%8 offset1:%9\n\t"
+        "ds_write2_b32 %1, %4, %5 offset0:%10 offset1:%11\n\t"
+        "ds_write2_b32 %1, %6, %7 offset0:%12 offset1:%13\n\t"
+        "s_mov_b64 exec, -1" ::"s"(1ull << 63),
+        "v"(at), "v"(U[0]), "v"(V[0]), "v"(p[0]), "v"(U[1]), "v"(V[1]), "v"(p[1]), "n"(off), "n"(off + 1),
+        "n"(off + 2), "n"(off + 4), "n"(off + 5), "n"(off + 6));
+  }
+}
+
+// One block of B steps of a wave. gi, Kin: this block's boundary rows in LDS (Kin, Kout at this
+// lane); k: the first step's K row; mk: the masks. Each step
+// first takes what it needs from its neighbours (the loads of the step before have arrived),
+// then stores what the step before left, loads for the next step, and updates: so no step waits
+// for its own LDS traffic. The code of a block is straight, a copy for each mode and output.
+template <int S, int B, int GP, int MODE, int OUT, bool FULL>
+__device__ __forceinline__ void run_block(Sweeps<S>& Q, float (&k)[3], const uint32_t (&mk)[S], const float* gi,
+                                          const float4* Kin, float4* Kout, uint32_t go, const char* tab,
+                                          __amdgpu_buffer_rsrc_t kbuf, uint32_t kbyte, uint32_t tag, float damping,
+                                          float cp) {
+  constexpr int GN = (3 * S + 3) / 4 * 4;
+  float g[2][GN], kr[2][3];  // the boundary and K rows of this step and the next, in turn
+  CellW cw[S], cn[S];
+  auto load_gi = [&](int u) {
+    float(&d)[GN] = g[u % 2];
+#pragma unroll
+    for (int x = 0; x < 3 * S; x += 4) {
+      if (x + 2 < 3 * S) {
+        *reinterpret_cast<float4*>(&d[x]) = *reinterpret_cast<const float4*>(gi + u * GP + x);
+      } else {
+        *reinterpret_cast<float2*>(&d[x]) = *reinterpret_cast<const float2*>(gi + u * GP + x);
+      }
+    }
+  };
+  auto load_k = [&](int u) {  // what step u reads
+    const float4 v = Kin[(u - 1) * LANES];
+    kr[u % 2][0] = v.x;
+    kr[u % 2][1] = v.y;
+    kr[u % 2][2] = v.z;
+  };
+  auto load_cw = [&](int u, CellW (&d)[S]) {
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      const char* at = tab + ((u == 0 ? mk[c] << 4 : mk[c] >> (4 * u - 4)) & 0xF0u);
+      d[c].w = *reinterpret_cast<const float4*>(at);
+      d[c].d = *reinterpret_cast<const float4*>(at + 256);
+    }
+  };
+  auto put = [&](int u) {
+    if constexpr (OUT == OUT_LDS)
+      Kout[u * LANES] = make_float4(Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], 0.0f);
+    else
+      st_word(kbuf, kbyte + u * (LANES * 16), Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], tag);
+    store_lane63<S>(go, 4 * S * u, Q.UrO, Q.VbO, Q.pO);
+  };
+  load_gi(0);
+  load_gi(1);
+  load_k(1);
+#pragma unroll
+  for (int f = 0; f < 3; f++) kr[0][f] = k[f];
+  if constexpr (MODE != BLOCK_PLAIN) load_cw(0, cw);
+#pragma unroll
+  for (int u = 0; u < B; u++) {
+    Cells<S> x;
+    float pnext[S];
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      x.Ul[c] = from_lane_below(g[u % 2][3 * c + 2], Q.UrO[c]);
+      x.Vt[c] = from_lane_below(g[u % 2][3 * c], c ? Q.VbO[c - 1] : kr[u % 2][1]);
+      pnext[c] = from_lane_below(g[u % 2][3 * c + 1], c ? Q.pO[c - 1] : kr[u % 2][2]);
+      x.Ur[c] = c ? Q.UlO[c - 1] : kr[u % 2][0];
+      x.Vb[c] = Q.Vt[c];
+      x.p[c] = Q.pn[c];
+      Q.pn[c] = pnext[c];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (u > 0) put(u - 1);
+    if (u + 2 < B) load_gi(u + 2);
+    if (u + 2 <= B) load_k(u + 2);
+    if constexpr (MODE == BLOCK_ANY)
+      if (u + 1 < B) load_cw(u + 1, cn);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MODE == BLOCK_PLAIN)
+      update_plain<S>(x, Q.md, Q.om, cp);
+    else
+      update_any<S, FULL>(x, Q.md, Q.om, damping, cp, cw);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      Q.UrO[c] = x.Ur[c];
+      Q.Vt[c] = x.Vt[c];
+      Q.UlO[c] = x.Ul[c];
+      Q.VbO[c] = x.Vb[c];
+      Q.pO[c] = x.p[c];
+    }
+    if (MODE == BLOCK_ANY && u + 1 < B) {
+#pragma unroll
+      for (int c = 0; c < S; c++) cw[c] = cn[c];
+    }
+  }
+  put(B - 1);
+#pragma unroll
+  for (int f = 0; f < 3; f++) k[f] = kr[0][f];
+  asm volatile("" ::: "memory");  // lane 63's stores are not known to the compiler
+}
+
+typedef __attribute__((address_space(3))) float lds_float;
+
+// S sweeps per wave, W waves per workgroup (TK = S W sweeps per tile), B columns per block.
+template <int S, int W, int B, bool FULL, class M>
+__global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun R) {
+  constexpr int TK = S * W, GP = GsShared<S, W, B>::GP;
+  constexpr uint32_t BITS = B == 4 ? 0xFFFFu : 0xFFFFFFFFu;  // of a word of masks that a block uses
+  constexpr int MB = MASK_STEPS / B;                         // blocks a load of masks holds
+  constexpr uint32_t KROW = 16 * LANES, GROW = 16 * TK;      // bytes of a row of words
+  static_assert(B * (S + 1) <= LANES, "a lane loads one G word per block");
+  __shared__ GsShared<S, W, B> sh;
   const int lane = threadIdx.x & (LANES - 1);
   // wave-uniform, and held in a scalar register so every test on it is a scalar branch
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LANES);
-  const int tid = threadIdx.x;
-  constexpr int NT = TK * LANES;
-
-  __shared__ float xU[2][TK][LANES];
-  __shared__ float2 xVP[2][TK][LANES];
-  __shared__ float4 Kst[2][BLK][LANES + 1];
-  __shared__ float4 Gst[2][BLK][TK];
-  __shared__ float4 Gos[2][BLK][TK];
-  __shared__ int s_tile;
+  const int w = uniform((int)(threadIdx.x / LANES));
   // a re-run launch with nothing to re-run ends here, in every workgroup alike
   if (R.rerun && *R.rerun == 0) return;
+  if (threadIdx.x < 16) {
+    const CellW c = cell_weights(threadIdx.x);
+    sh.tabw[threadIdx.x] = c.w;
+    sh.tabd[threadIdx.x] = c.d;
+  }
+  const uint32_t tag0 = 2u * (uint32_t)uniform(*R.solve) & 0xffffu, tag = (tag0 + (uint32_t)R.which) & 0xffffu;
+  int vzero = 0;  // a zero the compiler keeps in a vector register: LDS addresses built on it stay there too
+  asm volatile("" : "+v"(vzero));
+  const float* gi = &sh.Gi[w][1][0] + vzero;
+  const uint32_t go = (uint32_t)(uintptr_t)(lds_float*)&sh.Go[w][0][0] + vzero;
+  const char* tab = reinterpret_cast<const char*>(sh.tabw);
 
   for (;;) {
-    if (tid == 0) s_tile = atomicAdd(R.ticket, 1);
+    if (threadIdx.x == 0) sh.tile = atomicAdd(R.ticket, 1);
     __syncthreads();
-    const int t = __builtin_amdgcn_readfirstlane(s_tile);
+    const int t = uniform(sh.tile);
     __syncthreads();
     if (t >= R.ntiles) break;
     const int2 te = R.tiles[t];
     const int sim = te.x, g = te.y >> 16, kb = te.y & 0xffff;
     const SimDesc& D = sim_desc(m, sim);
     const int NX = D.g.NX, NY = D.g.NY, rows = D.rows, KB = D.KB;
-    const int nblk = rows / BLK;
-    const int me = g * KB + kb;
-    int32_t* prog = D.prog + R.which * D.G * KB;
+    const int nblk = rows / B;
     int32_t* err = D.ctrl + 3;
     const int K = R.which ? D.ctrl[1] : R.K;
-    if (tile_empty(g, kb, K, TK, NX)) {
-      if (tid == 0) __hip_atomic_store(&prog[me], rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      continue;
-    }
-    const float* Uin = D.buf[B_U];
-    const float* Vin = D.buf[B_V];
-    const float* Pin = R.rPin >= 0 ? D.buf[R.rPin] : nullptr;
-    float* Uout = D.buf[B_U2];
-    float* Vout = D.buf[B_V2];
-    float* Pout = D.buf[R.rPout];
-    const uint8_t* fdiag = D.diag;
-    float* kout = D.kout;
-    float* gout = D.gout;
-    const float cp = D.cp;
-    const float damping = R.damping;
+    const int Kp = (K + S - 1) / S * S;  // with the sweeps that only fill the last wave
+    if (tile_empty(g, kb, Kp, TK, NX)) continue;
+    const float cp = D.cp, damping = R.damping;
     const int k0 = kb * TK;
-    const int k = k0 + wave;
-    const bool wave_on = k < K;
-    // wave-uniform in a scalar register: the other waves skip the output block with one branch
-    const int last = __builtin_amdgcn_readfirstlane((int)(k == K - 1));
-    const int first_out = SNAP ? __builtin_amdgcn_readfirstlane((int)(R.which == 0 && k == 0)) : 0;
-    const int i0 = LANES * g - k0;           // row of (lane 0, wave 0)
-    const int row = i0 + lane - wave;        // this thread's row
-    const bool real_row = row >= 0 && row <= NX - 1;
-    // this sweep's relaxation, read once into a scalar register: a vector-loaded value used in
-    // the step loop would make every step wait for all of the wave's memory operations
-    const float om = __int_as_float(
-        __builtin_amdgcn_readfirstlane(__float_as_int(wave_on ? R.omega[min(k, K - 1)] : 0.0f)));
-    const int d0 = LANES * g - k0 - 2 * wave;  // anti-diagonal of column 0 for this wave
+    const int i0 = LANES * g - k0;     // row of (lane 0, sweep 0)
+    const int b0 = w * S;              // this wave's first sweep in the tile
+    const bool wave_on = k0 + b0 < K;
+    const bool words = w == W - 1 || k0 + b0 + S >= K;  // its rows go to the next sweeps' tile, or are the result
+    const bool g_wave = g + 1 < D.G;                    // lane 63's faces go to the next row-tile
+    // Producers: G stream (g-1,kb), K stream (g,kb-1), corner (g-1,kb-1); the first sweeps take the
+    // K stream's place from the initial state's rows (k_gs_skew).
+    const bool hG = g > 0 && !tile_empty(g - 1, kb, Kp, TK, NX);
+    const bool hK = kb == 0 || !tile_empty(g, kb - 1, Kp, TK, NX);
+    const bool hC = g > 0 && (kb == 0 || !tile_empty(g - 1, kb - 1, Kp, TK, NX));
+    const size_t gtile = (size_t)rows * GROW, ktile = (size_t)rows * KROW, itile = (size_t)(rows + 1) * KROW;
+    const __amdgpu_buffer_rsrc_t kmine = word_buffer(D.kout + (size_t)(g * KB + kb) * ktile);
+    const __amdgpu_buffer_rsrc_t gmine = word_buffer(D.gout + (size_t)(g * KB + kb) * gtile);
+    const __amdgpu_buffer_rsrc_t gprod = word_buffer(D.gout + (hG ? (size_t)((g - 1) * KB + kb) * gtile : 0));
+    const uint8_t* ksrc = kb ? D.kout + (size_t)(kb - 1) * ktile : D.kinit;  // of row-tile 0
+    const size_t kstep = kb ? KB * ktile : itile;                            // to the next row-tile
+    const __amdgpu_buffer_rsrc_t kprod = word_buffer(ksrc + (hK ? g * kstep : 0));
+    const __amdgpu_buffer_rsrc_t cprod = word_buffer(ksrc + (hC ? (g - 1) * kstep : 0));
+    const uint32_t ktag = kb ? tag : tag0;
+    const int kfirst = kb ? TK : 1, klast = kb ? rows - 1 : rows;  // row of step 1, last row
 
-    // Producers: G stream (g-1,kb), K stream (g,kb-1), corner (g-1,kb-1).
-    const int pG = (g > 0 && !tile_empty(g - 1, kb, K, TK, NX)) ? (g - 1) * KB + kb : -1;
-    const int pK = (kb > 0 && !tile_empty(g, kb - 1, K, TK, NX)) ? g * KB + kb - 1 : -1;
-    const int pC = (g > 0 && kb > 0 && !tile_empty(g - 1, kb - 1, K, TK, NX)) ? (g - 1) * KB + kb - 1 : -1;
-    int seenG = 0, seenK = 0;  // producer progress last observed (thread 0)
-
-    // Wait until every producer has published the rows block `blk` stages: G stream rows up to
-    // s1 + 63, K stream rows up to s1 + TK - 1, corner rows up to s1 + 63 + TK (s1 = the block's
-    // last step). The corner producer (g-1, kb-1) is the G producer's K producer, and
-    // progress is published in whole blocks: G progress >= s1 + 64 = BLK (blk+1) + 63 means
-    // progress >= BLK (blk+1) + 64 = s1 + 65, which the G producer could publish only after it
-    // waited for corner progress >= s1 + 64 + TK (both clamped to rows). So with a G producer
-    // the corner needs no poll of its own; without one (g-1, kb) is empty, and the corner is
-    // polled in the G slot.
-    const int pGp = pG >= 0 ? pG : pC;
-    const int lagG = pG >= 0 ? LANES : LANES + TK;
-    auto wait_block = [&](int blk) {
-      if (tid == 0) {
-        const int s1 = blk * BLK + BLK - 1;  // last step of the block
-        const int needG = pGp >= 0 ? min(s1 + lagG, rows) : 0;
-        const int needK = pK >= 0 ? min(s1 + TK, rows) : 0;
-        wait_producers(prog + max(pGp, 0), needG, prog + max(pK, 0), needK, seenG, seenK, err);
-      }
-    };
-
-    // Staged boundary items of one block: K stream BLK x 65, G stream BLK x TK.
-    // Items [0, KITEM) are the K stream; the G stream starts at the next wave boundary, so no
-    // wave holds lanes of both (a wave running both branches would wait, in the second, for
-    // the loads the first issued into the registers both use).
-    constexpr int KITEM = BLK * (LANES + 1);
-    constexpr int GITEM0 = (KITEM + LANES - 1) / LANES * LANES;
-    constexpr int NITEM = GITEM0 + BLK * TK;
-    constexpr int PER = (NITEM + NT - 1) / NT;
-    float4 stage[PER];
-    float2 corner[PER];  // K-stream lane 0: V and p of the corner producer, merged in store_block
-    auto load_block = [&](int blk) {
+    Sweeps<S> Q;
+    uint32_t mrow[S], mk[S], mkeep[S];
+    int mcol[S];
+    const uint32_t mpitch = mask_pitch(NY);
 #pragma unroll
-      for (int q = 0; q < PER; q++) {
-        const int it = tid + q * NT;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        float2 cz = make_float2(0.f, 0.f);
-        if (it < KITEM) {
-          const int u = it / (LANES + 1), slot = it % (LANES + 1);
-          const int s = blk * BLK + u;
-          if (kb == 0) {
-            // initial state: lane `slot` of wave 0 is row i0+slot at column s-slot
-            const int r = i0 + slot, j = s - slot;
-            if (slot < LANES && j >= 0 && j <= NY - 1) {
-              if (r + 1 >= 0 && r + 1 <= NX - 1) v.x = Uin[(size_t)(r + 1) * NY + j];
-              if (r >= 0 && r <= NX - 1 && j + 1 <= NY - 1) {
-                v.y = Vin[(size_t)r * NY + j + 1];
-                v.z = Pin ? Pin[(size_t)r * NY + j + 1] : 0.0f;
+    for (int c = 0; c < S; c++) {
+      // read once into a scalar register: a vector-loaded value used in the step would make
+      // every step wait for the wave's memory operations
+      Q.om[c] = uniform(k0 + b0 + c < K ? R.omega[min(k0 + b0 + c, K - 1)] : 1.0f);
+      Q.UrO[c] = Q.UlO[c] = Q.VbO[c] = Q.pO[c] = Q.Vt[c] = Q.pn[c] = Q.md[c] = 0.0f;
+      mkeep[c] = k0 + b0 + c < K ? BITS : 0u;  // past the solve's last sweep the cells pass their faces on
+      // rows 0 and NX - 1 are all 0; the copy in which this lane's columns start a byte (an odd
+      // first column j: byte (j + 1) / 2 of the odd copy)
+      mrow[c] = (((lane + b0 + c) & 1) ? NX * mpitch : 0u) +
+                (uint32_t)min(max(i0 + lane - b0 - c, 0), NX - 1) * mpitch + MASK_PAD / 2;
+      mcol[c] = (1 - lane - b0 - c) >> 1;
+    }
+    const uint8_t* masks = D.masks;
+    const int mlast = (NY + 2) >> 1;
+    float k[3] = {0.0f, 0.0f, 0.0f};
+
+    // The G words of a block this lane loads: word (u, x) is what sweep b0 - 1 + x of the tile
+    // below left at lane 63 for this wave's step u; a tile's first sweep (w = 0, x = 0) takes lane
+    // 63 of that tile's K row instead.
+    const int gu = lane / (S + 1), gx = lane - gu * (S + 1);
+    const bool gcorner = w == 0 && gx == 0, gstage = gu < B, ghas = gstage && (gcorner ? hC : hG);
+    const uint32_t gat = gcorner ? 16 * (LANES - 1) : 16 * (b0 - 1 + gx);
+    const uint32_t goff = gat + (gcorner ? (gu + LANES - 1 + kfirst) * KROW : (gu + LANES - 1) * GROW);
+    const uint32_t glast = gat + (gcorner ? klast * KROW : (rows - 1) * GROW);
+    lds_float* const gdst = (lds_float*)&sh.Gi[w][min(gu, B - 1) + 1][3 * gx];
+    const uint32_t gotid = min(lane, B * S - 1);  // the word of lane 63's this lane stores: step / S, sweep % S
+    const uint32_t goword = (gotid / S) * GROW + 16 * (b0 + gotid % S);
+    // Ends a wait for words that all carry this solve's tag. Bounded: after SPIN_LIMIT tries, or
+    // once another wait of this simulation has expired (err set), err is set and the solve goes
+    // on, so one whose producers stall ends within about a second with FL_ERR_INTERNAL.
+    auto expired = [&](bool done, int it) __attribute__((always_inline)) {
+      if (done) return true;
+      if (it > SPIN_LIMIT || ((it & 255) == 255 && ld_err(err) != 0)) {
+        if (lane == 0) atomicOr(err, 1);
+        return true;
+      }
+      __builtin_amdgcn_s_sleep(2);
+      return false;
+    };
+    // One wave's part of the tile: FIRST, whether it is the tile's first wave and loads K words; OUT,
+    // where its rows go. A copy of the code for each, so that none carries another's registers. Wave w
+    // stages its first block in phase w - 1 and runs block n in phase w + n; a phase ends in a barrier.
+    auto run_wave = [&](auto first_c, auto out_c) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_c)::value;
+      constexpr int OUT = decltype(out_c)::value;
+      // The words and masks of a block. The loads are issued without a condition on the lane, at
+      // addresses that are always valid, so none waits for another.
+      struct Block {
+        word4 gw, gc, kw[B];
+      };
+      word2_any mw[S];  // masks of the MB blocks that the next block to stage is one of
+      auto load_g = [&](Block& x, int n) __attribute__((always_inline)) {
+        x.gw = ld_word(gprod, gcorner ? 0u : min(goff + n * (B * GROW), glast));
+        if constexpr (FIRST) x.gc = ld_word(cprod, gcorner ? min(goff + n * (B * KROW), glast) : 0u);
+      };
+      auto load_k = [&](Block& x, int n, int u) __attribute__((always_inline)) {
+        x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(kprod, 16 * lane, min(n * B + u + kfirst, klast) * KROW,
+                                                        SC1 | VOLATILE_OP);
+      };
+      auto load = [&](Block& x, int n) __attribute__((always_inline)) {
+        load_g(x, n);
+        if constexpr (FIRST) {
+#pragma unroll
+          for (int u = 0; u < B; u++) load_k(x, n, u);
+        }
+        if (n % MB == 0) {
+#pragma unroll
+          for (int c = 0; c < S; c++)
+            mw[c] = *reinterpret_cast<const word2_any*>(
+                masks + (mrow[c] + min(max(n * (B / 2) + mcol[c], -(MASK_PAD / 2)), mlast)));
+        }
+      };
+      auto stage = [&](Block& x, int n) __attribute__((always_inline)) {
+        auto arrived = [&]() __attribute__((always_inline)) {
+          uint32_t d = 0;
+          if constexpr (FIRST) {
+            if (gcorner) x.gw = x.gc;
+            if (ghas) d = word_tag(x.gw, gcorner ? ktag : tag);
+            if (hK) {
+#pragma unroll
+              for (int u = 0; u < B; u++) d |= word_tag(x.kw[u], ktag);
+            }
+          } else {
+            if (ghas) d = word_tag(x.gw, tag);
+          }
+          return __all(d < 0x10000u);
+        };
+        // The first check stands before the loop: at the loop's head it would have to wait for every
+        // store issued since. A wait polls with the G words and the block's last K row only: 256 CUs
+        // that reload whole blocks would take the bandwidth their producers need.
+        if (!arrived()) {
+          for (int it = 0; !expired(false, it); it++) {
+            load_g(x, n);
+            if constexpr (FIRST) {
+              load_k(x, n, B - 1);
+              if (hK && __all(word_tag(x.kw[B - 1], ktag) < 0x10000u)) {
+#pragma unroll
+                for (int u = 0; u < B - 1; u++) load_k(x, n, u);
               }
             }
-          } else {
-            if (pK >= 0) {
-              const int rr = min(s + TK - 1, rows - 1);
-              v = ld_dev3(kout + ((size_t)pK * rows + rr) * 3 * (LANES + 1) + slot, LANES + 1);
-            }
-            // lane 0 takes V and p from the corner producer instead (zero without one); the
-            // values are merged in store_block, so no wait for these loads happens here
-            if (slot == 0 && pC >= 0) {
-              const int rr = min(s + 63 + TK, rows - 1);
-              const float* cpp = kout + ((size_t)pC * rows + rr) * 3 * (LANES + 1) + LANES;
-              cz.x = ld_dev(cpp + (LANES + 1));
-              cz.y = ld_dev(cpp + 2 * (LANES + 1));
-            }
-          }
-        } else if (it >= GITEM0 && it < NITEM) {
-          const int e = it - GITEM0;
-          const int u = e / TK, b = e % TK;
-          const int s = blk * BLK + u;
-          if (pG >= 0) {
-            const int rr = min(s + 63, rows - 1);
-            v = ld_dev3(gout + ((size_t)pG * rows + rr) * 3 * TK + b, TK);
+            if (arrived()) break;
           }
         }
-        stage[q] = v;
-        corner[q] = cz;
-      }
-    };
-    auto store_block = [&](int buf) {
-#pragma unroll
-      for (int q = 0; q < PER; q++) {
-        const int it = tid + q * NT;
-        if (it < KITEM) {
-          float4 v = stage[q];
-          // lane 0 of each K-stream row takes V and p of the corner producer (zero without one)
-          const bool lane0 = kb > 0 && it % (LANES + 1) == 0;
-          v.y = lane0 ? corner[q].x : v.y;
-          v.z = lane0 ? corner[q].y : v.z;
-          Kst[buf][it / (LANES + 1)][it % (LANES + 1)] = v;
-        } else if (it >= GITEM0 && it < NITEM) {
-          const int e = it - GITEM0;
-          Gst[buf][e / TK][e % TK] = stage[q];
+        // (a producer that does not exist leaves arbitrary values to lane 0, or to lanes off the
+        // grid, whose cells lie outside the interior in every sweep)
+        if (gstage) {
+          gdst[-1] = word_u(x.gw);
+          gdst[0] = word_v(x.gw);
+          gdst[1] = word_p(x.gw);
         }
-      }
-    };
-    // Flags of this thread's cells for the BLK columns of a block (anti-diagonal layout), one
-    // byte load each into its own register.
-    auto load_flags = [&](int blk, uint32_t* fl) {
+        if constexpr (FIRST) {
+          float4* dst = &sh.K[0][n & 1][0][lane];
 #pragma unroll
-      for (int u = 0; u < BLK; u++) {
-        const int s = blk * BLK + u;
-        const int dd = d0 + s;
-        uint32_t f = 0;
-        if (wave_on && real_row && dd >= 0 && dd <= NX + NY - 2) f = fdiag[(size_t)dd * NX + row];
-        fl[u] = f;
-      }
-    };
-    // The flags of the block being run: with 8-sweep tiles packed four to a register at the
-    // block's end (when the loads have returned; packing them as they arrive would make the wave
-    // wait for them, and for every load issued before them, at the block's start). That holds
-    // the 8x8 kernel to 119 VGPRs, two workgroups per CU instead of one: 4096^2 cavity 12.42 ->
-    // 11.89 ms/step. The unpacking costs a bit-field extract per step, which loses 5% where it
-    // does not change the occupancy (16-sweep tiles), so other shapes keep one flag a register.
-    constexpr bool PACK = TK == 8;
-    constexpr int FW = PACK ? (BLK + 3) / 4 : BLK;
-    auto take_flags = [&](const uint32_t* fl, uint32_t* cur) {
-      if constexpr (PACK) {
-#pragma unroll
-        for (int w = 0; w < FW; w++) cur[w] = 0;
-#pragma unroll
-        for (int u = 0; u < BLK; u++) cur[u / 4] |= fl[u] << (8 * (u % 4));
-      } else {
-#pragma unroll
-        for (int u = 0; u < BLK; u++) cur[u] = fl[u];
-      }
-    };
-    // Producer side, in two halves run by the last wave (which also stores the K-stream
-    // rows, three stores per step). publish_data(blk) copies the G stream of block blk to
-    // global without waiting. publish_rows(n) makes handoff rows [0, n) visible: it waits
-    // for the wave's stores of those rows, then stores the progress counter. On time
-    // (R.defer 0), the rows of block blk are published at the start of block blk + 1 after a
-    // full wait. With R.defer 1 they are published at the start of block blk + 2, right after
-    // publish_data(blk + 1): by then the wave has issued at least NEWER stores after them
-    // (the 3 * BLK K-stream stores of block blk + 1 and the G copy of block blk + 1), and
-    // stores retire in issue order, so waiting until at most NEWER are in flight completes
-    // them without waiting for the stores just issued. With R.defer 2 they are published
-    // after step MID - 1 of block blk + 1, when the 3 * MID K-stream stores of that block's
-    // first MID steps are the newer ones. Deferring removes a store round trip from every
-    // block and lengthens the pipeline fill by the steps of delay per producer hop. After the
-    // loop the last blocks are published with a full wait.
-    constexpr int NEWER = 3 * BLK + 3 * ((BLK * TK + LANES - 1) / LANES);
-    constexpr int MID = BLK / 2;
-    auto publish_data = [&](int blk) {
-      if (wave == TK - 1) {
-        for (int e = lane; e < BLK * TK; e += LANES) {
-          const int u = e / TK, b = e % TK;
-          const float4 v = Gos[blk & 1][u][b];
-          float* dst = gout + ((size_t)me * rows + blk * BLK + u) * 3 * TK + b;
-          st_dev(dst, v.x);
-          st_dev(dst + TK, v.y);
-          st_dev(dst + 2 * TK, v.z);
+          for (int u = 0; u < B; u++)
+            dst[u * LANES] = make_float4(word_u(x.kw[u]), word_v(x.kw[u]), word_p(x.kw[u]), 0.0f);
         }
-      }
-    };
-    auto publish_rows = [&](int n, bool all) {
-      if (wave == TK - 1) {
-        if (all)
-          wait_stores();
-        else
-          wait_stores_but<NEWER>();
-        if (lane == 0) __hip_atomic_store(&prog[me], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    };
-    auto publish_rows_mid = [&](int n) {
-      if (wave == TK - 1) {
-        wait_stores_but<3 * MID>();
-        if (lane == 0) __hip_atomic_store(&prog[me], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    };
-
-    // Prologue: block 0 staged synchronously.
-    wait_block(0);
-    __syncthreads();
-    load_block(0);
-    store_block(0);
-    uint32_t fcur[FW], fnext[BLK];
-    if constexpr (PACK) {
-      load_flags(0, fnext);
-      take_flags(fnext, fcur);
-    } else {
-      load_flags(0, fcur);
-    }
-    __syncthreads();
-
-    float UrOut = 0.f, Vreg = 0.f, pn = 0.f, md = 0.f;
-    for (int blk = 0; blk < nblk; blk++) {
-      const int cb = blk & 1;
-      if (blk > 0) {
-        publish_data(blk - 1);
-        if (R.defer == 0)
-          publish_rows(blk * BLK, true);
-        else if (R.defer == 1 && blk > 1)
-          publish_rows((blk - 1) * BLK, false);
-      }
-      const bool more = blk + 1 < nblk;
-      if (more) {
-        wait_block(blk + 1);
-        __syncthreads();
-        load_block(blk + 1);
-        load_flags(blk + 1, fnext);
-      }
 #pragma unroll
-      for (int u = 0; u < BLK; u++) {
-        const int s = blk * BLK + u;
-        const int pb = (s + 1) & 1;  // buffer written at step s-1
-        const int wb = s & 1;
-        // ---- inputs
-        const float4 gin = Gst[cb][u][wave];
-        float Ul = __int_as_float(
-            __builtin_amdgcn_update_dpp(__float_as_int(gin.x), __float_as_int(UrOut), 0x138, 0xF, 0xF, false));
-        float Ur, Vt, pnew;
-        if (wave == 0) {
-          const float4 kin = Kst[cb][u][lane];
-          Ur = kin.x;
-          Vt = kin.y;
-          pnew = kin.z;
+        for (int c = 0; c < S; c++) {
+          const uint32_t lo = mw[c].x, hi = mw[c].y;
+          if constexpr (B == 8)
+            mk[c] = (n % 2 ? hi : lo) & mkeep[c];
+          else
+            mk[c] = ((n & 2 ? hi : lo) >> (n & 1 ? 16 : 0)) & mkeep[c];
+          asm volatile("" : "+v"(mk[c]));  // now: the scheduler would wait for the masks after the next stores
+        }
+      };
+      auto run = [&](int n) __attribute__((always_inline)) {
+        const float4* Kin = &sh.K[w][n & 1][0][lane];
+        float4* Kout = &sh.K[w + 1 < W ? w + 1 : w][n & 1][0][lane];
+        const uint32_t kbyte = (uint32_t)n * (B * KROW) + 16 * lane;
+        bool plain = true, same = true;
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          plain = plain && mk[c] == BITS;
+          same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
+        }
+#define FL_RUN(MODE) \
+  run_block<S, B, GP, MODE, OUT, FULL>(Q, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
+        if (!FULL && __all(plain)) {
+          FL_RUN(BLOCK_PLAIN);
+        } else if (__all(same)) {
+          FL_RUN(BLOCK_SAME);
         } else {
-          Ur = xU[pb][wave - 1][lane];
-          if (lane == 0) {
-            Vt = gin.y;
-            pnew = gin.z;
-          } else {
-            const float2 vp = xVP[pb][wave - 1][lane - 1];
-            Vt = vp.x;
-            pnew = vp.y;
-          }
+          FL_RUN(BLOCK_ANY);
         }
-        float Vb = Vreg;
-        float p = pn;
-        pn = pnew;
-        // ---- the reference cell update (fluid.go:196-229)
-        const uint32_t f = PACK ? (fcur[u / 4] >> (8 * (u % 4))) & 0xFFu : fcur[u];
-        const bool plain = __all((f & 0x3Fu) == 0x3Fu);
-        if (std::is_same<M, OneSim>::value ? __builtin_expect(plain, 1) : plain) {
-          // Every lane holds a fluid interior cell whose four neighbours are fluid: s = 4 and
-          // all weights are 1, so (-div)/4 is the exact product with 0.25 and the face updates
-          // are plain adds -- the same float results with a third of the instructions. For a
-          // single simulation laid out as the fall-through path (1% per step on the 4096^2
-          // cavity and the 256^2 jet); the batched 8x8 kernel would spill at 128 VGPRs with it.
-          const float div = Ur - Ul + Vt - Vb;
-          const float ad = fabsf(div);
-          if (ad > md) md = ad;
-          float q = -div * 0.25f;
-          q *= om;
-          q *= damping;
-          p += cp * q;
-          Ul -= q;
-          Ur += q;
-          Vb -= q;
-          Vt += q;
-        } else if (f & CF_GS) {
-          // spread neighbour bits 1..4 to bytes 0..3, then convert each byte (0 or 1)
-          const uint32_t w = (((f >> 1) & 0xFu) * 0x00204081u) & 0x01010101u;
-          const float sx0 = (float)(w & 0xFFu);
-          const float sx1 = (float)((w >> 8) & 0xFFu);
-          const float sy0 = (float)((w >> 16) & 0xFFu);
-          const float sy1 = (float)(w >> 24);
-          const float sum = sx0 + sx1 + sy0 + sy1;
-          const float div = Ur - Ul + Vt - Vb;
-          const float ad = fabsf(div);
-          if (ad > md) md = ad;
-          float q = -div / sum;
-          q *= om;
-          q *= damping;
-          p += cp * q;
-          Ul -= sx0 * q;
-          Ur += sx1 * q;
-          Vb -= sy0 * q;
-          Vt += sy1 * q;
+#undef FL_RUN
+      };
+      for (int p = 0; p < w; p++) __syncthreads();
+      if constexpr (FIRST) {
+        // what sweep 0 reads at step 0, the row before block 0's
+        for (int it = 0;; it++) {
+          const word4 v = ld_word(kprod, (kfirst - 1) * KROW + 16 * lane);
+          k[0] = word_u(v);
+          k[1] = word_v(v);
+          k[2] = word_p(v);
+          if (expired(!hK || __all(word_tag(v, ktag) < 0x10000u), it)) break;
         }
-        // ---- outputs
-        UrOut = Ur;
-        Vreg = Vt;
-        xU[wb][wave][lane] = Ul;
-        xVP[wb][wave][lane] = make_float2(Vb, p);
-        if (lane == LANES - 1) {
-          Gos[cb][u][wave].x = Ur;
-          if (wave + 1 < TK) {
-            Gos[cb][u][wave + 1].y = Vb;
-            Gos[cb][u][wave + 1].z = p;
-          }
-        }
-        if (wave == TK - 1) {
-          float* kr = kout + ((size_t)me * rows + s) * 3 * (LANES + 1);
-          st_dev(kr + lane, Ul);
-          st_dev(kr + (LANES + 1) + lane + 1, Vb);
-          st_dev(kr + 2 * (LANES + 1) + lane + 1, p);
-        }
-        // halfway publication of the previous block's rows (R.defer 2): the K-stream stores of
-        // steps 0..MID-1 of this block are the 3 * MID newest of this wave
-        if (u == MID - 1 && R.defer == 2 && blk > 0) publish_rows_mid(blk * BLK);
-        if (last) {  // only the wave of the final sweep writes the results
-          const int j = s - lane - wave;
-          if (real_row && j >= 0 && j <= NY - 1) {
-            const size_t c = (size_t)row * NY + j;
-            const bool tu = row >= 1 && j >= 1 && j <= NY - 2;
-            const bool tv = row >= 1 && row <= NX - 2 && j >= 1;
-            const bool tp = row >= 1 && row <= NX - 2 && j >= 1 && j <= NY - 2;
-            if (tu) Uout[c] = Ul;
-            if (tv) Vout[c] = Vb;
-            if (tp) Pout[c] = p;
-          }
-        }
-        if (first_out) {  // the first sweep's result, kept for an early exit after it
-          const int j = s - lane - wave;
-          if (real_row && j >= 0 && j <= NY - 1) {
-            const size_t c = (size_t)row * NY + j;
-            if (row >= 1 && j >= 1 && j <= NY - 2) D.buf[B_T0][c] = Ul;
-            if (row >= 1 && row <= NX - 2 && j >= 1) D.buf[B_T1][c] = Vb;
-            if (row >= 1 && row <= NX - 2 && j >= 1 && j <= NY - 2) D.buf[B_T2][c] = p;
-          }
+      }
+      {
+        Block x;
+        load(x, 0);
+        stage(x, 0);
+      }
+      __syncthreads();
+      for (int n = 0; n < nblk; n++) {
+        // Block n runs while the words of block n + 1 are on their way (the last block's once more
+        // after the end). They are waited for before the stores of lane 63's words are issued: vector
+        // memory operations complete in order, and a wait behind a store would last as long as the
+        // store's way to memory.
+        const int n1 = min(n + 1, nblk - 1);
+        Block x;
+        load(x, n1);
+        run(n);
+        stage(x, n1);
+        if (g_wave) {
+          const float4 v = (&sh.Go[w][0][0])[gotid];
+          if (lane < B * S) st_word(gmine, goword + n * (B * GROW), v.x, v.y, v.z, tag);
         }
         __syncthreads();
       }
-      if (more) {
-        store_block(cb ^ 1);
-        take_flags(fnext, fcur);
-        __syncthreads();
-      }
+      for (int p = w + 1; p < W; p++) __syncthreads();
+    };
+    using first_t = std::true_type;
+    using later_t = std::false_type;
+    using lds_t = std::integral_constant<int, OUT_LDS>;
+    using words_t = std::integral_constant<int, OUT_WORDS>;
+    if (!wave_on) {
+      for (int p = 0; p < nblk + W; p++) __syncthreads();
+    } else if (w == 0) {
+      if (words)
+        run_wave(first_t{}, words_t{});
+      else if constexpr (W > 1)
+        run_wave(first_t{}, lds_t{});
+    } else if constexpr (W > 1) {
+      if (words)
+        run_wave(later_t{}, words_t{});
+      else
+        run_wave(later_t{}, lds_t{});
     }
-    publish_data(nblk - 1);
-    publish_rows(rows, true);  // rows = nblk * BLK
     // per-sweep max |div|
-    float mv = md;
-    for (int o = 32; o > 0; o >>= 1) mv = fmaxf(mv, __shfl_xor(mv, o, 64));
-    if (lane == 0 && wave_on && mv > 0.0f) atomicMax(&D.maxdiv[R.which * D.nmax + k], __float_as_uint(mv));
-    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      float mv = Q.md[c];
+      for (int o = 32; o > 0; o >>= 1) mv = fmaxf(mv, __shfl_xor(mv, o, 64));
+      if (lane == 0 && k0 + b0 + c < K && mv > 0.0f)
+        atomicMax(&D.maxdiv[R.which * D.nmax + k0 + b0 + c], __float_as_uint(mv));
+    }
+  }
+}
+
+// The initial state in the solve's layout, and the result out of it. An item is 64 rows of words of
+// one row-tile; each of a workgroup's four waves moves 16 of the tile's 64 grid rows, 64 columns
+// each, through LDS, so that both sides read and write whole lines.
+__device__ __forceinline__ bool skew_item(const OneSim& m, int, const SimDesc*& D, int& g, int& t0) {
+  D = &m.d;
+  const int nt = (D->rows + 1 + LANES - 1) / LANES;
+  g = blockIdx.x / nt;
+  t0 = (blockIdx.x % nt) * LANES;
+  return true;
+}
+__device__ __forceinline__ bool skew_item(const ManySims& m, const SkewItem* items, const SimDesc*& D, int& g, int& t0) {
+  const SkewItem it = items[blockIdx.x];
+  D = &m.sims[it.sim];
+  g = it.g;
+  t0 = it.t0;
+  return true;
+}
+__device__ __forceinline__ bool skew_item(const OneSim& m, const SkewItem*, const SimDesc*& D, int& g, int& t0) {
+  return skew_item(m, 0, D, g, t0);
+}
+
+// Row t (stored at t + 1) of row-tile g holds, at lane a, U, V and p of cell (64 g + a + 1, t - a + 1):
+// what lane a of a sweep before the first would have left at step t.
+template <class M>
+__global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int rPin) {
+  __shared__ float sh[3][LANES][LANES + 1];
+  const SimDesc* D;
+  int g, t0;
+  skew_item(m, items, D, g, t0);
+  const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY;
+  const float* src[3] = {D->buf[B_U], D->buf[B_V], rPin >= 0 ? D->buf[rPin] : nullptr};
+#pragma unroll 4
+  for (int x = 0; x < 16; x++) {
+    const int a = 16 * w + x, r = LANES * g + a + 1, j = t0 - a + lane;
+    const bool in = r < NX && j >= 0 && j < NY;
+#pragma unroll
+    for (int f = 0; f < 3; f++) sh[f][a][lane] = in && src[f] ? src[f][(size_t)r * NY + j] : 0.0f;
+  }
+  __syncthreads();
+  const uint32_t tag = 2u * (uint32_t)*solve & 0xffffu;
+  const __amdgpu_buffer_rsrc_t dst = word_buffer(D->kinit + (size_t)g * (D->rows + 1) * (16 * LANES));
+#pragma unroll 4
+  for (int x = 0; x < 16; x++) {
+    const int u = 16 * w + x;
+    if (t0 + u <= D->rows)
+      st_word(dst, (uint32_t)(t0 + u) * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
+  }
+}
+
+// The rows of the last sweep's wave (its last sweep b, padded to the wave's S) to U2, V2 and role
+// rPout: row t of row-tile g holds cell (64 g + a - k0 - b, t - a - b) at lane a. An early exit
+// (ctrl[1] sweeps) takes the re-run's. Also numbers the next solve.
+template <class M>
+__global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, int32_t* solve, int N, int tk, int S,
+                                                   int rPout) {
+  __shared__ float sh[3][LANES][LANES + 1];
+  const SimDesc* D;
+  int g, t0;
+  skew_item(m, items, D, g, t0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) ++*solve;
+  const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY, rows = D->rows;
+  const int kept = D->early_exit ? D->ctrl[1] : 0, K = kept > 0 ? kept : N;
+  const int kb = (K - 1) / tk, k0 = kb * tk, b = (K - 1 - k0) / S * S + S - 1;
+  const int r0 = LANES * g - k0 - b;  // row of lane 0
+  if (r0 > NX - 1 || r0 + LANES - 1 < 1) return;
+  const __amdgpu_buffer_rsrc_t src = word_buffer(D->kout + (size_t)(g * D->KB + kb) * rows * (16 * LANES));
+#pragma unroll 4
+  for (int x = 0; x < 16; x++) {
+    const int u = 16 * w + x;
+    const word4 v = ld_word(src, (uint32_t)min(t0 + u, rows - 1) * (16 * LANES) + 16 * lane);
+    sh[0][lane][u] = word_u(v);
+    sh[1][lane][u] = word_v(v);
+    sh[2][lane][u] = word_p(v);
+  }
+  __syncthreads();
+  float* const dst[3] = {D->buf[B_U2], D->buf[B_V2], D->buf[rPout]};
+#pragma unroll 4
+  for (int x = 0; x < 16; x++) {
+    const int a = 16 * w + x, r = r0 + a, j = t0 + lane - a - b;
+    if (r < 1 || r > NX - 1 || j < 1 || j > NY - 1 || t0 + lane >= rows) continue;
+    const size_t c = (size_t)r * NY + j;
+    if (j <= NY - 2) dst[0][c] = sh[0][a][lane];
+    if (r <= NX - 2) dst[1][c] = sh[1][a][lane];
+    if (r <= NX - 2 && j <= NY - 2) dst[2][c] = sh[2][a][lane];
   }
 }
 
@@ -554,12 +763,10 @@ template <class M> __global__ void k_gs_ring(M m, int rPin, int rPout) {
   }
 }
 
-// Zero the counters of both runs, the per-sweep maxima and the re-run requests of every
+// Zero the ticket counters of both runs, the per-sweep maxima and the re-run requests of every
 // simulation of the launch (graph-safe: no memset).
-__global__ void k_gs_init(int32_t* prog, int nprog, uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim,
-                          int32_t* ticket) {
+__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim, int32_t* ticket) {
   const int stride = blockDim.x * gridDim.x;
-  for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nprog; t += stride) prog[t] = 0;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nmd; t += stride) maxdiv[t] = 0u;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nsim; t += stride) ctrl[4 * t] = ctrl[4 * t + 1] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -570,8 +777,8 @@ __global__ void k_gs_init(int32_t* prog, int nprog, uint32_t* maxdiv, int nmd, i
 }
 
 // k_gs_ring and k_gs_init of a single simulation in one launch (both only precede the solve).
-__global__ void k_gs_prep(OneSim m, int rPin, int rPout, int32_t* prog, int nprog, uint32_t* maxdiv, int nmd,
-                          int32_t* ctrl, int32_t* ticket) {
+__global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int nmd, int32_t* ctrl,
+                          int32_t* ticket) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const SimDesc& D = m.d;
   const int NX = D.g.NX, NY = D.g.NY;
@@ -584,7 +791,6 @@ __global__ void k_gs_prep(OneSim m, int rPin, int rPout, int32_t* prog, int npro
     ring_copy(D, NX - 1, t, rPin, rPout);
   }
   const int stride = blockDim.x * gridDim.x;
-  for (int i = t; i < nprog; i += stride) prog[i] = 0;
   for (int i = t; i < nmd; i += stride) maxdiv[i] = 0u;
   if (t == 0) {
     ctrl[0] = ctrl[1] = 0;
@@ -594,14 +800,10 @@ __global__ void k_gs_prep(OneSim m, int rPin, int rPout, int32_t* prog, int npro
 
 // Early exit of solveSingleGrid (fluid.go:175-177), one wave per simulation: the first
 // sweep whose max |div| is below 1e-5 ends the solve; if that is not the last sweep,
-// request a re-run of k*+1 sweeps (and flag the launch, rerun[0], for the re-run kernel),
-// or, when the main run kept the first sweep's result (snap) and k* = 0, mark it to be
-// taken instead (ctrl[0], k_gs_take_first). ctrl[1] holds the kept sweeps either way.
-// hint (host memory, may be null): whether this solve ended after sweep 0, which decides
-// whether the next solve keeps the first sweep's result.
+// request a re-run of k*+1 sweeps (ctrl[1]) and flag the launch (rerun[0]) for the re-run kernel.
 // Lane l scans sweeps l, l+64, ...; the wave's minimum is the first such sweep.
 template <class M>
-__global__ void k_gs_decide(M m, int nsim, int N, int32_t* rerun, int snap, int32_t* hint) {
+__global__ void k_gs_decide(M m, int nsim, int N, int32_t* rerun) {
   const int e = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES;
   const int lane = threadIdx.x & (LANES - 1);
   if (e >= nsim) return;
@@ -616,29 +818,9 @@ __global__ void k_gs_decide(M m, int nsim, int N, int32_t* rerun, int snap, int3
   for (int o = LANES / 2; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, LANES));
   if (lane == 0) {
     const int kept = first < N ? first + 1 : N;
-    const bool take = snap && kept == 1 && kept < N;
-    D.ctrl[0] = take ? 1 : 0;
     D.ctrl[1] = kept < N ? kept : 0;
-    if (kept < N && !take) atomicOr(rerun, 1);
-    if (hint) *hint = kept == 1 && kept < N ? 1 : 0;
+    if (kept < N) atomicOr(rerun, 1);
   }
-}
-
-// An early exit after sweep 0 with the first sweep's result kept: copy it into the solve's
-// outputs (the faces and p the sweeps write; the ring is already there) and its max |div| into
-// the re-run's record, which is where a re-run of one sweep would have put it.
-template <class M> __global__ void k_gs_take_first(M m, int rPout) {
-  const SimDesc& D = sim_desc(m, 0);
-  if (D.ctrl[0] == 0) return;
-  const int NX = D.g.NX, NY = D.g.NY;
-  const size_t n = (size_t)NX * NY;
-  for (size_t c = threadIdx.x + (size_t)blockIdx.x * blockDim.x; c < n; c += (size_t)gridDim.x * blockDim.x) {
-    const int row = (int)(c / NY), j = (int)(c % NY);
-    if (row >= 1 && j >= 1 && j <= NY - 2) D.buf[B_U2][c] = D.buf[B_T0][c];
-    if (row >= 1 && row <= NX - 2 && j >= 1) D.buf[B_V2][c] = D.buf[B_T1][c];
-    if (row >= 1 && row <= NX - 2 && j >= 1 && j <= NY - 2) D.buf[rPout][c] = D.buf[B_T2][c];
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) D.maxdiv[D.nmax] = D.maxdiv[0];
 }
 
 static bool tile_empty_h(int g, int kb, int K, int TK, int NX) {
@@ -649,6 +831,18 @@ static bool tile_empty_h(int g, int kb, int K, int TK, int NX) {
   return rmax < 0 || rmin > NX - 1;
 }
 
+// Waves per workgroup of a tile of tk sweeps: two sweeps to a wave; one in the small tiles, whose
+// few waves leave the CU's issue slots free (4 sweeps, 256^2 jet: 0.218 ms against 0.223 with two
+// waves of two; 300x251 0.153 against 0.171). Four to a wave lost everywhere (4096^2 6.1 ms
+// against 5.7 at 16 sweeps).
+static int tile_waves(int tk) { return tk <= 4 ? tk : tk / 2; }
+static int tile_sweeps(int tk) { return tk / tile_waves(tk); }  // sweeps per wave
+// N sweeps with those that only fill the last wave: their cells pass their faces on.
+static int padded(int N, int tk) {
+  const int s = tile_sweeps(tk);
+  return (N + s - 1) / s * s;
+}
+
 // Tile geometry of one simulation for N sweeps with tk sweeps per tile and blk columns per
 // block.
 struct TileGeom {
@@ -656,71 +850,63 @@ struct TileGeom {
 };
 static TileGeom geom(int NX, int NY, int N, int tk, int blk) {
   TileGeom t;
-  t.G = (NX + N - 1 + LANES - 1) / LANES;
+  t.G = (NX + padded(N, tk) - 1 + LANES - 1) / LANES;
   t.KB = (N + tk - 1) / tk;
   const int steps = NY + LANES - 1 + tk - 1;
   t.rows = (steps + blk - 1) / blk * blk;
   return t;
 }
-// Tiles are handed out in the order their producers let them start: a tile can start about
-// 64 + 2 BLK columns after the tile one row-tile up and TK + 2 BLK after the tile one sweep block
-// back (the consumer stages a block ahead and rows are published in whole blocks), so the key
-// is that estimate of its start. Producers always get smaller keys (a topological order, which
+// Tiles are handed out in the order their producers let them start: a consumer loads a block
+// ahead, so it runs 64 + 2 BLK columns behind the tile one row-tile up, and TK + 2 BLK plus the
+// (W - 1) blocks between the first and the last wave behind the tile one sweep block back; the
+// key is that estimate of its start. Producers always get smaller keys (a topological order, which
 // the persistent kernel needs: a workgroup never waits on a tile no workgroup has taken).
 static void append_tiles(std::vector<std::pair<long long, int2>>& out, int sim, int NX, int N, int tk, int blk,
                          const TileGeom& t) {
   for (int g = 0; g < t.G; g++)
     for (int kb = 0; kb < t.KB; kb++)
-      if (!tile_empty_h(g, kb, N, tk, NX)) {
-        const long long start = (long long)(LANES + 2 * blk) * g + (long long)(tk + 2 * blk) * kb;
+      if (!tile_empty_h(g, kb, padded(N, tk), tk, NX)) {
+        const long long start = (long long)(LANES + 2 * blk) * g + (long long)(tk + (tile_waves(tk) + 1) * blk) * kb;
         long long key = (start << 32) | ((long long)sim << 12) | kb;
         out.push_back({key, make_int2(sim, (g << 16) | kb)});
       }
 }
 
-// Tile shapes the kernel is instantiated for: sweeps per tile (waves per workgroup) and columns
-// per staging/publish block.
-static bool shape_ok(int tk, int blk) {
-  return (tk == 2 || tk == 4 || tk == 8 || tk == 16) && (blk == 4 || blk == 8 || blk == 16);
+// Sweeps per tile: the knob if set; otherwise the smallest tile of which the solve has no more
+// than about one per CU (two, of eight sweeps). Small tiles spread a small grid over the CUs and
+// step faster; once there are more of them than CUs, large ones hand over less and take fewer
+// turns. Solve times in ms with 2, 4, 8, 16 sweeps: 300x251 8 sweeps 0.142 0.153 0.184 0.185;
+// 777x391 33 sweeps 0.322 0.340 0.404 0.516; 1024^2 40 sweeps 0.533 0.517 0.619 0.787; 512^2 200
+// sweeps 0.839 0.680 0.639 0.797; 2048x1024 100 sweeps 1.533 1.156 1.163 1.356; 2048^2 200 sweeps
+// 4.50 2.97 2.22 2.09; 4096^2 40 sweeps 4.38 3.29 2.86 3.19, 200 sweeps 16.0 10.5 6.8 5.7.
+int pick_tk(const fl_params& P, int NX, int N) {
+  if (P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16) return P.block_sweeps;
+  const long long G = (NX + N - 1 + LANES - 1) / LANES;
+  if (G * ((N + 1) / 2) <= 256) return 2;
+  if (G * ((N + 3) / 4) <= 256) return 4;
+  return G * ((N + 7) / 8) <= 512 ? 8 : 16;
 }
-// Sweeps per tile: the knob if set; otherwise 4 for solves of at most 8 sweeps (Simulate's own
-// count: one wave per SIMD, 300x251 frame 0.466 -> 0.447 ms), else 8: twice the tiles of 16 and
-// a shorter pipeline fill, and with its flags packed two workgroups per CU. Measured against 16
-// on the 4096^2 cavity (11.8 against 12.4 ms/step, each with its best publication) and on the
-// 256-member ensemble (17.0 against 17.6).
-int pick_tk(const fl_params& P, int N) {
-  if (P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16)
-    return P.block_sweeps;
-  return N <= 8 ? 4 : 8;
-}
-// Columns per block: the knob if set, else 8.
-int pick_blk(const fl_params& P) { return (P.block_cols == 4 || P.block_cols == 16) ? P.block_cols : 8; }
-// When handoff rows are published: on time (handoff_lag 1: GsRun.defer 0), one block late
-// (2: defer 1) or halfway through the next block (3: defer 2); automatic (0) picks halfway
-// when the tiles fill the persistent grid at least twice (the solve is throughput-bound and the
-// per-block store wait costs more than the longer pipeline fill: 4096^2 cavity 12.10 ms/step on
-// time, 12.15 one block late, 11.89 halfway), else on time.
-static int defer_handoff(const fl_params& P, int ntiles, int grid) {
-  if (P.handoff_lag >= 1 && P.handoff_lag <= 3) return P.handoff_lag - 1;
-  return ntiles >= 2 * grid ? 2 : 0;
+// Columns per block: 4 with the knob, else 8, which won at every size (4096^2 200 sweeps 5.7 ms
+// against 7.6, 512^2 0.639 against 0.651). 16, which the knob also takes, would not fit in LDS.
+int pick_blk(const fl_params& P) { return P.block_cols == 4 ? 4 : 8; }
+// The update that leaves inactive cells alone by the signs of zeros needs these; any other
+// parameters take the FULL kernels.
+static bool regular(const fl_params& P, float cp) {
+  return P.pressure_damping == 1.0f && cp > 0.0f && std::isfinite(cp) && P.relaxation > 0.0f &&
+         std::isfinite(P.relaxation);
 }
 
 // The kernel of one tile shape and launch map, and its persistent grid for `ntiles` tiles: as
 // many workgroups as fit on the device at once (and no more than there are tiles).
 template <class M> struct GsKernels {
   using Fn = void (*)(M, GsRun);
-  // snap: the instantiation that keeps the first sweep's result (single simulations only)
-  static Fn get(int tk, int blk, bool snap = false) {
-#define FL_GS_CASE(T, B)                               \
-  if (tk == T && blk == B) {                           \
-    if constexpr (std::is_same<M, OneSim>::value)      \
-      if (snap) return k_gs_wave<T, B, M, true>;       \
-    return snap ? nullptr : k_gs_wave<T, B, M, false>; \
-  }
-    FL_GS_CASE(2, 4) FL_GS_CASE(2, 8) FL_GS_CASE(2, 16)
-    FL_GS_CASE(4, 4) FL_GS_CASE(4, 8) FL_GS_CASE(4, 16)
-    FL_GS_CASE(8, 4) FL_GS_CASE(8, 8) FL_GS_CASE(8, 16)
-    FL_GS_CASE(16, 4) FL_GS_CASE(16, 8) FL_GS_CASE(16, 16)
+  static Fn get(int tk, int blk, bool full) {
+#define FL_GS_CASE(S, W, B) \
+  if (tk == S * W && blk == B) return full ? k_gs_wave<S, W, B, true, M> : k_gs_wave<S, W, B, false, M>;
+    FL_GS_CASE(1, 2, 4) FL_GS_CASE(1, 2, 8)
+    FL_GS_CASE(1, 4, 4) FL_GS_CASE(1, 4, 8)
+    FL_GS_CASE(2, 4, 4) FL_GS_CASE(2, 4, 8)
+    FL_GS_CASE(2, 8, 4) FL_GS_CASE(2, 8, 8)
 #undef FL_GS_CASE
     return nullptr;
   }
@@ -729,27 +915,26 @@ template <class M> static int occupancy_grid(int dev, int tk, int blk, int ntile
   int per_cu = 0;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 1;
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, GsKernels<M>::get(tk, blk), tk * LANES, 0);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, GsKernels<M>::get(tk, blk, false), tile_waves(tk) * LANES, 0);
   return std::max(1, std::min(ntiles, std::max(1, per_cu) * prop.multiProcessorCount));
 }
 template <class M>
-static int launch_gs(int tk, int blk, int grid, hipStream_t stream, const M& m, const GsRun& R, bool snap = false) {
-  auto fn = GsKernels<M>::get(tk, blk, snap);
+static int launch_gs(int tk, int blk, int grid, hipStream_t stream, const M& m, const GsRun& R, bool full) {
+  auto fn = GsKernels<M>::get(tk, blk, full);
   if (!fn) {
     set_error("no Gauss-Seidel kernel for " + std::to_string(tk) + " sweeps x " + std::to_string(blk) + " columns");
     return FL_ERR_INTERNAL;
   }
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(tk * LANES), 0, stream, m, R);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(tile_waves(tk) * LANES), 0, stream, m, R);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
 
 static int layout(Ctx* c, int N) {
   GsWork& W = c->gs;
-  const int tk = pick_tk(c->prm, N);
+  const int tk = pick_tk(c->prm, c->NX, N);
   const int blk = pick_blk(c->prm);
   if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
-  if (!shape_ok(tk, blk)) return FL_ERR_INTERNAL;
   FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
   pressure_free(c);
   const TileGeom t = geom(c->NX, c->NY, N, tk, blk);
@@ -766,13 +951,17 @@ static int layout(Ctx* c, int N) {
   for (auto& o : order) tiles.push_back(o.second);
   W.ntiles = (int)tiles.size();
   const size_t nt = (size_t)W.G * W.KB;
-  W.kout_elems = nt * W.rows * 3 * (LANES + 1);
-  W.gout_elems = nt * W.rows * 3 * tk;
+  const size_t kbytes = 16 * nt * W.rows * LANES, gbytes = 16 * nt * W.rows * tk;
   FL_HIP(hipMalloc(&W.d_tile, sizeof(int2) * std::max(1, W.ntiles)));
-  FL_HIP(hipMalloc(&W.d_kout, sizeof(float) * W.kout_elems));
-  FL_HIP(hipMalloc(&W.d_gout, sizeof(float) * W.gout_elems));
-  FL_HIP(hipMalloc(&W.d_prog, sizeof(int32_t) * 2 * nt));
-  FL_HIP(hipMalloc(&W.d_ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag
+  FL_HIP(hipMalloc(&W.d_kout, kbytes));
+  FL_HIP(hipMalloc(&W.d_gout, gbytes));
+  FL_HIP(hipMalloc(&W.d_kinit, (size_t)16 * W.G * (W.rows + 1) * LANES));
+  FL_HIP(hipMalloc(&W.d_ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag, solve number
+  // no word may carry a tag before a solve writes it: the words start at tag 0, the solves at 1
+  FL_HIP(hipMemsetAsync(W.d_kout, 0, kbytes, c->stream));
+  FL_HIP(hipMemsetAsync(W.d_gout, 0, gbytes, c->stream));
+  const int32_t first[4] = {0, 0, 0, 1};
+  FL_HIP(hipMemcpy(W.d_ticket, first, sizeof(first), hipMemcpyHostToDevice));
   FL_HIP(hipMemcpy(W.d_tile, tiles.data(), sizeof(int2) * W.ntiles, hipMemcpyHostToDevice));
   W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, W.ntiles);
   return FL_OK;
@@ -788,46 +977,39 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   SimDesc d = c->desc();
   d.cp = cp;
   OneSim m{d};
-  const int nprog = W.G * W.KB;
   const int mr = std::max(c->NX, c->NY);
   // Simulate's fill(p, 0) left to this solve: the initial p is zero and is not read
   const int rPin = c->gs_p_zero ? -1 : (int)B_P;
   c->gs_p_zero = false;
   hipLaunchKernelGGL(k_gs_prep, dim3(std::max(4, (mr + 255) / 256)), dim3(256), 0, c->stream, m, rPin, (int)B_T3,
-                     W.d_prog, 2 * nprog, c->d_maxdiv, 2 * c->nmax, c->d_ctrl, W.d_ticket);
+                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl, W.d_ticket);
+  const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_ticket + 3, rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
   R.ntiles = W.ntiles;
   R.K = N;
+  R.solve = W.d_ticket + 3;
   R.omega = c->d_omega;
   R.damping = c->prm.pressure_damping;
-  R.rPin = rPin;  // then p and T3 trade places
-  R.rPout = B_T3;
-  R.defer = defer_handoff(c->prm, W.ntiles, W.grid);
-  W.defer = R.defer;
+  W.lag = c->prm.handoff_lag >= 1 && c->prm.handoff_lag <= 3 ? c->prm.handoff_lag : 1;
+  const bool full = !regular(c->prm, cp);
   // without the early exit no re-run can be requested: the decision and re-run are skipped
   const int runs = c->prm.early_exit ? 2 : 1;
-  // Keep the first sweep's result (in T0-T2, scratch during the solve) when the last solve that
-  // reported back ended after sweep 0: a quiescent field then takes it instead of a re-run
-  // launch that costs as much as the main one on small grids.
-  const bool snap = runs > 1 && N > 1 && c->snap_hint && __atomic_load_n(c->snap_hint, __ATOMIC_RELAXED) != 0;
   for (int which = 0; which < runs; which++) {
     R.which = which;
     R.ticket = W.d_ticket + which;
     R.rerun = which ? W.d_ticket + 2 : nullptr;
-    if ((rc = launch_gs(W.tk, W.blk, W.grid, c->stream, m, R, snap && which == 0))) return rc;
+    if ((rc = launch_gs(W.tk, W.blk, W.grid, c->stream, m, R, full))) return rc;
     if (which == 0 && runs > 1) {
-      hipLaunchKernelGGL(k_gs_decide<OneSim>, dim3(1), dim3(LANES), 0, c->stream, m, 1, N, W.d_ticket + 2,
-                         (int)snap, N > 1 ? c->snap_hint : nullptr);
+      hipLaunchKernelGGL(k_gs_decide<OneSim>, dim3(1), dim3(LANES), 0, c->stream, m, 1, N, W.d_ticket + 2);
       FL_HIP(hipGetLastError());
-      if (snap) {
-        const int nb = (int)std::min<size_t>(1024, (c->N + 255) / 256);
-        hipLaunchKernelGGL(k_gs_take_first<OneSim>, dim3(nb), dim3(256), 0, c->stream, m, (int)B_T3);
-        FL_HIP(hipGetLastError());
-      }
     }
   }
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_ticket + 3, N, W.tk,
+                     tile_sweeps(W.tk), (int)B_T3);
+  FL_HIP(hipGetLastError());
   std::swap(c->U, c->U2);
   std::swap(c->V, c->V2);
   std::swap(c->p, c->T3);
@@ -840,7 +1022,7 @@ int pressure_free(Ctx* c) {
   if (W.d_tile) (void)hipFree(W.d_tile);
   if (W.d_kout) (void)hipFree(W.d_kout);
   if (W.d_gout) (void)hipFree(W.d_gout);
-  if (W.d_prog) (void)hipFree(W.d_prog);
+  if (W.d_kinit) (void)hipFree(W.d_kinit);
   if (W.d_ticket) (void)hipFree(W.d_ticket);
   W = GsWork{};
   return FL_OK;
@@ -851,10 +1033,15 @@ int pressure_free(Ctx* c) {
 // drains it (and one more for the members that early-exit). The initial p is read from role
 // rPin (rPin < 0: all zero, Simulate's fill(p, 0)), the solve's p written to rPout, the
 // velocity to U2, V2.
+// A batch's sweeps per tile: as for one grid, by the tiles of all members.
+static int batch_tk(const fl_params& P, const std::vector<SimDesc>& descs, int N) {
+  long long nx = 0;
+  for (const SimDesc& d : descs) nx += (d.g.NX + N - 1 + LANES - 1) / LANES * LANES;
+  return pick_tk(P, (int)std::min<long long>(std::max<long long>(nx - N + 1, 1), 1 << 30), N);
+}
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
-  const int tk = pick_tk(B->prm, N);
+  const int tk = batch_tk(B->prm, descs, N);
   const int blk = pick_blk(B->prm);
-  if (!shape_ok(tk, blk)) return FL_ERR_INTERNAL;
   auto fill = [&]() {
     for (size_t e = 0; e < descs.size(); e++) {
       const SimDesc& f = B->gs_fields[e];
@@ -864,7 +1051,7 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
       d.rows = f.rows;
       d.kout = f.kout;
       d.gout = f.gout;
-      d.prog = f.prog;
+      d.kinit = f.kinit;
     }
   };
   if (B->gs_n == N && B->tk == tk && B->blk == blk && B->gs_fields.size() == descs.size()) {
@@ -875,33 +1062,46 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   if (B->d_tiles) (void)hipFree(B->d_tiles);
   if (B->kout) (void)hipFree(B->kout);
   if (B->gout) (void)hipFree(B->gout);
-  if (B->prog) (void)hipFree(B->prog);
+  if (B->kinit) (void)hipFree(B->kinit);
+  if (B->d_skews) (void)hipFree(B->d_skews);
   if (B->ticket) (void)hipFree(B->ticket);
   B->d_tiles = nullptr;
-  B->kout = B->gout = nullptr;
-  B->prog = B->ticket = nullptr;
+  B->kout = B->gout = B->kinit = nullptr;
+  B->d_skews = nullptr;
+  B->ticket = nullptr;
   std::vector<std::pair<long long, int2>> order;
-  size_t kelems = 0, gelems = 0, nprog = 0;
+  size_t kbytes = 0, gbytes = 0, ibytes = 0;
+  std::vector<SkewItem> skews;
   std::vector<TileGeom> tg(descs.size());
   for (size_t e = 0; e < descs.size(); e++) {
     tg[e] = geom(descs[e].g.NX, descs[e].g.NY, N, tk, blk);
     append_tiles(order, (int)e, descs[e].g.NX, N, tk, blk, tg[e]);
     const size_t nt = (size_t)tg[e].G * tg[e].KB;
-    kelems += nt * tg[e].rows * 3 * (LANES + 1);
-    gelems += nt * tg[e].rows * 3 * tk;
-    nprog += 2 * nt;
+    kbytes += 16 * nt * tg[e].rows * LANES;
+    gbytes += 16 * nt * tg[e].rows * tk;
+    ibytes += (size_t)16 * tg[e].G * (tg[e].rows + 1) * LANES;
+    for (int g = 0; g < tg[e].G; g++)
+      for (int t0 = 0; t0 <= tg[e].rows; t0 += LANES) skews.push_back(SkewItem{(int)e, g, t0, 0});
   }
   std::sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
   std::vector<int2> tiles;
   for (auto& o : order) tiles.push_back(o.second);
   B->ntiles = (int)tiles.size();
   FL_HIP(hipMalloc(&B->d_tiles, sizeof(int2) * std::max(1, B->ntiles)));
-  FL_HIP(hipMalloc(&B->kout, sizeof(float) * std::max<size_t>(kelems, 1)));
-  FL_HIP(hipMalloc(&B->gout, sizeof(float) * std::max<size_t>(gelems, 1)));
-  FL_HIP(hipMalloc(&B->prog, sizeof(int32_t) * std::max<size_t>(nprog, 1)));
-  FL_HIP(hipMalloc(&B->ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag
+  FL_HIP(hipMalloc(&B->kout, std::max<size_t>(kbytes, 16)));
+  FL_HIP(hipMalloc(&B->gout, std::max<size_t>(gbytes, 16)));
+  FL_HIP(hipMalloc(&B->ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag, solve number
+  // no word may carry a tag before a solve writes it: the words start at tag 0, the solves at 1
+  FL_HIP(hipMemsetAsync(B->kout, 0, kbytes, B->stream));
+  FL_HIP(hipMemsetAsync(B->gout, 0, gbytes, B->stream));
+  FL_HIP(hipMalloc(&B->kinit, std::max<size_t>(ibytes, 16)));
+  FL_HIP(hipMalloc(&B->d_skews, sizeof(SkewItem) * std::max<size_t>(skews.size(), 1)));
+  FL_HIP(hipMemcpy(B->d_skews, skews.data(), sizeof(SkewItem) * skews.size(), hipMemcpyHostToDevice));
+  B->nskew = (int)skews.size();
+  const int32_t first[4] = {0, 0, 0, 1};
+  FL_HIP(hipMemcpy(B->ticket, first, sizeof(first), hipMemcpyHostToDevice));
   FL_HIP(hipMemcpy(B->d_tiles, tiles.data(), sizeof(int2) * B->ntiles, hipMemcpyHostToDevice));
-  size_t ko = 0, go = 0, po = 0;
+  size_t ko = 0, go = 0, io = 0;
   B->gs_fields.assign(descs.size(), SimDesc{});
   for (size_t e = 0; e < descs.size(); e++) {
     SimDesc& d = B->gs_fields[e];
@@ -910,16 +1110,15 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
     d.rows = tg[e].rows;
     d.kout = B->kout + ko;
     d.gout = B->gout + go;
-    d.prog = B->prog + po;
+    d.kinit = B->kinit + io;
     const size_t nt = (size_t)d.G * d.KB;
-    ko += nt * d.rows * 3 * (LANES + 1);
-    go += nt * d.rows * 3 * tk;
-    po += 2 * nt;
+    ko += 16 * nt * d.rows * LANES;
+    go += 16 * nt * d.rows * tk;
+    io += (size_t)16 * d.G * (d.rows + 1) * LANES;
   }
   B->tk = tk;
   B->blk = blk;
   B->gs_n = N;
-  B->gs_nprog = (int)nprog;
   B->grid = occupancy_grid<ManySims>(B->dev, tk, blk, B->ntiles);
   fill();
   return FL_OK;
@@ -929,33 +1128,37 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   ManySims m{B->d_sims, B->d_cells, B->d_rings};
   const int E = (int)B->members.size();
   hipLaunchKernelGGL(k_gs_ring<ManySims>, dim3(B->nring_items), dim3(256), 0, B->stream, m, rPin, rPout);
-  // progress counters, per-sweep maxima and re-run requests of all members are contiguous
-  hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->prog, B->gs_nprog, B->maxdiv_pool,
-                     2 * B->nmax * E, B->ctrl_pool, E, B->ticket);
+  // per-sweep maxima and re-run requests of all members are contiguous
+  hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E,
+                     B->ticket);
+  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->ticket + 3, rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = B->d_tiles;
   R.ntiles = B->ntiles;
   R.K = N;
+  R.solve = B->ticket + 3;
   R.omega = B->d_omega;
   R.damping = B->prm.pressure_damping;
-  R.rPin = rPin;
-  R.rPout = rPout;
-  R.defer = defer_handoff(B->prm, B->ntiles, B->grid);
+  // every member's cp is density h / dt with the batch's density, h and dt
+  const bool full = !regular(B->prm, B->descs.empty() ? 0.0f : B->descs[0].cp);
   const int runs = B->prm.early_exit ? 2 : 1;  // no early exit: nothing to decide or re-run
   for (int which = 0; which < runs; which++) {
     R.which = which;
     R.ticket = B->ticket + which;
     R.rerun = which ? B->ticket + 2 : nullptr;
-    int rc = launch_gs(B->tk, B->blk, B->grid, B->stream, m, R);
+    int rc = launch_gs(B->tk, B->blk, B->grid, B->stream, m, R, full);
     if (rc) return rc;
     if (which == 0 && runs > 1) {
       // one wave per member, four per workgroup
       hipLaunchKernelGGL(k_gs_decide<ManySims>, dim3((E + 3) / 4), dim3(4 * LANES), 0, B->stream, m, E, N,
-                         B->ticket + 2, 0, nullptr);
+                         B->ticket + 2);
       FL_HIP(hipGetLastError());
     }
   }
+  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->ticket + 3, N,
+                     B->tk, tile_sweeps(B->tk), rPout);
+  FL_HIP(hipGetLastError());
   return FL_OK;
 }
 

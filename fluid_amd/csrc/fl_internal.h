@@ -55,19 +55,27 @@ struct SimDesc {
   Grid g;
   float* buf[NBUF];
   uint8_t* flags;
-  uint8_t* diag;
+  uint8_t* masks;     // [2][NX][mask_pitch(NY)]: the masks of fluid neighbours of the cells a GS sweep
+                      // updates (0 elsewhere), four bits each, two cells to a byte, from column
+                      // -MASK_PAD in the first copy and -MASK_PAD - 1 in the second; written by k_masks
   uint32_t* keep;     // [NX][ceil(NY/64)]: per row and 64-column block, bit 0 some interior velocity
                       // face is not advected (advection keeps newU/newV), bit 1 some interior cell
                       // is solid (keeps newM); written by k_flags with the flags
   int32_t* ctrl;      // [4]: [1] re-run sweeps, [2] invalid sample flag, [3] GS wait timeout
   uint32_t* maxdiv;   // [2][nmax]
-  float* kout;        // GS K-stream handoff planes
-  float* gout;        // GS G-stream handoff planes
-  int32_t* prog;      // [2][G*KB] GS progress counters
+  uint8_t* kout;      // GS K-stream handoff words, 16 bytes each
+  uint8_t* gout;      // GS G-stream handoff words
+  uint8_t* kinit;     // the initial state as K-stream words, one set per row-tile
   int G, KB, rows, nmax;
   float cp;           // density*h/dt of this step
   int early_exit;
 };
+
+// A row of SimDesc::masks: its cells between at least MASK_PAD zeros on either side, which the
+// solve's loads of 16 columns read where they lie off the grid. Bytes of a row, and of both copies.
+static constexpr int MASK_PAD = 18;
+__host__ __device__ inline uint32_t mask_pitch(int NY) { return ((uint32_t)NY + 2 * MASK_PAD + 3) / 2; }
+inline size_t mask_bytes(int NX, int NY) { return 2 * (size_t)NX * mask_pitch(NY); }
 
 // A 64x4 block of cells of one simulation (batched cell kernels) and a 256-cell chunk
 // of one simulation's ring (batched ring kernels).
@@ -76,6 +84,10 @@ struct CellItem {
 };
 struct RingItem {
   int sim, blk;
+};
+// 64 rows of handoff words, from row t0, of a row-tile of one simulation.
+struct SkewItem {
+  int sim, g, t0, pad;
 };
 
 // Workgroups are dispatched to the 8 XCDs in turn (workgroup b runs on XCD b % 8), and each
@@ -100,20 +112,19 @@ struct ManySims {
 
 // Pressure workspace of the temporal-blocked Gauss-Seidel kernel.
 struct GsWork {
-  int tk = 0;              // sweeps per tile (waves per workgroup)
-  int blk = 0;             // columns per staging/publish block
+  int tk = 0;              // sweeps per tile
+  int blk = 0;             // columns per block
   int n_alloc = -1;        // sweep count the layout was built for
   int G = 0, KB = 0;       // tiles along skewed rows and along sweeps
   int rows = 0;            // handoff rows per tile (= steps per tile)
   int ntiles = 0;          // non-empty tiles in ticket order
   int grid = 0;            // persistent workgroups launched
-  int defer = -1;          // handoff publication of the last solve (GsRun.defer; -1: none yet)
+  int lag = 0;             // handoff_lag of the last solve (0: none yet)
   int32_t* d_tile = nullptr;    // [ntiles] packed (g << 16 | kb), ticket order
-  float* d_kout = nullptr;      // [G*KB][rows][3][65]  K-stream handoff planes U, V, p
-  float* d_gout = nullptr;      // [G*KB][rows][3][tk]  G-stream handoff planes
-  int32_t* d_prog = nullptr;    // [2][G*KB] progress counters (main run, rerun)
-  int32_t* d_ticket = nullptr;  // [2]
-  size_t kout_elems = 0, gout_elems = 0;
+  uint8_t* d_kout = nullptr;    // [G*KB][rows][64] K-stream handoff words
+  uint8_t* d_gout = nullptr;    // [G*KB][rows][tk] G-stream handoff words
+  uint8_t* d_kinit = nullptr;   // [G][rows + 1][64] the initial state as K-stream words
+  int32_t* d_ticket = nullptr;  // [4]: tickets of the main run and the re-run, re-run flag, solve number
 };
 
 struct Batch;
@@ -139,8 +150,7 @@ struct Ctx {
   float *T0 = nullptr, *T1 = nullptr, *T2 = nullptr, *T3 = nullptr;  // BFECC / curl scratch
   uint8_t* flags = nullptr;      // cell flags, i-major
   uint32_t* keep = nullptr;      // SimDesc::keep
-  int32_t* snap_hint = nullptr;  // host-pinned: the last solve that reported back ended after sweep 0
-  uint8_t* flags_diag = nullptr; // cell flags, anti-diagonal-major [d=i+j][i]
+  uint8_t* masks = nullptr;      // SimDesc::masks
   bool flags_dirty = true;
 
   // Solver control block on the device.
@@ -213,13 +223,13 @@ struct Ctx {
     float* b[NBUF] = {U, V, nU, nV, p, S, M, nM, U2, V2, M2, T0, T1, T2, T3};
     for (int k = 0; k < NBUF; k++) d.buf[k] = b[k];
     d.flags = flags;
-    d.diag = flags_diag;
+    d.masks = masks;
     d.keep = keep;
     d.ctrl = d_ctrl;
     d.maxdiv = d_maxdiv;
     d.kout = gs.d_kout;
     d.gout = gs.d_gout;
-    d.prog = gs.d_prog;
+    d.kinit = gs.d_kinit;
     d.G = gs.G;
     d.KB = gs.KB;
     d.rows = gs.rows;
@@ -237,7 +247,7 @@ struct Batch {
   std::vector<Ctx*> members;
   float* pool[NBUF] = {};
   uint8_t* flags_pool = nullptr;
-  uint8_t* diag_pool = nullptr;
+  uint8_t* mask_pool = nullptr;
   uint32_t* keep_pool = nullptr;
   int32_t* ctrl_pool = nullptr;
   uint32_t* maxdiv_pool = nullptr;
@@ -251,13 +261,15 @@ struct Batch {
   int ncell_items = 0, nring_items = 0;
   std::vector<SimDesc> descs;  // what d_sims holds
   // batched Gauss-Seidel layout
-  int tk = 0, blk = 0, gs_n = -1, gs_nprog = 0;
+  int tk = 0, blk = 0, gs_n = -1;
   int ntiles = 0, grid = 0;
-  std::vector<SimDesc> gs_fields;  // per member: G, KB, rows and its handoff/progress slices
+  std::vector<SimDesc> gs_fields;  // per member: G, KB, rows and its handoff slices
   int2* d_tiles = nullptr;
-  float* kout = nullptr;
-  float* gout = nullptr;
-  int32_t* prog = nullptr;
+  uint8_t* kout = nullptr;
+  uint8_t* gout = nullptr;
+  uint8_t* kinit = nullptr;
+  SkewItem* d_skews = nullptr;
+  int nskew = 0;
   int32_t* ticket = nullptr;
   float* d_omega = nullptr;
   int omega_n = -1;
@@ -351,7 +363,7 @@ int batch_apply_sources(Batch* B);
 int batch_apply_edits(Batch* B, const uint32_t* keys, const float* vals, const int32_t* seg, const int32_t* segsim,
                       int nseg);
 // batched pressure solve (fl_gs_wave.hip): sets the GS fields of `descs`
-int pick_tk(const fl_params& P, int N);
+int pick_tk(const fl_params& P, int NX, int N);
 bool gs_wave_supported(Ctx* c, int numIters);
 int pick_blk(const fl_params& P);
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs);

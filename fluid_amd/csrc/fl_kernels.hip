@@ -136,15 +136,38 @@ template <class M> __global__ void k_flags(M m) {
   if (interior) f |= CF_INTERIOR;
   if (interior && fluid && (f & (CF_X0 | CF_X1 | CF_Y0 | CF_Y1))) f |= CF_GS;
   d->flags[c] = (uint8_t)f;
-  d->diag[(size_t)(i + j) * NX + i] = (uint8_t)f;
   // the keep map: a wavefront is one row's 64-column block (BX = 64 lanes from j = 64*block)
   const bool kv = interior && !(fluid && (f & CF_X0) && (f & CF_Y0)), ks = interior && !fluid;
   const uint32_t kb = (wave_any(kv) ? 1u : 0u) | (wave_any(ks) ? 2u : 0u);
   if ((j & (BX - 1)) == 0) d->keep[i * ((NY + BX - 1) / BX) + j / BX] = kb;
 }
 
+// SimDesc::masks from the flags: one thread per cell (i, j) writes the byte of columns j, j + 1 of
+// the copy with j's parity; the first column also writes the byte of columns -1, 0 of the odd copy.
+template <class M> __global__ void k_masks(M m) {
+  const SimDesc* d;
+  int i, j;
+  if (!cell_of(m, d, i, j)) return;
+  const int NX = d->g.NX, NY = d->g.NY;
+  const uint32_t pitch = mask_pitch(NY);
+  auto mask = [&](int x) -> uint32_t {
+    const uint32_t f = x < NY ? d->flags[(size_t)i * NY + x] : 0;
+    return (f & CF_GS) ? (f >> 1) & 0xFu : 0u;
+  };
+  uint8_t* row = d->masks + (size_t)i * pitch + MASK_PAD / 2;
+  const uint32_t lo = mask(j), hi = mask(j + 1);
+  if (j & 1)
+    row[(size_t)NX * pitch + (j + 1) / 2] = (uint8_t)(lo | hi << 4);
+  else
+    row[j / 2] = (uint8_t)(lo | hi << 4);
+  if (j == 0) row[(size_t)NX * pitch] = (uint8_t)(lo << 4);
+}
+
 int launch_flags(Ctx* c) {
-  launch_cells(c, [](const OneSim& m, dim3 g, dim3 b, hipStream_t s) { hipLaunchKernelGGL(k_flags<OneSim>, g, b, 0, s, m); });
+  launch_cells(c, [](const OneSim& m, dim3 g, dim3 b, hipStream_t s) {
+    hipLaunchKernelGGL(k_flags<OneSim>, g, b, 0, s, m);
+    hipLaunchKernelGGL(k_masks<OneSim>, g, b, 0, s, m);
+  });
   FL_HIP(hipGetLastError());
   c->flags_dirty = false;
   return FL_OK;
@@ -968,6 +991,7 @@ int batch_swap_roles(Batch* B, int a, int b) {
 }
 int batch_flags(Batch* B) {
   hipLaunchKernelGGL(k_flags<ManySims>, FL_BATCH_CELLS(B), many(B));
+  hipLaunchKernelGGL(k_masks<ManySims>, FL_BATCH_CELLS(B), many(B));
   FL_HIP(hipGetLastError());
   return FL_OK;
 }

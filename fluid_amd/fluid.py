@@ -86,8 +86,8 @@ def _init_knobs(o):
     # Addition: back-trace in cell units (no reference counterpart; off = the reference's
     # absolute-position arithmetic, bit for bit).
     o.PreciseAdvection = False
-    o.HandoffLag = 0     # temporal-blocked solve: 0 auto, 1 on time, 2 one block late
-    o.BlockCols = 0      # temporal-blocked solve: columns per block, 0 auto (8), 4, 8 or 16
+    o.HandoffLag = 0     # temporal-blocked solve: accepted (0 to 3), all run alike
+    o.BlockCols = 0      # temporal-blocked solve: columns per block, 0 auto (8), 4, 8 or 16 (as 8)
 
 
 def _params_of(o):

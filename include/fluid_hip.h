@@ -68,15 +68,13 @@ typedef struct fl_params {
   int32_t pressure_iters;    /* sweeps per Simulate, default 8 */
   int32_t early_exit;        /* 1: stop after the first sweep with maxDiv < 1e-5 */
   int32_t solver;            /* 0 auto, 1 hyperplane kernel, 2 temporal-blocked kernel */
-  int32_t block_sweeps;      /* sweeps per temporal block: 0 auto (8; 4 for at most 8 sweeps),
-                                2, 4, 8 or 16 */
+  int32_t block_sweeps;      /* sweeps per temporal block: 0 auto (by the number of tiles that the
+                                grid and the sweeps make), 2, 4, 8 or 16 */
   int32_t precise_advection; /* 1: back-trace in cell units (no reference counterpart), default 0 */
-  int32_t handoff_lag;       /* temporal-blocked solve: 0 auto, 1 publish each block's handoff rows
-                                at the next block's start, 2 one block later (fewer waits, longer
-                                pipeline fill), 3 halfway through the next block; auto picks 3
-                                from two rounds of tiles up, else 1 */
-  int32_t block_cols;        /* temporal-blocked solve: columns per staging and publish block,
-                                0 auto (8), 4, 8 or 16 */
+  int32_t handoff_lag;       /* temporal-blocked solve: accepted (0 to 3) and reported; handoff words
+                                are published as they are computed, so all values run alike */
+  int32_t block_cols;        /* temporal-blocked solve: columns between two barriers of a workgroup,
+                                0 auto (8), 4, 8 or 16 (run as 8) */
 } fl_params;
 
 /* Statistics of the last Simulate (no reference counterpart). */
@@ -140,7 +138,7 @@ int fl_sweep_maxdiv(fl_ctx* ctx, float* out, int cap, int* count);
 typedef struct fl_gs_layout {
   int32_t sweeps_per_tile;  /* TK */
   int32_t cols_per_block;   /* BLK: columns per staging and publication block */
-  int32_t handoff_lag;      /* publication used: 1 on time, 2 one block late, 3 halfway */
+  int32_t handoff_lag;      /* params.handoff_lag of the last solve, 1 if auto */
   int32_t row_tiles;        /* G: tiles along the skewed rows (64 rows each) */
   int32_t sweep_blocks;     /* KB: tiles along the sweeps */
   int32_t steps_per_tile;   /* column steps each tile runs */
@@ -235,7 +233,7 @@ int fl_scene_draw_line(fl_ctx* ctx, int x0, int y0, int x1, int y1, int solid); 
 int fl_scene_smoke_brush(fl_ctx* ctx, int ci, int cj, int radius, float strength); /* main.go:453 */
 
 /* Gauss-Seidel tile-shape autotuner for one context: times the candidate shapes (sweeps per
- * tile, columns per block, handoff publication) of the temporal-blocked solve on the current
+ * tile, columns per block) of the temporal-blocked solve on the current
  * state (which it leaves unchanged), re-times the three fastest, and keeps the best in
  * params.block_sweeps, block_cols and handoff_lag. The reference has no counterpart (its
  * solve is a serial loop, fluid.go:188-234). */

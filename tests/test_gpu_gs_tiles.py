@@ -1,0 +1,55 @@
+"""The temporal-blocked solve at the edges of its tiles, bit for bit against the oracle: grids of
+one cell, one lane more or less than a 64-row tile and one column more or less than a block of
+columns; sweep counts that do not fill a tile or a wave's pair of sweeps; blocks of cells with all
+neighbours, walls only and scattered solids; the parameters that need the selecting update
+(damping, negative relaxation and dt); faces that are infinite or NaN. The tolerance is zero: the
+solve performs the oracle's float32 operations in the oracle's order (NaN compares by position)."""
+import numpy as np
+import pytest
+
+from fluid_amd import Fluid
+from oracle.pyoracle import OracleFluid
+
+pytestmark = pytest.mark.gpu
+
+
+def run(w, h, sweeps, tk, blk, solid=0.03, early=False, dt=0.1, special=False, steps=2, **knobs):
+    rng = np.random.default_rng([w, h, sweeps])
+    shape = (w + 2, h + 2)
+    st = {"S": (rng.random(shape) >= solid).astype(np.float32)}
+    st["S"][0, :] = 0
+    for k in ("U", "V", "newU", "newV"):
+        st[k] = (0.5 * rng.standard_normal(shape)).astype(np.float32)
+    if special:
+        for k, v in (("U", np.inf), ("V", -np.inf), ("U", np.nan), ("V", 1e-42), ("U", -0.0)):
+            st[k][tuple(rng.integers(0, n) for n in shape)] = v
+    g, o = Fluid(1000.0, w, h, 0.01), OracleFluid(1000.0, w, h, 0.01)
+    for f in (g, o):
+        f.load_state(st)
+        f.PressureIters, f.EarlyExit = sweeps, early
+        for k, v in knobs.items():
+            setattr(f, k, v)
+    g.Solver, g.BlockSweeps, g.BlockCols = 2, tk, blk
+    for step in range(steps):
+        g.Simulate(dt)
+        o.Simulate(dt)
+        for k in ("U", "V", "p"):
+            a, b = g.get(k), o.get(k)
+            bad = (a.view(np.uint32) != b.view(np.uint32)) & ~(np.isnan(a) & np.isnan(b))
+            assert not bad.any(), "step %d: %s differs at %d cells, first %s" % (
+                step, k, int(bad.sum()), np.argwhere(bad)[0])
+    g.close()
+
+
+@pytest.mark.parametrize("tk,blk", [(tk, blk) for tk in (0, 2, 4, 8, 16) for blk in (4, 8)])
+@pytest.mark.parametrize("w,h,sweeps", [(1, 1, 1), (1, 9, 3), (62, 7, 5), (63, 8, 16), (65, 17, 19), (130, 33, 33)])
+def test_edges_of_tiles(w, h, sweeps, tk, blk):
+    run(w, h, sweeps, tk, blk)
+
+
+@pytest.mark.parametrize("tk,blk", [(2, 8), (4, 4), (8, 8), (16, 8)])
+@pytest.mark.parametrize("case", [dict(solid=0.0), dict(solid=0.5), dict(PressureDamping=0.75),
+                                  dict(Relaxation=-0.5), dict(dt=-0.05), dict(early=True, solid=0.9),
+                                  dict(special=True, steps=1)], ids=str)
+def test_cells_and_parameters(case, tk, blk):
+    run(150, 41, 21, tk, blk, **case)
