@@ -36,7 +36,7 @@ static void batch_free(Batch* B) {
     if (p) (void)hipFree(p);
   for (void* p : {(void*)B->flags_pool, (void*)B->mask_pool, (void*)B->keep_pool, (void*)B->ctrl_pool, (void*)B->maxdiv_pool,
                   (void*)B->d_sims, (void*)B->d_cells, (void*)B->d_rings, (void*)B->d_tiles, (void*)B->kout,
-                  (void*)B->gout, (void*)B->kinit, (void*)B->d_skews, (void*)B->ticket, (void*)B->d_omega, (void*)B->d_src,
+                  (void*)B->gout, (void*)B->kinit, (void*)B->d_skews, (void*)B->state, (void*)B->d_first, (void*)B->d_omega, (void*)B->d_src,
                   (void*)B->d_src_seg, (void*)B->d_src_sim, (void*)B->d_ekeys, (void*)B->d_evals,
                   (void*)B->d_eseg, (void*)B->d_esim})
     if (p) (void)hipFree(p);

@@ -19,9 +19,10 @@
 // The solve is a wavefront over a chain of dependent steps, so its time is steps times the time
 // of a step, not memory or arithmetic rate; and a step is the issue of one wave's instructions: a
 // lone wave issues an independent vector instruction every 4.7 cycles, a dependent one after 8,
-// a 16-byte LDS write takes 28 and a 4-byte one 16 (measured). So a step is about 15 vector
-// instructions per sweep and the few LDS accesses around them: 280 cycles for one sweep to a
-// wave, 340 for two, 530 for four, where one sweep a wave with a barrier a step took 640.
+// a 16-byte LDS write takes 28 and a 4-byte one 16 (measured). So a step is about 18 vector
+// instructions per sweep and the few LDS accesses around them: 160 cycles for one sweep to a
+// wave, 270 for two, and 60 more for its share of the block's loads, checks and barrier; one
+// sweep a wave with a barrier a step took 640.
 //
 // The waves of a workgroup run one block of B steps apart, with one barrier per block: wave
 // w runs block n while wave w-1 runs block n+1 into the other half of their LDS buffer. Between
@@ -31,13 +32,18 @@
 // of the solve, in each half, and the consumer loads the words until they carry the tag of this
 // solve. So a handoff costs one trip of the data: no wait for stores, no progress counters, no
 // polls beside the loads themselves. A block's words are loaded while the block before it runs.
-// Tiles run as a persistent kernel in ticket order (a topological order of the tile graph), so
+// The compiler has to know
+// how many stores were issued since a load to wait for the load alone, so every path of a block issues
+// the same loads and stores, under branches that it sees are uniform
+// (with a wait for the stores 256^2 took 0.180 ms, 512^2 0.540). Tiles run as a persistent kernel in ticket order (a topological order of the tile graph), so
 // whatever a workgroup waits for was taken earlier by a workgroup that runs. k_gs_skew lays the
 // initial state out as K-stream words and k_gs_unskew takes the last sweep's back, so tiles
 // read and write nothing but words, whole lines at a time.
 //
-// Solves, start of the change to this form -> now: 256^2 40 sweeps 0.49 -> 0.21 ms, 300x251 8
-// sweeps 0.42 -> 0.14, 512^2 200 sweeps 1.32 -> 0.64, 4096^2 200 sweeps 10.5 -> 5.7.
+// What it measured, one sweep a wave with a barrier a step -> now: 256^2 40 sweeps 0.49 -> 0.154 ms,
+// 300x251 8 sweeps 0.42 -> 0.110, 512^2 200 sweeps 1.32 -> 0.473, 4096^2 200 sweeps 10.5 -> 5.04.
+// At 4096^2 the two waves of a SIMD are bound by their issue: 43 instructions a step of two
+// sweeps, 34 of them the shifts and updates.
 //
 // Cells outside the interior or solid pass their faces through unchanged, exactly like
 // the skipped cells of the serial loop. Faces no interior cell touches keep their input
@@ -59,15 +65,33 @@ namespace fl {
 static constexpr int LANES = 64;
 static constexpr int SPIN_LIMIT = 1 << 20;     // bounded wait (about a second); then error and continue
 
+// Tiles whose K streams stay in one XCD's L2 (queue_of_tiles).
+__host__ __device__ constexpr bool near_tiles(int tk) { return tk == 16; }
+static constexpr int MAXQ = 16;  // queues of tiles, one per XCD
+// The counters of one launch (main run or re-run), zero before it.
+struct GsCounters {
+  int32_t ticket[MAXQ + 1];  // of each XCD's queue, and of all tiles in one
+  int32_t here;              // XCDs of which a workgroup has started, a bit each
+  int32_t mode;              // how the launch hands out its tiles (MODE_NEAR, MODE_FAR), 0 before it is known
+};
+// A solve's state on the device: the counters of its two launches; whether some simulation asks for
+// the re-run; the number of the solve, from which its tags are made (kept from solve to solve).
+struct GsState {
+  GsCounters run[2];
+  int32_t rerun, solve;
+};
+enum { MODE_NEAR = 1, MODE_FAR = 2 };
+
 // One launch of the solve (main run or early-exit re-run).
 struct GsRun {
-  const int2* tiles;  // ticket order: (simulation, (g << 16) | kb)
-  int ntiles;
+  const int2* tiles;  // (simulation, (g << 16) | kb): each queue's tiles in ticket order, then all of them
+  const int* first;   // [nq + 2] where each queue's tiles begin, then all tiles, and the end
+  int nq;             // 0: all tiles from one queue
   int which;          // 0 main run (K sweeps), 1 re-run (ctrl[1] sweeps of each simulation)
   int K;
-  int32_t* ticket;
+  GsCounters* count;
   const int32_t* rerun;  // re-run launch only: nonzero when some simulation asked for one
-  const int32_t* solve;  // the number of this solve, from which its tags are made
+  const int32_t* solve;
   const float* omega;
   float damping;
 };
@@ -87,20 +111,21 @@ __device__ __forceinline__ bool tile_empty(int g, int kb, int K, int TK, int NX)
 // last solves. Device-coherent accesses (sc1), so that neither side needs a cache writeback or
 // invalidate.
 typedef uint32_t word4 __attribute__((ext_vector_type(4)));
-static constexpr int SC1 = 16, VOLATILE_OP = (int)0x80000000;  // cache policy of the buffer intrinsics
+static constexpr int CACHED = 0, SC1 = 16, VOLATILE_OP = (int)0x80000000;  // cache policy of the buffer intrinsics
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t word_buffer(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffff, 0x00027000);
 }
 __device__ __forceinline__ word4 ld_word(__amdgpu_buffer_rsrc_t b, uint32_t byte) {
   return __builtin_amdgcn_raw_buffer_load_b128(b, byte, 0, SC1 | VOLATILE_OP);
 }
+template <int POLICY>
 __device__ __forceinline__ void st_word(__amdgpu_buffer_rsrc_t b, uint32_t byte, float u, float v, float p, uint32_t tag) {
   word4 w;
   w.x = __float_as_uint(u);
   w.y = (__float_as_uint(v) & 0xffffu) | (tag << 16);
   w.z = __float_as_uint(p);
   w.w = __builtin_amdgcn_alignbit(tag, __float_as_uint(v), 16);
-  __builtin_amdgcn_raw_buffer_store_b128(w, b, byte, 0, SC1);
+  __builtin_amdgcn_raw_buffer_store_b128(w, b, byte, 0, POLICY);
 }
 // Zero in the upper 16 bits when both halves carry the tag.
 __device__ __forceinline__ uint32_t word_tag(word4 w, uint32_t tag) { return (w.y ^ (tag << 16)) | (w.w ^ (tag << 16)); }
@@ -119,6 +144,12 @@ __device__ __forceinline__ float from_lane_below(float first, float v) {
   return __int_as_float(
       __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138, 0xF, 0xF, false));
 }
+// Lane a takes lane a+1's v; lane 63 takes its own `last`.
+__device__ __forceinline__ float from_lane_above(float last, float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(__float_as_int(last), __float_as_int(v), 0x130, 0xF, 0xF, false));
+}
+__device__ __forceinline__ bool every_lane(bool v) { return __builtin_amdgcn_ballot_w64(!v) == 0; }
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ float uniform(float v) { return __int_as_float(uniform(__float_as_int(v))); }
 
@@ -219,19 +250,16 @@ __device__ __forceinline__ void update_any(Cells<S>& x, float (&md)[S], const fl
   }
 }
 
-// The masks of a sweep's cells in a row, four bits each, eight steps to a word; loaded sixteen
-// steps at a time, at any byte.
-typedef uint32_t word2_any __attribute__((ext_vector_type(2), aligned(1)));
-typedef uint32_t word4_any __attribute__((ext_vector_type(4), aligned(1)));
-static constexpr int MASK_STEPS = 16;
+// The masks of a block's cells of a sweep in a row, four bits each; loaded from any byte.
+typedef uint32_t mask8_any __attribute__((aligned(1)));
+typedef uint16_t mask4_any __attribute__((aligned(1)));
 
 template <int S, int W, int B> struct GsShared {
   static constexpr int GP = (3 * S + 3 + 3) / 4 * 4;  // pitch of a Gi row, one float before and two after it
-  float4 K[W][2][B][LANES];    // K[w]: the rows (U, V, p) wave w's first sweep reads
+  float4 K[W > 1 ? W - 1 : 1][2][B][W > 1 ? LANES : 1];  // K[w - 1]: the rows (U, V, p) wave w's first sweep reads
   float Gi[W][B + 1][GP];      // boundary below lane 0: V, p of the sweep before, U of this one
-  float4 Go[W][B][S];          // lane 63's U, V, p of each sweep
   float4 tabw[16], tabd[16];   // CellW by mask
-  int tile;
+  int tile, far;
 };
 
 // How a block's cells are updated: all plain; with weights looked up once (along a wall, say: every
@@ -240,42 +268,20 @@ enum { BLOCK_PLAIN, BLOCK_SAME, BLOCK_ANY };
 // Where a wave's rows go: to the next wave's LDS rows, or to memory as handoff words.
 enum { OUT_LDS, OUT_WORDS };
 
-// Lane 63's U, V, p of S sweeps to LDS words off.. (four per sweep) of `at`. One change of the exec
-// mask and back for all of them: a branch would cut the block's straight code in pieces, and a
-// store by every lane would take the LDS bandwidth that the waves' rows need.
-template <int S>
-__device__ __forceinline__ void store_lane63(uint32_t at, int off, const float (&U)[S], const float (&V)[S],
-                                             const float (&p)[S]) {
-  if constexpr (S == 1) {
-    asm volatile(
-        "s_mov_b64 exec, %0\n\t"
-        "ds_write2_b32 %1, %2, %3 offset0:%5 offset1:%6\n\t"
-        "ds_write_b32 %1, %4 offset:%7\n\t"
-        "s_mov_b64 exec, -1" ::"s"(1ull << 63),
-        "v"(at), "v"(U[0]), "v"(V[0]), "v"(p[0]), "n"(off), "n"(off + 1), "n"(4 * (off + 2)));
-  } else {
-    static_assert(S == 2, "one or two sweeps per wave");
-    asm volatile(
-        "s_mov_b64 exec, %0\n\t"
-        "ds_write2_b32 %1, %2, %3 offset0:%8 offset1:%9\n\t"
-        "ds_write2_b32 %1, %4, %5 offset0:%10 offset1:%11\n\t"
-        "ds_write2_b32 %1, %6, %7 offset0:%12 offset1:%13\n\t"
-        "s_mov_b64 exec, -1" ::"s"(1ull << 63),
-        "v"(at), "v"(U[0]), "v"(V[0]), "v"(p[0]), "v"(U[1]), "v"(V[1]), "v"(p[1]), "n"(off), "n"(off + 1),
-        "n"(off + 2), "n"(off + 4), "n"(off + 5), "n"(off + 6));
-  }
-}
-
 // One block of B steps of a wave. gi, Kin: this block's boundary rows in LDS (Kin, Kout at this
-// lane); k: the first step's K row; mk: the masks. Each step
+// lane); k: the first step's K row; mk: the masks. A FIRST wave's rows are the words kw instead,
+// row u for step u. Each step
 // first takes what it needs from its neighbours (the loads of the step before have arrived),
 // then stores what the step before left, loads for the next step, and updates: so no step waits
 // for its own LDS traffic. The code of a block is straight, a copy for each mode and output.
-template <int S, int B, int GP, int MODE, int OUT, bool FULL>
-__device__ __forceinline__ void run_block(Sweeps<S>& Q, float (&k)[3], const uint32_t (&mk)[S], const float* gi,
-                                          const float4* Kin, float4* Kout, uint32_t go, const char* tab,
-                                          __amdgpu_buffer_rsrc_t kbuf, uint32_t kbyte, uint32_t tag, float damping,
-                                          float cp) {
+// go: lane 63's U, V, p of each sweep after step u, at lane 64 - B + u: every step shifts them down
+// a lane and lets lane 63 in, one instruction a value into the register that the value leaves (a
+// store of lane 63 to LDS took two exec changes and two writes, 44 cycles a step for one sweep).
+template <int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL>
+__device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST ? B : 1], float (&k)[3],
+                                          const uint32_t (&mk)[S], const float* gi, const float4* Kin, float4* Kout,
+                                          float (&go)[S][3], const char* tab, __amdgpu_buffer_rsrc_t kbuf,
+                                          uint32_t kbyte, uint32_t tag, float damping, float cp) {
   constexpr int GN = (3 * S + 3) / 4 * 4;
   float g[2][GN], kr[2][3];  // the boundary and K rows of this step and the next, in turn
   CellW cw[S], cn[S];
@@ -291,6 +297,7 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, float (&k)[3], const uin
     }
   };
   auto load_k = [&](int u) {  // what step u reads
+    if constexpr (FIRST) return;
     const float4 v = Kin[(u - 1) * LANES];
     kr[u % 2][0] = v.x;
     kr[u % 2][1] = v.y;
@@ -308,19 +315,33 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, float (&k)[3], const uin
     if constexpr (OUT == OUT_LDS)
       Kout[u * LANES] = make_float4(Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], 0.0f);
     else
-      st_word(kbuf, kbyte + u * (LANES * 16), Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], tag);
-    store_lane63<S>(go, 4 * S * u, Q.UrO, Q.VbO, Q.pO);
+      st_word<POLICY>(kbuf, kbyte + u * (LANES * 16), Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], tag);
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      go[c][0] = from_lane_above(Q.UrO[c], go[c][0]);
+      go[c][1] = from_lane_above(Q.VbO[c], go[c][1]);
+      go[c][2] = from_lane_above(Q.pO[c], go[c][2]);
+    }
   };
   load_gi(0);
   load_gi(1);
   load_k(1);
+  if constexpr (!FIRST) {
 #pragma unroll
-  for (int f = 0; f < 3; f++) kr[0][f] = k[f];
+    for (int f = 0; f < 3; f++) kr[0][f] = k[f];
+  }
+#pragma unroll
+  for (int c = 0; c < S; c++) go[c][0] = go[c][1] = go[c][2] = 0.0f;
   if constexpr (MODE != BLOCK_PLAIN) load_cw(0, cw);
 #pragma unroll
   for (int u = 0; u < B; u++) {
     Cells<S> x;
     float pnext[S];
+    if constexpr (FIRST) {
+      kr[u % 2][0] = word_u(kw[u]);
+      kr[u % 2][1] = word_v(kw[u]);
+      kr[u % 2][2] = word_p(kw[u]);
+    }
 #pragma unroll
     for (int c = 0; c < S; c++) {
       x.Ul[c] = from_lane_below(g[u % 2][3 * c + 2], Q.UrO[c]);
@@ -357,19 +378,47 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, float (&k)[3], const uin
     }
   }
   put(B - 1);
+  if constexpr (!FIRST) {
 #pragma unroll
-  for (int f = 0; f < 3; f++) k[f] = kr[0][f];
-  asm volatile("" ::: "memory");  // lane 63's stores are not known to the compiler
+    for (int f = 0; f < 3; f++) k[f] = kr[0][f];
+  }
 }
 
-typedef __attribute__((address_space(3))) float lds_float;
+// The queue a workgroup takes its tiles from (called by one thread of it). A row-tile's tiles are
+// all in the queue of one XCD, so that their K streams, one 1 KB row a step each, stay in that XCD's
+// L2 (written through to memory, the 4096^2 solve took 5.81 ms
+// against 5.04, 2048^2 1.99 against 1.72). Only for tiles of 16 sweeps, which make
+// more rows than XCDs: on small grids whole rows divide unevenly (512^2 0.530 ms against 0.475): a workgroup serves the XCD that it runs on. Each queue needs a workgroup, or tiles
+// would wait for ever for those of a queue without one, so the first workgroups wait until one has
+// started on every XCD (a few microseconds). If that fails (an XCD that is busy with something
+// else, or kept from this stream) the launch takes all tiles from one queue instead and writes
+// its L2 back after every block, slowly.
+static __device__ int queue_of_tiles(const GsRun& R) {
+  const int q = __builtin_amdgcn_s_getreg(20 | (3 << 11)) % R.nq;  // HW_REG_XCC_ID, 4 bits
+  GsCounters* C = R.count;
+  int seen = atomicOr(&C->here, 1 << q) | 1 << q;
+  const int all = (1 << R.nq) - 1;
+  int mode = 0;
+  for (int it = 0; seen != all && it < 256 && !mode; it++) {
+    __builtin_amdgcn_s_sleep(4);
+    seen = ld_err(&C->here);
+    mode = ld_err(&C->mode);
+  }
+  if (!mode) {
+    const int want = seen == all ? MODE_NEAR : MODE_FAR, was = atomicCAS(&C->mode, 0, want);
+    mode = was ? was : want;
+  }
+  return mode == MODE_NEAR ? q : R.nq;
+}
+
+typedef __attribute__((address_space(3))) float lds_float;  // a pointer that lanes compute stays an LDS one
 
 // S sweeps per wave, W waves per workgroup (TK = S W sweeps per tile), B columns per block.
 template <int S, int W, int B, bool FULL, class M>
 __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun R) {
   constexpr int TK = S * W, GP = GsShared<S, W, B>::GP;
+  constexpr bool NEAR = near_tiles(TK);
   constexpr uint32_t BITS = B == 4 ? 0xFFFFu : 0xFFFFFFFFu;  // of a word of masks that a block uses
-  constexpr int MB = MASK_STEPS / B;                         // blocks a load of masks holds
   constexpr uint32_t KROW = 16 * LANES, GROW = 16 * TK;      // bytes of a row of words
   static_assert(B * (S + 1) <= LANES, "a lane loads one G word per block");
   __shared__ GsShared<S, W, B> sh;
@@ -383,19 +432,23 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     sh.tabw[threadIdx.x] = c.w;
     sh.tabd[threadIdx.x] = c.d;
   }
+  const int queue = NEAR && threadIdx.x == 0 ? queue_of_tiles(R) : 0;
   const uint32_t tag0 = 2u * (uint32_t)uniform(*R.solve) & 0xffffu, tag = (tag0 + (uint32_t)R.which) & 0xffffu;
   int vzero = 0;  // a zero the compiler keeps in a vector register: LDS addresses built on it stay there too
   asm volatile("" : "+v"(vzero));
   const float* gi = &sh.Gi[w][1][0] + vzero;
-  const uint32_t go = (uint32_t)(uintptr_t)(lds_float*)&sh.Go[w][0][0] + vzero;
   const char* tab = reinterpret_cast<const char*>(sh.tabw);
 
   for (;;) {
-    if (threadIdx.x == 0) sh.tile = atomicAdd(R.ticket, 1);
+    if (threadIdx.x == 0) {
+      const int t = R.first[queue] + atomicAdd(&R.count->ticket[queue], 1);
+      sh.tile = t < R.first[queue + 1] ? t : -1;
+      sh.far = NEAR && queue == R.nq;
+    }
     __syncthreads();
-    const int t = uniform(sh.tile);
+    const int t = uniform(sh.tile), far = uniform(sh.far);
     __syncthreads();
-    if (t >= R.ntiles) break;
+    if (t < 0) break;
     const int2 te = R.tiles[t];
     const int sim = te.x, g = te.y >> 16, kb = te.y & 0xffff;
     const SimDesc& D = sim_desc(m, sim);
@@ -417,19 +470,21 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const bool hG = g > 0 && !tile_empty(g - 1, kb, Kp, TK, NX);
     const bool hK = kb == 0 || !tile_empty(g, kb - 1, Kp, TK, NX);
     const bool hC = g > 0 && (kb == 0 || !tile_empty(g - 1, kb - 1, Kp, TK, NX));
+    // The G stream has a column of tiles before the first for the initial state (k_gs_skew), so the
+    // corner's words lie a tile before the G stream's.
     const size_t gtile = (size_t)rows * GROW, ktile = (size_t)rows * KROW, itile = (size_t)(rows + 1) * KROW;
     const __amdgpu_buffer_rsrc_t kmine = word_buffer(D.kout + (size_t)(g * KB + kb) * ktile);
-    const __amdgpu_buffer_rsrc_t gmine = word_buffer(D.gout + (size_t)(g * KB + kb) * gtile);
-    const __amdgpu_buffer_rsrc_t gprod = word_buffer(D.gout + (hG ? (size_t)((g - 1) * KB + kb) * gtile : 0));
+    const __amdgpu_buffer_rsrc_t gmine = word_buffer(D.gout + (size_t)(g * (KB + 1) + kb + 1) * gtile);
+    const __amdgpu_buffer_rsrc_t gprod = word_buffer(D.gout + (g > 0 ? (size_t)((g - 1) * (KB + 1) + kb) * gtile : 0));
     const uint8_t* ksrc = kb ? D.kout + (size_t)(kb - 1) * ktile : D.kinit;  // of row-tile 0
     const size_t kstep = kb ? KB * ktile : itile;                            // to the next row-tile
     const __amdgpu_buffer_rsrc_t kprod = word_buffer(ksrc + (hK ? g * kstep : 0));
-    const __amdgpu_buffer_rsrc_t cprod = word_buffer(ksrc + (hC ? (g - 1) * kstep : 0));
     const uint32_t ktag = kb ? tag : tag0;
-    const int kfirst = kb ? TK : 1, klast = kb ? rows - 1 : rows;  // row of step 1, last row
+    const int kfirst = kb ? TK - 1 : 0, klast = kb ? rows - 1 : rows;  // row of step 0, last row
 
     Sweeps<S> Q;
-    uint32_t mrow[S], mk[S], mkeep[S];
+    uint32_t mk[S], mkeep[S];
+    const uint8_t* mrow[S];
     int mcol[S];
     const uint32_t mpitch = mask_pitch(NY);
 #pragma unroll
@@ -441,30 +496,29 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       mkeep[c] = k0 + b0 + c < K ? BITS : 0u;  // past the solve's last sweep the cells pass their faces on
       // rows 0 and NX - 1 are all 0; the copy in which this lane's columns start a byte (an odd
       // first column j: byte (j + 1) / 2 of the odd copy)
-      mrow[c] = (((lane + b0 + c) & 1) ? NX * mpitch : 0u) +
-                (uint32_t)min(max(i0 + lane - b0 - c, 0), NX - 1) * mpitch + MASK_PAD / 2;
+      mrow[c] = D.masks + (((lane + b0 + c) & 1) ? (size_t)NX * mpitch : 0) +
+                (size_t)min(max(i0 + lane - b0 - c, 0), NX - 1) * mpitch + MASK_PAD / 2;
       mcol[c] = (1 - lane - b0 - c) >> 1;
     }
-    const uint8_t* masks = D.masks;
     const int mlast = (NY + 2) >> 1;
     float k[3] = {0.0f, 0.0f, 0.0f};
 
     // The G words of a block this lane loads: word (u, x) is what sweep b0 - 1 + x of the tile
-    // below left at lane 63 for this wave's step u; a tile's first sweep (w = 0, x = 0) takes lane
-    // 63 of that tile's K row instead.
+    // below left at lane 63 for this wave's step u; a tile's first sweep (w = 0, x = 0) takes the
+    // last sweep of the corner tile instead. need: all ones in the lanes that wait for a producer.
     const int gu = lane / (S + 1), gx = lane - gu * (S + 1);
-    const bool gcorner = w == 0 && gx == 0, gstage = gu < B, ghas = gstage && (gcorner ? hC : hG);
-    const uint32_t gat = gcorner ? 16 * (LANES - 1) : 16 * (b0 - 1 + gx);
-    const uint32_t goff = gat + (gcorner ? (gu + LANES - 1 + kfirst) * KROW : (gu + LANES - 1) * GROW);
-    const uint32_t glast = gat + (gcorner ? klast * KROW : (rows - 1) * GROW);
+    const bool gcorner = w == 0 && gx == 0, gstage = gu < B;
+    const uint32_t gat = gcorner ? 16 * (TK - 1) : (uint32_t)gtile + 16 * (b0 - 1 + gx);
+    const uint32_t goff = gat + (gcorner ? gu + LANES + kfirst : gu + LANES - 1) * GROW;
+    const uint32_t glast = gat + (rows - 1) * GROW;
+    const uint32_t gtag = gcorner ? ktag : tag, gneed = gstage && (gcorner ? hC : hG) ? ~0u : 0u, kneed = hK ? ~0u : 0u;
     lds_float* const gdst = (lds_float*)&sh.Gi[w][min(gu, B - 1) + 1][3 * gx];
-    const uint32_t gotid = min(lane, B * S - 1);  // the word of lane 63's this lane stores: step / S, sweep % S
-    const uint32_t goword = (gotid / S) * GROW + 16 * (b0 + gotid % S);
+    const bool gout = g_wave && lane >= LANES - B;  // stores lane 63's words of step lane - (64 - B)
+    const uint32_t goword = max(lane - (LANES - B), 0) * GROW + 16 * b0;
     // Ends a wait for words that all carry this solve's tag. Bounded: after SPIN_LIMIT tries, or
     // once another wait of this simulation has expired (err set), err is set and the solve goes
     // on, so one whose producers stall ends within about a second with FL_ERR_INTERNAL.
-    auto expired = [&](bool done, int it) __attribute__((always_inline)) {
-      if (done) return true;
+    auto expired = [&](int it) __attribute__((always_inline)) {
       if (it > SPIN_LIMIT || ((it & 255) == 255 && ld_err(err) != 0)) {
         if (lane == 0) atomicOr(err, 1);
         return true;
@@ -478,57 +532,55 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     auto run_wave = [&](auto first_c, auto out_c) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_c)::value;
       constexpr int OUT = decltype(out_c)::value;
-      // The words and masks of a block. The loads are issued without a condition on the lane, at
-      // addresses that are always valid, so none waits for another.
+      // The words and masks of a block. The loads are issued without a condition, at addresses that
+      // are always valid, so that the compiler can count them and none waits for another.
       struct Block {
-        word4 gw, gc, kw[B];
+        uint32_t mw[S];
+        word4 gw, kw[FIRST ? B : 1];
       };
-      word2_any mw[S];  // masks of the MB blocks that the next block to stage is one of
       auto load_g = [&](Block& x, int n) __attribute__((always_inline)) {
-        x.gw = ld_word(gprod, gcorner ? 0u : min(goff + n * (B * GROW), glast));
-        if constexpr (FIRST) x.gc = ld_word(cprod, gcorner ? min(goff + n * (B * KROW), glast) : 0u);
+        x.gw = ld_word(gprod, min(goff + n * (B * GROW), glast));
       };
       auto load_k = [&](Block& x, int n, int u) __attribute__((always_inline)) {
         x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(kprod, 16 * lane, min(n * B + u + kfirst, klast) * KROW,
                                                         SC1 | VOLATILE_OP);
       };
       auto load = [&](Block& x, int n) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          const uint8_t* at = mrow[c] + min(max(n * (B / 2) + mcol[c], -(MASK_PAD / 2)), mlast);
+          if constexpr (B == 8)
+            x.mw[c] = *reinterpret_cast<const mask8_any*>(at);
+          else
+            x.mw[c] = *reinterpret_cast<const mask4_any*>(at);
+        }
         load_g(x, n);
         if constexpr (FIRST) {
 #pragma unroll
           for (int u = 0; u < B; u++) load_k(x, n, u);
         }
-        if (n % MB == 0) {
-#pragma unroll
-          for (int c = 0; c < S; c++)
-            mw[c] = *reinterpret_cast<const word2_any*>(
-                masks + (mrow[c] + min(max(n * (B / 2) + mcol[c], -(MASK_PAD / 2)), mlast)));
-        }
       };
       auto stage = [&](Block& x, int n) __attribute__((always_inline)) {
         auto arrived = [&]() __attribute__((always_inline)) {
-          uint32_t d = 0;
+          uint32_t d = word_tag(x.gw, gtag) & gneed;
           if constexpr (FIRST) {
-            if (gcorner) x.gw = x.gc;
-            if (ghas) d = word_tag(x.gw, gcorner ? ktag : tag);
-            if (hK) {
+            uint32_t e = 0;
 #pragma unroll
-              for (int u = 0; u < B; u++) d |= word_tag(x.kw[u], ktag);
-            }
-          } else {
-            if (ghas) d = word_tag(x.gw, tag);
+            for (int u = 0; u < B; u++) e |= word_tag(x.kw[u], ktag);
+            d |= e & kneed;
           }
-          return __all(d < 0x10000u);
+          return every_lane(d < 0x10000u);
         };
         // The first check stands before the loop: at the loop's head it would have to wait for every
         // store issued since. A wait polls with the G words and the block's last K row only: 256 CUs
         // that reload whole blocks would take the bandwidth their producers need.
         if (!arrived()) {
-          for (int it = 0; !expired(false, it); it++) {
+          for (int it = 0; !expired(it); it++) {
+            if (NEAR && far) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             load_g(x, n);
             if constexpr (FIRST) {
               load_k(x, n, B - 1);
-              if (hK && __all(word_tag(x.kw[B - 1], ktag) < 0x10000u)) {
+              if (every_lane(word_tag(x.kw[B - 1], ktag) < 0x10000u)) {
 #pragma unroll
                 for (int u = 0; u < B - 1; u++) load_k(x, n, u);
               }
@@ -543,25 +595,16 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           gdst[0] = word_v(x.gw);
           gdst[1] = word_p(x.gw);
         }
-        if constexpr (FIRST) {
-          float4* dst = &sh.K[0][n & 1][0][lane];
-#pragma unroll
-          for (int u = 0; u < B; u++)
-            dst[u * LANES] = make_float4(word_u(x.kw[u]), word_v(x.kw[u]), word_p(x.kw[u]), 0.0f);
-        }
 #pragma unroll
         for (int c = 0; c < S; c++) {
-          const uint32_t lo = mw[c].x, hi = mw[c].y;
-          if constexpr (B == 8)
-            mk[c] = (n % 2 ? hi : lo) & mkeep[c];
-          else
-            mk[c] = ((n & 2 ? hi : lo) >> (n & 1 ? 16 : 0)) & mkeep[c];
+          mk[c] = x.mw[c] & mkeep[c];
           asm volatile("" : "+v"(mk[c]));  // now: the scheduler would wait for the masks after the next stores
         }
       };
-      auto run = [&](int n) __attribute__((always_inline)) {
-        const float4* Kin = &sh.K[w][n & 1][0][lane];
-        float4* Kout = &sh.K[w + 1 < W ? w + 1 : w][n & 1][0][lane];
+      float go[S][3];
+      auto run = [&](const Block& x, int n) __attribute__((always_inline)) {
+        const float4* Kin = FIRST ? nullptr : &sh.K[w - 1][n & 1][0][lane];
+        float4* Kout = OUT == OUT_WORDS ? nullptr : &sh.K[w][n & 1][0][lane];
         const uint32_t kbyte = (uint32_t)n * (B * KROW) + 16 * lane;
         bool plain = true, same = true;
 #pragma unroll
@@ -570,10 +613,10 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<S, B, GP, MODE, OUT, FULL>(Q, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
-        if (!FULL && __all(plain)) {
+  run_block<S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
+        if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
-        } else if (__all(same)) {
+        } else if (every_lane(same)) {
           FL_RUN(BLOCK_SAME);
         } else {
           FL_RUN(BLOCK_ANY);
@@ -581,37 +624,35 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
 #undef FL_RUN
       };
       for (int p = 0; p < w; p++) __syncthreads();
-      if constexpr (FIRST) {
-        // what sweep 0 reads at step 0, the row before block 0's
-        for (int it = 0;; it++) {
-          const word4 v = ld_word(kprod, (kfirst - 1) * KROW + 16 * lane);
-          k[0] = word_u(v);
-          k[1] = word_v(v);
-          k[2] = word_p(v);
-          if (expired(!hK || __all(word_tag(v, ktag) < 0x10000u), it)) break;
-        }
-      }
-      {
-        Block x;
-        load(x, 0);
-        stage(x, 0);
-      }
-      __syncthreads();
-      for (int n = 0; n < nblk; n++) {
-        // Block n runs while the words of block n + 1 are on their way (the last block's once more
-        // after the end). They are waited for before the stores of lane 63's words are issued: vector
-        // memory operations complete in order, and a wait behind a store would last as long as the
-        // store's way to memory.
+      // Block n runs while the words of block n + 1 are on their way (the last block's once more
+      // after the end). They are waited for before the stores of lane 63's words are issued: vector
+      // memory operations complete in order, and a wait behind a store would last as long as the
+      // store's way to memory.
+      auto phase = [&](const Block& x, Block& next, int n) __attribute__((always_inline)) {
         const int n1 = min(n + 1, nblk - 1);
-        Block x;
-        load(x, n1);
-        run(n);
-        stage(x, n1);
-        if (g_wave) {
-          const float4 v = (&sh.Go[w][0][0])[gotid];
-          if (lane < B * S) st_word(gmine, goword + n * (B * GROW), v.x, v.y, v.z, tag);
+        load(next, n1);
+        run(x, n);
+        stage(next, n1);
+        if (gout) {
+#pragma unroll
+          for (int c = 0; c < S; c++) st_word<SC1>(gmine, goword + n * (B * GROW) + 16 * c, go[c][0], go[c][1], go[c][2], tag);
         }
+        if (NEAR && OUT == OUT_WORDS && far) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
+      };
+      Block x, y;
+      load(x, 0);
+      stage(x, 0);
+      __syncthreads();
+      if constexpr (FIRST) {  // two blocks to a turn, so that their words stay where they were loaded
+        for (int n = 0;;) {
+          phase(x, y, n);
+          if (++n == nblk) break;
+          phase(y, x, n);
+          if (++n == nblk) break;
+        }
+      } else {
+        for (int n = 0; n < nblk; n++) phase(x, x, n);
       }
       for (int p = w + 1; p < W; p++) __syncthreads();
     };
@@ -667,7 +708,7 @@ __device__ __forceinline__ bool skew_item(const OneSim& m, const SkewItem*, cons
 // Row t (stored at t + 1) of row-tile g holds, at lane a, U, V and p of cell (64 g + a + 1, t - a + 1):
 // what lane a of a sweep before the first would have left at step t.
 template <class M>
-__global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int rPin) {
+__global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int tk, int rPin) {
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
   int g, t0;
@@ -684,11 +725,15 @@ __global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, con
   __syncthreads();
   const uint32_t tag = 2u * (uint32_t)*solve & 0xffffu;
   const __amdgpu_buffer_rsrc_t dst = word_buffer(D->kinit + (size_t)g * (D->rows + 1) * (16 * LANES));
+  // lane 63's also as the last sweep's of the G stream's first column
+  const __amdgpu_buffer_rsrc_t gdst = word_buffer(D->gout + (size_t)g * (D->KB + 1) * D->rows * (16 * tk));
 #pragma unroll 4
   for (int x = 0; x < 16; x++) {
     const int u = 16 * w + x;
     if (t0 + u <= D->rows)
-      st_word(dst, (uint32_t)(t0 + u) * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
+      st_word<CACHED>(dst, (uint32_t)(t0 + u) * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
+    if (lane == LANES - 1 && t0 + u < D->rows)
+      st_word<CACHED>(gdst, (uint32_t)(t0 + u) * (16 * tk) + 16 * (tk - 1), sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
   }
 }
 
@@ -763,22 +808,23 @@ template <class M> __global__ void k_gs_ring(M m, int rPin, int rPout) {
   }
 }
 
-// Zero the ticket counters of both runs, the per-sweep maxima and the re-run requests of every
+// Zero the counters of both runs, the per-sweep maxima and the re-run requests of every
 // simulation of the launch (graph-safe: no memset).
-__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim, int32_t* ticket) {
+__device__ __forceinline__ void clear_state(GsState* S, int t) {
+  int32_t* c = reinterpret_cast<int32_t*>(S->run);
+  for (; t < (int)(sizeof(S->run) / sizeof(int32_t)); t += blockDim.x) c[t] = 0;
+  if (threadIdx.x == 0) S->rerun = 0;
+}
+__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim, GsState* S) {
   const int stride = blockDim.x * gridDim.x;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nmd; t += stride) maxdiv[t] = 0u;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nsim; t += stride) ctrl[4 * t] = ctrl[4 * t + 1] = 0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    ticket[0] = 0;  // main run
-    ticket[1] = 0;  // re-run
-    ticket[2] = 0;  // re-run requested by some simulation
-  }
+  if (blockIdx.x == 0) clear_state(S, threadIdx.x);
 }
 
 // k_gs_ring and k_gs_init of a single simulation in one launch (both only precede the solve).
 __global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int nmd, int32_t* ctrl,
-                          int32_t* ticket) {
+                          GsState* S) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const SimDesc& D = m.d;
   const int NX = D.g.NX, NY = D.g.NY;
@@ -792,10 +838,8 @@ __global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int n
   }
   const int stride = blockDim.x * gridDim.x;
   for (int i = t; i < nmd; i += stride) maxdiv[i] = 0u;
-  if (t == 0) {
-    ctrl[0] = ctrl[1] = 0;
-    ticket[0] = ticket[1] = ticket[2] = 0;
-  }
+  if (t == 0) ctrl[0] = ctrl[1] = 0;
+  if (blockIdx.x == 0) clear_state(S, t);
 }
 
 // Early exit of solveSingleGrid (fluid.go:175-177), one wave per simulation: the first
@@ -832,9 +876,9 @@ static bool tile_empty_h(int g, int kb, int K, int TK, int NX) {
 }
 
 // Waves per workgroup of a tile of tk sweeps: two sweeps to a wave; one in the small tiles, whose
-// few waves leave the CU's issue slots free (4 sweeps, 256^2 jet: 0.218 ms against 0.223 with two
-// waves of two; 300x251 0.153 against 0.171). Four to a wave lost everywhere (4096^2 6.1 ms
-// against 5.7 at 16 sweeps).
+// few waves leave the CU's issue slots free (4 sweeps, 256^2 jet: 0.154 ms against 0.175 with two
+// waves of two; 300x251 0.110 against 0.136). Four to a wave lost everywhere (2048^2 2.35 ms
+// against 1.72 at 16 sweeps, 2048x1024 1.55 against 1.09 at 8).
 static int tile_waves(int tk) { return tk <= 4 ? tk : tk / 2; }
 static int tile_sweeps(int tk) { return tk / tile_waves(tk); }  // sweeps per wave
 // N sweeps with those that only fill the last wave: their cells pass their faces on.
@@ -861,33 +905,81 @@ static TileGeom geom(int NX, int NY, int N, int tk, int blk) {
 // (W - 1) blocks between the first and the last wave behind the tile one sweep block back; the
 // key is that estimate of its start. Producers always get smaller keys (a topological order, which
 // the persistent kernel needs: a workgroup never waits on a tile no workgroup has taken).
-static void append_tiles(std::vector<std::pair<long long, int2>>& out, int sim, int NX, int N, int tk, int blk,
-                         const TileGeom& t) {
+struct GsTile {
+  long long key;
+  int row;  // of all simulations' row-tiles
+  int2 t;
+};
+static void append_tiles(std::vector<GsTile>& out, int sim, int row0, int NX, int N, int tk, int blk, const TileGeom& t) {
   for (int g = 0; g < t.G; g++)
     for (int kb = 0; kb < t.KB; kb++)
       if (!tile_empty_h(g, kb, padded(N, tk), tk, NX)) {
         const long long start = (long long)(LANES + 2 * blk) * g + (long long)(tk + (tile_waves(tk) + 1) * blk) * kb;
-        long long key = (start << 32) | ((long long)sim << 12) | kb;
-        out.push_back({key, make_int2(sim, (g << 16) | kb)});
+        out.push_back({(start << 32) | ((long long)sim << 12) | kb, row0 + g, make_int2(sim, (g << 16) | kb)});
       }
 }
-
-// Sweeps per tile: the knob if set; otherwise the smallest tile of which the solve has no more
-// than about one per CU (two, of eight sweeps). Small tiles spread a small grid over the CUs and
-// step faster; once there are more of them than CUs, large ones hand over less and take fewer
-// turns. Solve times in ms with 2, 4, 8, 16 sweeps: 300x251 8 sweeps 0.142 0.153 0.184 0.185;
-// 777x391 33 sweeps 0.322 0.340 0.404 0.516; 1024^2 40 sweeps 0.533 0.517 0.619 0.787; 512^2 200
-// sweeps 0.839 0.680 0.639 0.797; 2048x1024 100 sweeps 1.533 1.156 1.163 1.356; 2048^2 200 sweeps
-// 4.50 2.97 2.22 2.09; 4096^2 40 sweeps 4.38 3.29 2.86 3.19, 200 sweeps 16.0 10.5 6.8 5.7.
-int pick_tk(const fl_params& P, int NX, int N) {
-  if (P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16) return P.block_sweeps;
-  const long long G = (NX + N - 1 + LANES - 1) / LANES;
-  if (G * ((N + 1) / 2) <= 256) return 2;
-  if (G * ((N + 3) / 4) <= 256) return 4;
-  return G * ((N + 7) / 8) <= 512 ? 8 : 16;
+// The tiles of nq queues, each in ticket order, then all in ticket order; first[q]: where they begin.
+// Row-tiles go to the queue that has the fewest steps so far, in the order of their first tiles.
+// Returns the tiles of the longest queue.
+static int queue_tiles(std::vector<GsTile>& tiles, const std::vector<int>& row_steps, int nq, std::vector<int2>& out,
+                       std::vector<int>& first) {
+  std::sort(tiles.begin(), tiles.end(), [](const GsTile& a, const GsTile& b) { return a.key < b.key; });
+  std::vector<long long> load(row_steps.size(), 0), total(nq, 0);
+  std::vector<int> queue(row_steps.size(), -1);
+  for (const GsTile& t : tiles) load[t.row] += row_steps[t.row];
+  std::vector<std::vector<int2>> lists(nq);
+  for (const GsTile& t : tiles) {
+    int& q = queue[t.row];
+    if (q < 0 && nq > 0) {
+      q = (int)(std::min_element(total.begin(), total.end()) - total.begin());
+      total[q] += load[t.row];
+    }
+    if (nq > 0) lists[q].push_back(t.t);
+  }
+  size_t longest = 0;
+  for (auto& l : lists) {
+    first.push_back((int)out.size());
+    out.insert(out.end(), l.begin(), l.end());
+    longest = std::max(longest, l.size());
+  }
+  first.push_back((int)out.size());
+  for (const GsTile& t : tiles) out.push_back(t.t);
+  first.push_back((int)out.size());
+  return (int)longest;
 }
-// Columns per block: 4 with the knob, else 8, which won at every size (4096^2 200 sweeps 5.7 ms
-// against 7.6, 512^2 0.639 against 0.651). 16, which the knob also takes, would not fit in LDS.
+// One queue per XCD of 32 CUs.
+static int device_queues(int dev, int tk) {
+  int cus = 0;
+  if (!near_tiles(tk)) return 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+  return std::min(MAXQ, std::max(1, cus / 32));
+}
+
+// Tiles of tk sweeps that a solve has in flight at once: the row-tiles that start (80 steps one
+// after the other) before the first ends, by the blocks of sweeps.
+static long long tiles_in_flight(int NX, int NY, int N, int tk) {
+  const long long rows = std::min((NX + N - 1 + LANES - 1) / LANES, (NY + LANES + 79) / 80);
+  return rows * ((N + tk - 1) / tk);
+}
+// Sweeps per tile for the number of tiles in flight by their depth: the smallest tile of which
+// there is no more than one per CU. Small tiles spread a small grid over the CUs and
+// step faster; once there are more of them than CUs, large ones hand over less and take fewer
+// turns. Solve times in ms with 4, 8, 16 sweeps: 300x251 8 sweeps 0.110 0.142 0.146; 256^2 40 sweeps
+// 0.154 0.174 0.227; 777x391 33 sweeps 0.239 0.307 0.415; 1024^2 40 sweeps (140 in flight with 4)
+// 0.366 0.457 0.625; 1024^2 100 sweeps (350 with 4, 182 with 8) 0.633 0.585 0.734; 512^2 200 sweeps
+// (400, 200) 0.510 0.473 0.636; 2048x1024 100 sweeps (350, 182) 1.012 0.928 1.054; 4096^2 40 sweeps
+// (265 with 8) 3.12 2.90 2.51; 2048^2 200 sweeps (675) 2.83 2.10 1.72; 4096^2 200 sweeps 10.2 6.6 5.0.
+// Two sweeps (the knob takes them) gain nothing on 4: 300x251 0.111, 256^2 0.161.
+template <class F> static int depth_for(F in_flight) { return in_flight(4) <= 256 ? 4 : in_flight(8) <= 256 ? 8 : 16; }
+static bool tk_knob(const fl_params& P) {
+  return P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16;
+}
+int pick_tk(const fl_params& P, int NX, int NY, int N) {
+  if (tk_knob(P)) return P.block_sweeps;
+  return depth_for([&](int tk) { return tiles_in_flight(NX, NY, N, tk); });
+}
+// Columns per block: 4 with the knob, else 8, which won at every size (4096^2 200 sweeps 5.0 ms
+// against 7.1, 256^2 0.154 against 0.163). 16, which the knob also takes, would not fit in LDS.
 int pick_blk(const fl_params& P) { return P.block_cols == 4 ? 4 : 8; }
 // The update that leaves inactive cells alone by the signs of zeros needs these; any other
 // parameters take the FULL kernels.
@@ -911,7 +1003,7 @@ template <class M> struct GsKernels {
     return nullptr;
   }
 };
-template <class M> static int occupancy_grid(int dev, int tk, int blk, int ntiles) {
+template <class M> static int occupancy_grid(int dev, int tk, int blk, int ntiles) {  // ntiles: as if all queues were the longest
   int per_cu = 0;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 1;
@@ -932,7 +1024,7 @@ static int launch_gs(int tk, int blk, int grid, hipStream_t stream, const M& m, 
 
 static int layout(Ctx* c, int N) {
   GsWork& W = c->gs;
-  const int tk = pick_tk(c->prm, c->NX, N);
+  const int tk = pick_tk(c->prm, c->NX, c->NY, N);
   const int blk = pick_blk(c->prm);
   if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
   FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
@@ -944,26 +1036,30 @@ static int layout(Ctx* c, int N) {
   W.G = t.G;
   W.KB = t.KB;
   W.rows = t.rows;
-  std::vector<std::pair<long long, int2>> order;
-  append_tiles(order, 0, c->NX, N, tk, blk, t);
-  std::sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+  std::vector<GsTile> order;
+  append_tiles(order, 0, 0, c->NX, N, tk, blk, t);
   std::vector<int2> tiles;
-  for (auto& o : order) tiles.push_back(o.second);
-  W.ntiles = (int)tiles.size();
+  std::vector<int> first;
+  W.nq = device_queues(c->dev, tk);
+  const int longest = queue_tiles(order, std::vector<int>(t.G, t.rows), W.nq, tiles, first);
+  W.ntiles = (int)order.size();
   const size_t nt = (size_t)W.G * W.KB;
-  const size_t kbytes = 16 * nt * W.rows * LANES, gbytes = 16 * nt * W.rows * tk;
-  FL_HIP(hipMalloc(&W.d_tile, sizeof(int2) * std::max(1, W.ntiles)));
+  const size_t kbytes = 16 * nt * W.rows * LANES, gbytes = 16 * (nt + W.G) * W.rows * tk;
+  FL_HIP(hipMalloc(&W.d_tile, sizeof(int2) * std::max<size_t>(1, tiles.size())));
+  FL_HIP(hipMalloc(&W.d_first, sizeof(int) * first.size()));
   FL_HIP(hipMalloc(&W.d_kout, kbytes));
   FL_HIP(hipMalloc(&W.d_gout, gbytes));
   FL_HIP(hipMalloc(&W.d_kinit, (size_t)16 * W.G * (W.rows + 1) * LANES));
-  FL_HIP(hipMalloc(&W.d_ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag, solve number
+  FL_HIP(hipMalloc(&W.d_state, sizeof(GsState)));
   // no word may carry a tag before a solve writes it: the words start at tag 0, the solves at 1
   FL_HIP(hipMemsetAsync(W.d_kout, 0, kbytes, c->stream));
   FL_HIP(hipMemsetAsync(W.d_gout, 0, gbytes, c->stream));
-  const int32_t first[4] = {0, 0, 0, 1};
-  FL_HIP(hipMemcpy(W.d_ticket, first, sizeof(first), hipMemcpyHostToDevice));
-  FL_HIP(hipMemcpy(W.d_tile, tiles.data(), sizeof(int2) * W.ntiles, hipMemcpyHostToDevice));
-  W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, W.ntiles);
+  GsState state{};
+  state.solve = 1;
+  FL_HIP(hipMemcpy(W.d_state, &state, sizeof(state), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(W.d_tile, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(W.d_first, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice));
+  W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, std::max(W.ntiles, W.nq * longest));
   return FL_OK;
 }
 
@@ -982,15 +1078,16 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   const int rPin = c->gs_p_zero ? -1 : (int)B_P;
   c->gs_p_zero = false;
   hipLaunchKernelGGL(k_gs_prep, dim3(std::max(4, (mr + 255) / 256)), dim3(256), 0, c->stream, m, rPin, (int)B_T3,
-                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl, W.d_ticket);
+                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl, W.d_state);
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
-  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_ticket + 3, rPin);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
-  R.ntiles = W.ntiles;
+  R.first = W.d_first;
+  R.nq = W.nq;
   R.K = N;
-  R.solve = W.d_ticket + 3;
+  R.solve = &W.d_state->solve;
   R.omega = c->d_omega;
   R.damping = c->prm.pressure_damping;
   W.lag = c->prm.handoff_lag >= 1 && c->prm.handoff_lag <= 3 ? c->prm.handoff_lag : 1;
@@ -999,15 +1096,15 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   const int runs = c->prm.early_exit ? 2 : 1;
   for (int which = 0; which < runs; which++) {
     R.which = which;
-    R.ticket = W.d_ticket + which;
-    R.rerun = which ? W.d_ticket + 2 : nullptr;
+    R.count = &W.d_state->run[which];
+    R.rerun = which ? &W.d_state->rerun : nullptr;
     if ((rc = launch_gs(W.tk, W.blk, W.grid, c->stream, m, R, full))) return rc;
     if (which == 0 && runs > 1) {
-      hipLaunchKernelGGL(k_gs_decide<OneSim>, dim3(1), dim3(LANES), 0, c->stream, m, 1, N, W.d_ticket + 2);
+      hipLaunchKernelGGL(k_gs_decide<OneSim>, dim3(1), dim3(LANES), 0, c->stream, m, 1, N, &W.d_state->rerun);
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_ticket + 3, N, W.tk,
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, N, W.tk,
                      tile_sweeps(W.tk), (int)B_T3);
   FL_HIP(hipGetLastError());
   std::swap(c->U, c->U2);
@@ -1023,7 +1120,8 @@ int pressure_free(Ctx* c) {
   if (W.d_kout) (void)hipFree(W.d_kout);
   if (W.d_gout) (void)hipFree(W.d_gout);
   if (W.d_kinit) (void)hipFree(W.d_kinit);
-  if (W.d_ticket) (void)hipFree(W.d_ticket);
+  if (W.d_first) (void)hipFree(W.d_first);
+  if (W.d_state) (void)hipFree(W.d_state);
   W = GsWork{};
   return FL_OK;
 }
@@ -1035,9 +1133,12 @@ int pressure_free(Ctx* c) {
 // velocity to U2, V2.
 // A batch's sweeps per tile: as for one grid, by the tiles of all members.
 static int batch_tk(const fl_params& P, const std::vector<SimDesc>& descs, int N) {
-  long long nx = 0;
-  for (const SimDesc& d : descs) nx += (d.g.NX + N - 1 + LANES - 1) / LANES * LANES;
-  return pick_tk(P, (int)std::min<long long>(std::max<long long>(nx - N + 1, 1), 1 << 30), N);
+  if (tk_knob(P)) return P.block_sweeps;
+  return depth_for([&](int tk) {
+    long long n = 0;
+    for (const SimDesc& d : descs) n += tiles_in_flight(d.g.NX, d.g.NY, N, tk);
+    return n;
+  });
 }
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   const int tk = batch_tk(B->prm, descs, N);
@@ -1064,33 +1165,39 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   if (B->gout) (void)hipFree(B->gout);
   if (B->kinit) (void)hipFree(B->kinit);
   if (B->d_skews) (void)hipFree(B->d_skews);
-  if (B->ticket) (void)hipFree(B->ticket);
+  if (B->d_first) (void)hipFree(B->d_first);
+  if (B->state) (void)hipFree(B->state);
   B->d_tiles = nullptr;
   B->kout = B->gout = B->kinit = nullptr;
   B->d_skews = nullptr;
-  B->ticket = nullptr;
-  std::vector<std::pair<long long, int2>> order;
+  B->d_first = nullptr;
+  B->state = nullptr;
+  std::vector<GsTile> order;
+  std::vector<int> row_steps;
   size_t kbytes = 0, gbytes = 0, ibytes = 0;
   std::vector<SkewItem> skews;
   std::vector<TileGeom> tg(descs.size());
   for (size_t e = 0; e < descs.size(); e++) {
     tg[e] = geom(descs[e].g.NX, descs[e].g.NY, N, tk, blk);
-    append_tiles(order, (int)e, descs[e].g.NX, N, tk, blk, tg[e]);
+    append_tiles(order, (int)e, (int)row_steps.size(), descs[e].g.NX, N, tk, blk, tg[e]);
+    row_steps.insert(row_steps.end(), tg[e].G, tg[e].rows);
     const size_t nt = (size_t)tg[e].G * tg[e].KB;
     kbytes += 16 * nt * tg[e].rows * LANES;
-    gbytes += 16 * nt * tg[e].rows * tk;
+    gbytes += 16 * (nt + tg[e].G) * tg[e].rows * tk;
     ibytes += (size_t)16 * tg[e].G * (tg[e].rows + 1) * LANES;
     for (int g = 0; g < tg[e].G; g++)
       for (int t0 = 0; t0 <= tg[e].rows; t0 += LANES) skews.push_back(SkewItem{(int)e, g, t0, 0});
   }
-  std::sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
   std::vector<int2> tiles;
-  for (auto& o : order) tiles.push_back(o.second);
-  B->ntiles = (int)tiles.size();
-  FL_HIP(hipMalloc(&B->d_tiles, sizeof(int2) * std::max(1, B->ntiles)));
+  std::vector<int> first;
+  B->nq = device_queues(B->dev, tk);
+  const int longest = queue_tiles(order, row_steps, B->nq, tiles, first);
+  B->ntiles = (int)order.size();
+  FL_HIP(hipMalloc(&B->d_tiles, sizeof(int2) * std::max<size_t>(1, tiles.size())));
+  FL_HIP(hipMalloc(&B->d_first, sizeof(int) * first.size()));
   FL_HIP(hipMalloc(&B->kout, std::max<size_t>(kbytes, 16)));
   FL_HIP(hipMalloc(&B->gout, std::max<size_t>(gbytes, 16)));
-  FL_HIP(hipMalloc(&B->ticket, sizeof(int32_t) * 4));  // main, re-run, re-run flag, solve number
+  FL_HIP(hipMalloc(&B->state, sizeof(GsState)));
   // no word may carry a tag before a solve writes it: the words start at tag 0, the solves at 1
   FL_HIP(hipMemsetAsync(B->kout, 0, kbytes, B->stream));
   FL_HIP(hipMemsetAsync(B->gout, 0, gbytes, B->stream));
@@ -1098,9 +1205,11 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   FL_HIP(hipMalloc(&B->d_skews, sizeof(SkewItem) * std::max<size_t>(skews.size(), 1)));
   FL_HIP(hipMemcpy(B->d_skews, skews.data(), sizeof(SkewItem) * skews.size(), hipMemcpyHostToDevice));
   B->nskew = (int)skews.size();
-  const int32_t first[4] = {0, 0, 0, 1};
-  FL_HIP(hipMemcpy(B->ticket, first, sizeof(first), hipMemcpyHostToDevice));
-  FL_HIP(hipMemcpy(B->d_tiles, tiles.data(), sizeof(int2) * B->ntiles, hipMemcpyHostToDevice));
+  GsState state{};
+  state.solve = 1;
+  FL_HIP(hipMemcpy(B->state, &state, sizeof(state), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(B->d_tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(B->d_first, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice));
   size_t ko = 0, go = 0, io = 0;
   B->gs_fields.assign(descs.size(), SimDesc{});
   for (size_t e = 0; e < descs.size(); e++) {
@@ -1113,13 +1222,13 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
     d.kinit = B->kinit + io;
     const size_t nt = (size_t)d.G * d.KB;
     ko += 16 * nt * d.rows * LANES;
-    go += 16 * nt * d.rows * tk;
+    go += 16 * (nt + d.G) * d.rows * tk;
     io += (size_t)16 * d.G * (d.rows + 1) * LANES;
   }
   B->tk = tk;
   B->blk = blk;
   B->gs_n = N;
-  B->grid = occupancy_grid<ManySims>(B->dev, tk, blk, B->ntiles);
+  B->grid = occupancy_grid<ManySims>(B->dev, tk, blk, std::max(B->ntiles, B->nq * longest));
   fill();
   return FL_OK;
 }
@@ -1130,14 +1239,16 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   hipLaunchKernelGGL(k_gs_ring<ManySims>, dim3(B->nring_items), dim3(256), 0, B->stream, m, rPin, rPout);
   // per-sweep maxima and re-run requests of all members are contiguous
   hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E,
-                     B->ticket);
-  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->ticket + 3, rPin);
+                     B->state);
+  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, &B->state->solve, B->tk,
+                     rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = B->d_tiles;
-  R.ntiles = B->ntiles;
+  R.first = B->d_first;
+  R.nq = B->nq;
   R.K = N;
-  R.solve = B->ticket + 3;
+  R.solve = &B->state->solve;
   R.omega = B->d_omega;
   R.damping = B->prm.pressure_damping;
   // every member's cp is density h / dt with the batch's density, h and dt
@@ -1145,18 +1256,18 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   const int runs = B->prm.early_exit ? 2 : 1;  // no early exit: nothing to decide or re-run
   for (int which = 0; which < runs; which++) {
     R.which = which;
-    R.ticket = B->ticket + which;
-    R.rerun = which ? B->ticket + 2 : nullptr;
+    R.count = &B->state->run[which];
+    R.rerun = which ? &B->state->rerun : nullptr;
     int rc = launch_gs(B->tk, B->blk, B->grid, B->stream, m, R, full);
     if (rc) return rc;
     if (which == 0 && runs > 1) {
       // one wave per member, four per workgroup
       hipLaunchKernelGGL(k_gs_decide<ManySims>, dim3((E + 3) / 4), dim3(4 * LANES), 0, B->stream, m, E, N,
-                         B->ticket + 2);
+                         &B->state->rerun);
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->ticket + 3, N,
+  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, &B->state->solve, N,
                      B->tk, tile_sweeps(B->tk), rPout);
   FL_HIP(hipGetLastError());
   return FL_OK;

@@ -111,20 +111,23 @@ struct ManySims {
 };
 
 // Pressure workspace of the temporal-blocked Gauss-Seidel kernel.
+struct GsState;  // counters of a solve's launches, on the device (fl_gs_wave.hip)
 struct GsWork {
   int tk = 0;              // sweeps per tile
   int blk = 0;             // columns per block
   int n_alloc = -1;        // sweep count the layout was built for
   int G = 0, KB = 0;       // tiles along skewed rows and along sweeps
   int rows = 0;            // handoff rows per tile (= steps per tile)
-  int ntiles = 0;          // non-empty tiles in ticket order
+  int ntiles = 0;          // non-empty tiles
+  int nq = 0;              // queues they are handed out from
   int grid = 0;            // persistent workgroups launched
   int lag = 0;             // handoff_lag of the last solve (0: none yet)
-  int32_t* d_tile = nullptr;    // [ntiles] packed (g << 16 | kb), ticket order
+  int32_t* d_tile = nullptr;    // [2 ntiles] packed (g << 16 | kb), in ticket order by queue and of all
   uint8_t* d_kout = nullptr;    // [G*KB][rows][64] K-stream handoff words
   uint8_t* d_gout = nullptr;    // [G*KB][rows][tk] G-stream handoff words
   uint8_t* d_kinit = nullptr;   // [G][rows + 1][64] the initial state as K-stream words
-  int32_t* d_ticket = nullptr;  // [4]: tickets of the main run and the re-run, re-run flag, solve number
+  int* d_first = nullptr;       // where each queue's tiles begin
+  GsState* d_state = nullptr;
 };
 
 struct Batch;
@@ -265,12 +268,14 @@ struct Batch {
   int ntiles = 0, grid = 0;
   std::vector<SimDesc> gs_fields;  // per member: G, KB, rows and its handoff slices
   int2* d_tiles = nullptr;
+  int* d_first = nullptr;
+  int nq = 0;
   uint8_t* kout = nullptr;
   uint8_t* gout = nullptr;
   uint8_t* kinit = nullptr;
   SkewItem* d_skews = nullptr;
   int nskew = 0;
-  int32_t* ticket = nullptr;
+  GsState* state = nullptr;
   float* d_omega = nullptr;
   int omega_n = -1;
   float omega_relax = 0.0f;
@@ -363,7 +368,7 @@ int batch_apply_sources(Batch* B);
 int batch_apply_edits(Batch* B, const uint32_t* keys, const float* vals, const int32_t* seg, const int32_t* segsim,
                       int nseg);
 // batched pressure solve (fl_gs_wave.hip): sets the GS fields of `descs`
-int pick_tk(const fl_params& P, int NX, int N);
+int pick_tk(const fl_params& P, int NX, int NY, int N);
 bool gs_wave_supported(Ctx* c, int numIters);
 int pick_blk(const fl_params& P);
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs);
