@@ -160,7 +160,13 @@ typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // fo
 // bottom face); pn the p of the next column.
 template <int S> struct Sweeps {
   float UrO[S], UlO[S], VbO[S], pO[S], Vt[S], pn[S], md[S], om[S];
+  float rn[S];  // coarse solve: the right-hand side of the next column
 };
+
+// What a sweep solves: the pressure projection (SOLVE_GS), or the multigrid's coarse correction
+// (SOLVE_COARSE, fluid.go:686-716: its cell needs p of the same five cells and the right-hand side,
+// which travels where V does; its words hold p for U).
+enum { SOLVE_GS, SOLVE_COARSE };
 
 // The weights of a cell by the mask of its fluid neighbours (the index, 0 for a cell that no
 // sweep updates), in LDS: what the update multiplies its faces by, 1/s, s, and a mask for div.
@@ -262,6 +268,42 @@ template <int S, int W, int B> struct GsShared {
   int tile, far;
 };
 
+// The coarse update (fluid.go:699-711) of S sweeps' cells: p of the neighbours (i - 1, j), (i + 1, j),
+// (i, j - 1), (i, j + 1) and of the cell, and its right-hand side. As in the updates above.
+template <int S> struct CoarseCells {
+  float n[S], s[S], w[S], e[S], p[S], rhs[S];
+};
+static constexpr float COARSE_RELAX = 1.6f;
+template <int S> __device__ __forceinline__ void coarse_plain(CoarseCells<S>& x) {
+  float a[S], b[S];
+  FL_EACH a[c] = x.n[c] - x.p[c];
+  FL_EACH b[c] = x.s[c] - x.p[c];
+  FL_EACH a[c] += b[c];
+  FL_EACH b[c] = x.w[c] - x.p[c];
+  FL_EACH a[c] += b[c];
+  FL_EACH b[c] = x.e[c] - x.p[c];
+  FL_EACH a[c] += b[c];
+  FL_EACH a[c] = x.rhs[c] - a[c];
+  FL_EACH a[c] *= -0.25f;
+  FL_EACH a[c] *= COARSE_RELAX;
+  FL_EACH x.p[c] += a[c];
+}
+template <int S> __device__ __forceinline__ void coarse_any(CoarseCells<S>& x, const CellW (&w)[S]) {
+  float a[S], b[S], q[S], e[S];
+  FL_EACH a[c] = -w[c].w.x * (x.n[c] - x.p[c]);
+  FL_EACH a[c] = __builtin_fmaf(w[c].w.y, x.s[c] - x.p[c], a[c]);
+  FL_EACH a[c] = __builtin_fmaf(-w[c].w.z, x.w[c] - x.p[c], a[c]);
+  FL_EACH a[c] = __builtin_fmaf(w[c].w.w, x.e[c] - x.p[c], a[c]);
+  FL_EACH a[c] = x.rhs[c] - a[c];
+  FL_EACH q[c] = -a[c] * w[c].d.x;
+  FL_EACH e[c] = __builtin_fmaf(q[c], w[c].d.y, a[c]);
+  FL_EACH q[c] = __builtin_fmaf(e[c], -w[c].d.x, q[c]);
+  FL_EACH q[c] = __builtin_amdgcn_div_fixupf(q[c], w[c].d.y, -a[c]);
+  FL_EACH q[c] *= COARSE_RELAX;
+  FL_EACH b[c] = x.p[c] + q[c];
+  FL_EACH x.p[c] = __float_as_uint(w[c].d.z) != 0u ? b[c] : x.p[c];
+}
+
 // How a block's cells are updated: all plain; with weights looked up once (along a wall, say: every
 // lane's cells of a sweep have the same mask); or with weights looked up per cell.
 enum { BLOCK_PLAIN, BLOCK_SAME, BLOCK_ANY };
@@ -277,7 +319,7 @@ enum { OUT_LDS, OUT_WORDS };
 // go: lane 63's U, V, p of each sweep after step u, at lane 64 - B + u: every step shifts them down
 // a lane and lets lane 63 in, one instruction a value into the register that the value leaves (a
 // store of lane 63 to LDS took two exec changes and two writes, 44 cycles a step for one sweep).
-template <int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL>
+template <int SOLVE, int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL>
 __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST ? B : 1], float (&k)[3],
                                           const uint32_t (&mk)[S], const float* gi, const float4* Kin, float4* Kout,
                                           float (&go)[S][3], const char* tab, __amdgpu_buffer_rsrc_t kbuf,
@@ -312,13 +354,14 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
     }
   };
   auto put = [&](int u) {
+    const float ul = SOLVE == SOLVE_GS ? Q.UlO[S - 1] : Q.pO[S - 1];
     if constexpr (OUT == OUT_LDS)
-      Kout[u * LANES] = make_float4(Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], 0.0f);
+      Kout[u * LANES] = make_float4(ul, Q.VbO[S - 1], Q.pO[S - 1], 0.0f);
     else
-      st_word<POLICY>(kbuf, kbyte + u * (LANES * 16), Q.UlO[S - 1], Q.VbO[S - 1], Q.pO[S - 1], tag);
+      st_word<POLICY>(kbuf, kbyte + u * (LANES * 16), ul, Q.VbO[S - 1], Q.pO[S - 1], tag);
 #pragma unroll
     for (int c = 0; c < S; c++) {
-      go[c][0] = from_lane_above(Q.UrO[c], go[c][0]);
+      if (SOLVE == SOLVE_GS) go[c][0] = from_lane_above(Q.UrO[c], go[c][0]);
       go[c][1] = from_lane_above(Q.VbO[c], go[c][1]);
       go[c][2] = from_lane_above(Q.pO[c], go[c][2]);
     }
@@ -336,6 +379,7 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
 #pragma unroll
   for (int u = 0; u < B; u++) {
     Cells<S> x;
+    CoarseCells<S> y;
     float pnext[S];
     if constexpr (FIRST) {
       kr[u % 2][0] = word_u(kw[u]);
@@ -344,12 +388,23 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
     }
 #pragma unroll
     for (int c = 0; c < S; c++) {
-      x.Ul[c] = from_lane_below(g[u % 2][3 * c + 2], Q.UrO[c]);
-      x.Vt[c] = from_lane_below(g[u % 2][3 * c], c ? Q.VbO[c - 1] : kr[u % 2][1]);
+      const float vnext = from_lane_below(g[u % 2][3 * c], c ? Q.VbO[c - 1] : kr[u % 2][1]);
       pnext[c] = from_lane_below(g[u % 2][3 * c + 1], c ? Q.pO[c - 1] : kr[u % 2][2]);
-      x.Ur[c] = c ? Q.UlO[c - 1] : kr[u % 2][0];
-      x.Vb[c] = Q.Vt[c];
-      x.p[c] = Q.pn[c];
+      if constexpr (SOLVE == SOLVE_GS) {
+        x.Ul[c] = from_lane_below(g[u % 2][3 * c + 2], Q.UrO[c]);
+        x.Vt[c] = vnext;
+        x.Ur[c] = c ? Q.UlO[c - 1] : kr[u % 2][0];
+        x.Vb[c] = Q.Vt[c];
+        x.p[c] = Q.pn[c];
+      } else {
+        y.n[c] = from_lane_below(g[u % 2][3 * c + 2], Q.pO[c]);
+        y.s[c] = c ? Q.pO[c - 1] : kr[u % 2][0];
+        y.w[c] = Q.Vt[c];
+        y.e[c] = pnext[c];
+        y.p[c] = Q.pn[c];
+        y.rhs[c] = Q.rn[c];
+        Q.rn[c] = vnext;
+      }
       Q.pn[c] = pnext[c];
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -359,18 +414,28 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
     if constexpr (MODE == BLOCK_ANY)
       if (u + 1 < B) load_cw(u + 1, cn);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (MODE == BLOCK_PLAIN)
+    if constexpr (SOLVE == SOLVE_GS && MODE == BLOCK_PLAIN)
       update_plain<S>(x, Q.md, Q.om, cp);
-    else
+    else if constexpr (SOLVE == SOLVE_GS)
       update_any<S, FULL>(x, Q.md, Q.om, damping, cp, cw);
+    else if constexpr (MODE == BLOCK_PLAIN)
+      coarse_plain<S>(y);
+    else
+      coarse_any<S>(y, cw);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int c = 0; c < S; c++) {
-      Q.UrO[c] = x.Ur[c];
-      Q.Vt[c] = x.Vt[c];
-      Q.UlO[c] = x.Ul[c];
-      Q.VbO[c] = x.Vb[c];
-      Q.pO[c] = x.p[c];
+      if constexpr (SOLVE == SOLVE_GS) {
+        Q.UrO[c] = x.Ur[c];
+        Q.Vt[c] = x.Vt[c];
+        Q.UlO[c] = x.Ul[c];
+        Q.VbO[c] = x.Vb[c];
+        Q.pO[c] = x.p[c];
+      } else {
+        Q.Vt[c] = y.p[c];
+        Q.VbO[c] = y.rhs[c];
+        Q.pO[c] = y.p[c];
+      }
     }
     if (MODE == BLOCK_ANY && u + 1 < B) {
 #pragma unroll
@@ -414,7 +479,7 @@ static __device__ int queue_of_tiles(const GsRun& R) {
 typedef __attribute__((address_space(3))) float lds_float;  // a pointer that lanes compute stays an LDS one
 
 // S sweeps per wave, W waves per workgroup (TK = S W sweeps per tile), B columns per block.
-template <int S, int W, int B, bool FULL, class M>
+template <int SOLVE, int S, int W, int B, bool FULL, class M>
 __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun R) {
   constexpr int TK = S * W, GP = GsShared<S, W, B>::GP;
   constexpr bool NEAR = near_tiles(TK);
@@ -491,7 +556,8 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     for (int c = 0; c < S; c++) {
       // read once into a scalar register: a vector-loaded value used in the step would make
       // every step wait for the wave's memory operations
-      Q.om[c] = uniform(k0 + b0 + c < K ? R.omega[min(k0 + b0 + c, K - 1)] : 1.0f);
+      Q.om[c] = uniform(SOLVE == SOLVE_GS && k0 + b0 + c < K ? R.omega[min(k0 + b0 + c, K - 1)] : 1.0f);
+      Q.rn[c] = 0.0f;
       Q.UrO[c] = Q.UlO[c] = Q.VbO[c] = Q.pO[c] = Q.Vt[c] = Q.pn[c] = Q.md[c] = 0.0f;
       mkeep[c] = k0 + b0 + c < K ? BITS : 0u;  // past the solve's last sweep the cells pass their faces on
       // rows 0 and NX - 1 are all 0; the copy in which this lane's columns start a byte (an odd
@@ -613,7 +679,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
+  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
         if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
         } else if (every_lane(same)) {
@@ -635,7 +701,8 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         stage(next, n1);
         if (gout) {
 #pragma unroll
-          for (int c = 0; c < S; c++) st_word<SC1>(gmine, goword + n * (B * GROW) + 16 * c, go[c][0], go[c][1], go[c][2], tag);
+          for (int c = 0; c < S; c++)
+            st_word<SC1>(gmine, goword + n * (B * GROW) + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
         }
         if (NEAR && OUT == OUT_WORDS && far) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
@@ -673,6 +740,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       else
         run_wave(later_t{}, lds_t{});
     }
+    if (SOLVE != SOLVE_GS) continue;
     // per-sweep max |div|
 #pragma unroll
     for (int c = 0; c < S; c++) {
@@ -714,7 +782,8 @@ __global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, con
   int g, t0;
   skew_item(m, items, D, g, t0);
   const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY;
-  const float* src[3] = {D->buf[B_U], D->buf[B_V], rPin >= 0 ? D->buf[rPin] : nullptr};
+  const float* src[3] = {D->buf[B_U],  // (a coarse solve has none)
+                         D->buf[B_V], rPin >= 0 ? D->buf[rPin] : nullptr};
 #pragma unroll 4
   for (int x = 0; x < 16; x++) {
     const int a = 16 * w + x, r = LANES * g + a + 1, j = t0 - a + lane;
@@ -737,17 +806,28 @@ __global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, con
   }
 }
 
+// The number of the next solve and its counters (one workgroup of the solve's last kernel).
+__device__ __forceinline__ void next_solve(GsState* S) {
+  int32_t* c = reinterpret_cast<int32_t*>(S->run);
+  for (int t = threadIdx.x; t < (int)(sizeof(S->run) / sizeof(int32_t)); t += blockDim.x) c[t] = 0;
+  if (threadIdx.x == 0) {
+    S->rerun = 0;
+    ++S->solve;
+  }
+}
+
 // The rows of the last sweep's wave (its last sweep b, padded to the wave's S) to U2, V2 and role
 // rPout: row t of row-tile g holds cell (64 g + a - k0 - b, t - a - b) at lane a. An early exit
-// (ctrl[1] sweeps) takes the re-run's. Also numbers the next solve.
+// (ctrl[1] sweeps) takes the re-run's. A coarse solve has p alone. Also numbers the next solve and
+// zeroes its counters.
 template <class M>
-__global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, int32_t* solve, int N, int tk, int S,
-                                                   int rPout) {
+__global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, GsState* state, int N, int tk, int S,
+                                                   int rPout, bool coarse) {
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
   int g, t0;
   skew_item(m, items, D, g, t0);
-  if (blockIdx.x == 0 && threadIdx.x == 0) ++*solve;
+  if (blockIdx.x == 0) next_solve(state);
   const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY, rows = D->rows;
   const int kept = D->early_exit ? D->ctrl[1] : 0, K = kept > 0 ? kept : N;
   const int kb = (K - 1) / tk, k0 = kb * tk, b = (K - 1 - k0) / S * S + S - 1;
@@ -769,8 +849,8 @@ __global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, i
     const int a = 16 * w + x, r = r0 + a, j = t0 + lane - a - b;
     if (r < 1 || r > NX - 1 || j < 1 || j > NY - 1 || t0 + lane >= rows) continue;
     const size_t c = (size_t)r * NY + j;
-    if (j <= NY - 2) dst[0][c] = sh[0][a][lane];
-    if (r <= NX - 2) dst[1][c] = sh[1][a][lane];
+    if (!coarse && j <= NY - 2) dst[0][c] = sh[0][a][lane];
+    if (!coarse && r <= NX - 2) dst[1][c] = sh[1][a][lane];
     if (r <= NX - 2 && j <= NY - 2) dst[2][c] = sh[2][a][lane];
   }
 }
@@ -808,23 +888,16 @@ template <class M> __global__ void k_gs_ring(M m, int rPin, int rPout) {
   }
 }
 
-// Zero the counters of both runs, the per-sweep maxima and the re-run requests of every
-// simulation of the launch (graph-safe: no memset).
-__device__ __forceinline__ void clear_state(GsState* S, int t) {
-  int32_t* c = reinterpret_cast<int32_t*>(S->run);
-  for (; t < (int)(sizeof(S->run) / sizeof(int32_t)); t += blockDim.x) c[t] = 0;
-  if (threadIdx.x == 0) S->rerun = 0;
-}
-__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim, GsState* S) {
+// Zero the per-sweep maxima and the re-run sweeps of every simulation of the launch (graph-safe:
+// no memset).
+__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim) {
   const int stride = blockDim.x * gridDim.x;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nmd; t += stride) maxdiv[t] = 0u;
   for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nsim; t += stride) ctrl[4 * t] = ctrl[4 * t + 1] = 0;
-  if (blockIdx.x == 0) clear_state(S, threadIdx.x);
 }
 
 // k_gs_ring and k_gs_init of a single simulation in one launch (both only precede the solve).
-__global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int nmd, int32_t* ctrl,
-                          GsState* S) {
+__global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int nmd, int32_t* ctrl) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const SimDesc& D = m.d;
   const int NX = D.g.NX, NY = D.g.NY;
@@ -839,7 +912,6 @@ __global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int n
   const int stride = blockDim.x * gridDim.x;
   for (int i = t; i < nmd; i += stride) maxdiv[i] = 0u;
   if (t == 0) ctrl[0] = ctrl[1] = 0;
-  if (blockIdx.x == 0) clear_state(S, t);
 }
 
 // Early exit of solveSingleGrid (fluid.go:175-177), one wave per simulation: the first
@@ -994,7 +1066,7 @@ template <class M> struct GsKernels {
   using Fn = void (*)(M, GsRun);
   static Fn get(int tk, int blk, bool full) {
 #define FL_GS_CASE(S, W, B) \
-  if (tk == S * W && blk == B) return full ? k_gs_wave<S, W, B, true, M> : k_gs_wave<S, W, B, false, M>;
+  if (tk == S * W && blk == B) return full ? k_gs_wave<SOLVE_GS, S, W, B, true, M> : k_gs_wave<SOLVE_GS, S, W, B, false, M>;
     FL_GS_CASE(1, 2, 4) FL_GS_CASE(1, 2, 8)
     FL_GS_CASE(1, 4, 4) FL_GS_CASE(1, 4, 8)
     FL_GS_CASE(2, 4, 4) FL_GS_CASE(2, 4, 8)
@@ -1022,14 +1094,16 @@ static int launch_gs(int tk, int blk, int grid, hipStream_t stream, const M& m, 
   return FL_OK;
 }
 
-static int layout(Ctx* c, int N) {
-  GsWork& W = c->gs;
-  const int tk = pick_tk(c->prm, c->NX, c->NY, N);
-  const int blk = pick_blk(c->prm);
+static void free_work(GsWork& W) {
+  for (void* p : {(void*)W.d_tile, (void*)W.d_first, (void*)W.d_state, (void*)W.d_kout, (void*)W.d_gout, (void*)W.d_kinit})
+    if (p) (void)hipFree(p);
+  W = GsWork{};
+}
+static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
   FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
-  pressure_free(c);
-  const TileGeom t = geom(c->NX, c->NY, N, tk, blk);
+  free_work(W);
+  const TileGeom t = geom(NX, NY, N, tk, blk);
   W.tk = tk;
   W.blk = blk;
   W.n_alloc = N;
@@ -1037,7 +1111,7 @@ static int layout(Ctx* c, int N) {
   W.KB = t.KB;
   W.rows = t.rows;
   std::vector<GsTile> order;
-  append_tiles(order, 0, 0, c->NX, N, tk, blk, t);
+  append_tiles(order, 0, 0, NX, N, tk, blk, t);
   std::vector<int2> tiles;
   std::vector<int> first;
   W.nq = device_queues(c->dev, tk);
@@ -1066,9 +1140,9 @@ static int layout(Ctx* c, int N) {
 bool gs_wave_supported(Ctx* c, int numIters) { return numIters >= 1 && c->NX >= 3 && c->NY >= 3; }
 
 int gs_wave_solve(Ctx* c, int N, float cp) {
-  int rc = layout(c, N);
-  if (rc) return rc;
   GsWork& W = c->gs;
+  int rc = layout(W, c, c->NX, c->NY, N, pick_tk(c->prm, c->NX, c->NY, N), pick_blk(c->prm));
+  if (rc) return rc;
   if (c->flags_dirty && (rc = launch_flags(c))) return rc;
   SimDesc d = c->desc();
   d.cp = cp;
@@ -1078,7 +1152,7 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   const int rPin = c->gs_p_zero ? -1 : (int)B_P;
   c->gs_p_zero = false;
   hipLaunchKernelGGL(k_gs_prep, dim3(std::max(4, (mr + 255) / 256)), dim3(256), 0, c->stream, m, rPin, (int)B_T3,
-                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl, W.d_state);
+                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl);
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
   hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, rPin);
   FL_HIP(hipGetLastError());
@@ -1104,8 +1178,8 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, N, W.tk,
-                     tile_sweeps(W.tk), (int)B_T3);
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
+                     tile_sweeps(W.tk), (int)B_T3, false);
   FL_HIP(hipGetLastError());
   std::swap(c->U, c->U2);
   std::swap(c->V, c->V2);
@@ -1115,14 +1189,50 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
 }
 
 int pressure_free(Ctx* c) {
-  GsWork& W = c->gs;
-  if (W.d_tile) (void)hipFree(W.d_tile);
-  if (W.d_kout) (void)hipFree(W.d_kout);
-  if (W.d_gout) (void)hipFree(W.d_gout);
-  if (W.d_kinit) (void)hipFree(W.d_kinit);
-  if (W.d_first) (void)hipFree(W.d_first);
-  if (W.d_state) (void)hipFree(W.d_state);
-  W = GsWork{};
+  free_work(c->gs);
+  free_work(c->mg_gs);
+  return FL_OK;
+}
+
+// solveCoarseGrid's sweeps (fluid.go:686-716) from p = 0 by the same tiles. It
+// replaces one launch per diagonal of 32 x 64 tiles and sweep, 89 launches of 24 us at 257^2:
+// 2.16 ms -> 0.16.
+int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks) {
+  GsWork& W = c->mg_gs;
+  const int blk = 8;
+  int rc = layout(W, c, cNX, cNY, N, std::min(8, pick_tk(fl_params{}, cNX, cNY, N)), blk);
+  if (rc) return rc;
+  SimDesc d = c->desc();
+  d.g.NX = cNX;
+  d.g.NY = cNY;
+  d.buf[B_U] = nullptr;
+  d.buf[B_V] = const_cast<float*>(rhs);
+  d.buf[B_T3] = p;
+  d.masks = masks;
+  d.kout = W.d_kout;
+  d.gout = W.d_gout;
+  d.kinit = W.d_kinit;
+  d.G = W.G;
+  d.KB = W.KB;
+  d.rows = W.rows;
+  d.early_exit = 0;
+  OneSim m{d};
+  const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, -1);
+  FL_HIP(hipGetLastError());
+  GsRun R{};
+  R.tiles = (const int2*)W.d_tile;
+  R.first = W.d_first;
+  R.nq = W.nq;
+  R.K = N;
+  R.solve = &W.d_state->solve;
+  R.count = &W.d_state->run[0];
+  auto fn = W.tk == 4 ? k_gs_wave<SOLVE_COARSE, 1, 4, 8, false, OneSim> : k_gs_wave<SOLVE_COARSE, 2, 4, 8, false, OneSim>;
+  hipLaunchKernelGGL(fn, dim3(W.grid), dim3(tile_waves(W.tk) * LANES), 0, c->stream, m, R);
+  FL_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
+                     tile_sweeps(W.tk), (int)B_T3, true);
+  FL_HIP(hipGetLastError());
   return FL_OK;
 }
 
@@ -1238,8 +1348,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   const int E = (int)B->members.size();
   hipLaunchKernelGGL(k_gs_ring<ManySims>, dim3(B->nring_items), dim3(256), 0, B->stream, m, rPin, rPout);
   // per-sweep maxima and re-run requests of all members are contiguous
-  hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E,
-                     B->state);
+  hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E);
   hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, &B->state->solve, B->tk,
                      rPin);
   FL_HIP(hipGetLastError());
@@ -1267,8 +1376,8 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, &B->state->solve, N,
-                     B->tk, tile_sweeps(B->tk), rPout);
+  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->state, N,
+                     B->tk, tile_sweeps(B->tk), rPout, false);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }

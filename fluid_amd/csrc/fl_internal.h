@@ -172,8 +172,9 @@ struct Ctx {
   // Multigrid V-cycle workspace (coarse grid of ((NX+1)/2) x ((NY+1)/2) cells).
   float* mg_omega = nullptr;  // [6]: the pre-smoothing (1.5) and post-smoothing (1.2) relaxation
   float* mg_P = nullptr;      // coarse correction
-  float* mg_S = nullptr;      // coarse solid mask
   float* mg_R = nullptr;      // coarse right-hand side
+  uint8_t* mg_masks = nullptr;  // SimDesc::masks of the coarse grid
+  GsWork mg_gs;               // the coarse solve's layout
 
   // Scratch of rendering, range reductions and particles (fl_render.hip).
   char* rs_mem = nullptr;
@@ -380,6 +381,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout);  // p from rPin (< 0: 
 int pressure_solve(Ctx* c, int numIters, float dt);
 // solveMultigridVCycle (fluid.go:559-596): on return the result is in (c->U, c->V, c->p).
 int multigrid_solve(Ctx* c, int numIters, float dt);
+int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks);
 int pressure_free(Ctx* c);
 
 }  // namespace fl

@@ -192,9 +192,11 @@ __global__ void k_mg_residual(Grid g, const float* __restrict__ S, const float* 
   r[c] = out;
 }
 
-// restrictResidual (fluid.go:635-664) and the coarse mask of solveCoarseGrid (fluid.go:672-684).
+// restrictResidual (fluid.go:635-664), and the masks of the coarse cells that solveCoarseGrid
+// updates (fluid.go:672-684, 692-697; laid out as k_masks writes them).
+static constexpr int MG_COARSE_ITERS = 40;
 __global__ void k_mg_restrict(Grid g, int cNX, int cNY, const float* __restrict__ S, const float* __restrict__ r,
-                              float* __restrict__ rhs, float* __restrict__ cS, float* __restrict__ cP) {
+                              float* __restrict__ rhs, uint8_t* __restrict__ masks, float* __restrict__ cP) {
   const int j = blockIdx.x * MBX + threadIdx.x, i = blockIdx.y * MBY + threadIdx.y;
   if (i >= cNX || j >= cNY) return;
   const int NX = g.NX, NY = g.NY, cc = i * cNY + j;
@@ -210,170 +212,22 @@ __global__ void k_mg_restrict(Grid g, int cNX, int cNY, const float* __restrict_
     out = center + nb + co;
   }
   rhs[cc] = out;
-  cS[cc] = (fi < NX && fj < NY) ? S[fi * NY + fj] : 0.0f;
   cP[cc] = 0.0f;
-}
-
-// solveCoarseGrid's 40 in-place lexicographic sweeps at relaxation 1.6 (fluid.go:686-716),
-// bit-identical to the serial loop. The interior is cut into tiles (I, J) of 32 rows (i) by
-// 64 columns (j), 26 KB of LDS, six workgroups to a CU. Tile (I, J) runs sweep k in the launch
-// for diagonal T = I + J + 2k. Its four neighbour tiles then hold the values the serial order
-// reads: (I-1, J) and (I, J-1) have done sweep k (diagonal T-1), (I+1, J) and (I, J+1) sweep
-// k-1 but not k (T-1 and T+1). No two tiles of one diagonal are neighbours (their T would
-// differ by an odd number), so a tile reads its one-cell halo once at the start and writes its
-// interior back at the end. Inside, one wave walks the tile's anti-diagonals (the other three
-// waves help load and store the tile): lane l updates column l, row d - l at step d, after
-// (row - 1, l) and (row, l - 1) (step d - 1, this lane and lane l - 1) and before (row + 1, l)
-// and (row, l + 1). Every step runs the reference's expression on the same operands, so the
-// result is the serial loop's to the bit.
-// ALL: the interior is one tile of at most TR x 64 cells, and the launch runs all 40 sweeps on
-// it in LDS, the four waves walking successive sweeps three steps apart (below), instead of one
-// launch per sweep.
-static constexpr int MG_COARSE_ITERS = 40, MG_TR = 32, MG_TR_ALL = 64, MG_TC = 64, MG_PITCH = MG_TC + 2;
-
-template <int TR, bool ALL>
-__global__ __launch_bounds__(256) void k_mg_coarse_tiles(int cNX, int cNY, int nI, int nJ, int T, int klo,
-                                                         const float* __restrict__ cS,
-                                                         const float* __restrict__ rhs, float* __restrict__ cP) {
-  constexpr int MG_TR = TR;
-  const int k = klo + blockIdx.y, I = blockIdx.x, J = T - 2 * k - I;
-  if (J < 0 || J >= nJ) return;
-  __shared__ float lp[(MG_TR + 2) * MG_PITCH], ls[(MG_TR + 2) * MG_PITCH], lr[MG_TR * MG_TC];
-  const int W = cNX - 2, H = cNY - 2;
-  const int i0 = 1 + I * MG_TR, j0 = 1 + J * MG_TC;  // first interior cell of the tile
-  const int rows = min(MG_TR, W - I * MG_TR), cols = min(MG_TC, H - J * MG_TC);
-  const int tid = threadIdx.x, l = tid & 63;
-  // Load: rows i0-1 .. i0+rows and columns j0-1 .. j0+cols, all inside the grid (i0+rows <=
-  // W+1 = cNX-1), as one flat range over the four waves with every load in flight at once.
-  // The corners belong to diagonal tiles and are never read.
-  const int pw = cols + 2, n = (rows + 2) * pw;
-  constexpr int LU = ((MG_TR + 2) * MG_PITCH + 255) / 256;
-  float vp[LU], vs[LU], vr[LU];
-#pragma unroll
-  for (int u = 0; u < LU; u++) {
-    const int e = tid + 256 * u, r = e / pw - 1, q = e - (r + 1) * pw;
-    const bool in = e < n && !((r < 0 || r == rows) && (q == 0 || q == cols + 1));
-    const size_t g = (size_t)(i0 + r) * cNY + j0 - 1 + q;
-    vp[u] = in ? cP[g] : 0.0f;
-    vs[u] = in ? cS[g] : 0.0f;
-    vr[u] = (in && r >= 0 && r < rows && q >= 1 && q <= cols) ? rhs[g] : 0.0f;
-  }
-#pragma unroll
-  for (int u = 0; u < LU; u++) {
-    const int e = tid + 256 * u, r = e / pw - 1, q = e - (r + 1) * pw;
-    if (e < n) {
-      lp[(r + 1) * MG_PITCH + q] = vp[u];
-      ls[(r + 1) * MG_PITCH + q] = vs[u];
-      if (r >= 0 && r < rows && q >= 1 && q <= cols) lr[r * MG_TC + q - 1] = vr[u];
-    }
-  }
-  __syncthreads();
-  // The walk. Lane l is at row r = d - l at step d (also before and after its active rows, so
-  // its registers are there for its neighbours) and holds its column's S[r-1..r+1], the old
-  // P[r], P[r+1], rhs[r] and cur = P[r-1] after this sweep. Lane l-1 (row r+1) passes on the
-  // new P[r][l-1] and S[r][l-1]; lane l+1 (row r-1) the old P[r][l+1] and S[r][l+1], by wave
-  // shifts in full-wave control flow. Lane 0 and lane 63 take the halo columns instead; for a
-  // narrower tile, lane `cols` walks the east halo column. LDS is only read here (the cells a
-  // lane will still read are never the ones written), so the walk needs no barrier; results
-  // go to LDS for the write-back.
-  const float relax = 1.6f;
-  auto row_of = [&](int x) { return min(max(x, -1), rows) + 1; };  // LDS row of row x, clamped
-  const int col = l + 1;                                                // LDS column of this lane
-  int r = 0;
-  float sm1 = 0.0f, s0 = 0.0f, sp1 = 0.0f, po = 0.0f, po1 = 0.0f, cur = 0.0f, rh = 0.0f;
-  auto init = [&]() {
-    r = -l;
-    sm1 = ls[row_of(r - 1) * MG_PITCH + col];
-    s0 = ls[row_of(r) * MG_PITCH + col];
-    sp1 = ls[row_of(r + 1) * MG_PITCH + col];
-    po = lp[row_of(r) * MG_PITCH + col];
-    po1 = lp[row_of(r + 1) * MG_PITCH + col];
-    cur = lp[row_of(r - 1) * MG_PITCH + col];
-    rh = lr[min(max(r, 0), rows - 1) * MG_TC + l];
+  auto fluid = [&](int a, int b) -> uint32_t {  // coarse cell (a, b)
+    return 2 * a < NX && 2 * b < NY && S[(2 * a) * NY + 2 * b] != 0.0f;
   };
-  auto step = [&]() {
-    const int hrow = row_of(r) * MG_PITCH;
-    const float pWh = lp[hrow], sWh = ls[hrow], pEh = lp[hrow + cols + 1], sEh = ls[hrow + cols + 1];
-    const float pW = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(pWh), __float_as_int(cur), 0x138, 0xF, 0xF, false));
-    const float sy0 = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sWh), __float_as_int(sm1), 0x138, 0xF, 0xF, false));
-    const float pE = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(pEh), __float_as_int(po1), 0x130, 0xF, 0xF, false));
-    const float sy1 = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sEh), __float_as_int(sp1), 0x130, 0xF, 0xF, false));
-    // next row's values (prefetched before the update's dependent chain)
-    const float sp2 = ls[row_of(r + 2) * MG_PITCH + col], po2 = lp[row_of(r + 2) * MG_PITCH + col];
-    const float rh1 = lr[min(max(r + 1, 0), rows - 1) * MG_TC + l];
-    float pn = po;
-    const bool active = l < cols && r >= 0 && r < rows;
-    if (active && s0 != 0.0f) {
-      const float sx0 = sm1, sx1 = sp1;
-      const float s = sx0 + sx1 + sy0 + sy1;
-      if (s != 0.0f) {
-        const float pc = po;
-        const float lap = sx0 * (cur - pc) + sx1 * (po1 - pc) + sy0 * (pW - pc) + sy1 * (pE - pc);
-        const float res = rh - lap;
-        const float corr = -res / s * relax;
-        pn = pc + corr;
-      }
-    }
-    if (active) lp[(r + 1) * MG_PITCH + col] = pn;
-    cur = pn;
-    sm1 = s0;
-    s0 = sp1;
-    sp1 = sp2;
-    po = po1;
-    po1 = po2;
-    rh = rh1;
-    r++;
+  auto mask = [&](int b) -> uint32_t {  // of coarse cell (i, b)
+    if (i < 1 || i > cNX - 2 || b < 1 || b > cNY - 2 || !fluid(i, b)) return 0u;
+    return fluid(i - 1, b) | fluid(i + 1, b) << 1 | fluid(i, b - 1) << 2 | fluid(i, b + 1) << 3;
   };
-  if constexpr (ALL) {
-    // The 40 walks overlap on the four waves: wave w walks sweeps w, w+4, ..., and sweep k
-    // starts at step (k / 4) P + 3 (k % 4) of a common clock with a barrier per step. A walk
-    // at step d reads old values (the previous sweep's) on anti-diagonals up to d + 2, which
-    // that sweep wrote at its step d + 2, at least one barrier earlier (lag 3 >= 2 + 1); it
-    // writes anti-diagonal d after the previous sweep read it there (at that sweep's step d - 2).
-    // P >= 12 keeps the lag from sweep 4m+3 to 4m+4 at 3 or more on small tiles.
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int D = rows + cols - 1, P = max(D, 12), M = MG_COARSE_ITERS / 4;
-    const int total = (M - 1) * P + 9 + D;
-    for (int tau = 0; tau < total; tau++) {
-      const int x = tau - 3 * wv;
-      if (x >= 0 && x < M * P) {
-        const int d = x % P;
-        if (d == 0) init();
-        if (d < D) step();
-      }
-      __syncthreads();
-    }
-  } else if (tid < 64) {
-    init();
-    for (int d = 0; d < rows + cols - 1; d++) step();
-  }
-  __syncthreads();
-  for (int e = tid; e < rows * cols; e += 256) {
-    const int r = e / cols, q = e - r * cols;
-    cP[(size_t)(i0 + r) * cNY + j0 + q] = lp[(r + 1) * MG_PITCH + q + 1];
-  }
-}
-
-// All 40 coarse sweeps: one launch when the interior fits one tile of 64 x 64, else one
-// launch per tile diagonal, in order on the stream.
-static int mg_coarse_solve(Ctx* c, int cNX, int cNY) {
-  const int W = cNX - 2, H = cNY - 2, K = MG_COARSE_ITERS;
-  if (W < 1 || H < 1) return FL_OK;
-  if (W <= MG_TR_ALL && H <= MG_TC) {
-    hipLaunchKernelGGL((k_mg_coarse_tiles<MG_TR_ALL, true>), dim3(1, 1), dim3(256), 0, c->stream, cNX, cNY, 1, 1, 0,
-                       0, c->mg_S, c->mg_R, c->mg_P);
-    FL_HIP(hipGetLastError());
-    return FL_OK;
-  }
-  const int nI = (W + MG_TR - 1) / MG_TR, nJ = (H + MG_TC - 1) / MG_TC;
-  for (int T = 0; T <= (nI - 1) + (nJ - 1) + 2 * (K - 1); T++) {
-    const int klo = std::max(0, (T - (nI - 1) - (nJ - 1) + 1) / 2), khi = std::min(K - 1, T / 2);
-    if (klo > khi) continue;  // no tile on this diagonal (a one-tile grid has none on odd T)
-    hipLaunchKernelGGL((k_mg_coarse_tiles<MG_TR, false>), dim3(nI, khi - klo + 1), dim3(256), 0, c->stream, cNX, cNY,
-                       nI, nJ, T, klo, c->mg_S, c->mg_R, c->mg_P);
-  }
-  FL_HIP(hipGetLastError());
-  return FL_OK;
+  const uint32_t pitch = mask_pitch(cNY);
+  uint8_t* row = masks + (size_t)i * pitch + MASK_PAD / 2;
+  const uint32_t lo = mask(j), hi = mask(j + 1);
+  if (j & 1)
+    row[(size_t)cNX * pitch + (j + 1) / 2] = (uint8_t)(lo | hi << 4);
+  else
+    row[j / 2] = (uint8_t)(lo | hi << 4);
+  if (j == 0) row[(size_t)cNX * pitch] = (uint8_t)(lo << 4);
 }
 
 // prolongateCorrection (fluid.go:719-756) at one fine cell.
@@ -424,10 +278,11 @@ int multigrid_solve(Ctx* c, int numIters, float dt) {
   const size_t cN = (size_t)cNX * cNY;
   if (!c->mg_omega) {
     const float om[6] = {1.5f, 1.5f, 1.5f, 1.2f, 1.2f, 1.2f};
-    FL_HIP(hipMalloc(&c->mg_omega, sizeof(om)));
     FL_HIP(hipMalloc(&c->mg_P, 4 * cN));
-    FL_HIP(hipMalloc(&c->mg_S, 4 * cN));
+    FL_HIP(hipMalloc(&c->mg_masks, mask_bytes(cNX, cNY)));
     FL_HIP(hipMalloc(&c->mg_R, 4 * cN));
+    FL_HIP(hipMalloc(&c->mg_omega, sizeof(om)));
+    FL_HIP(hipMemsetAsync(c->mg_masks, 0, mask_bytes(cNX, cNY), c->stream));
     FL_HIP(hipMemcpy(c->mg_omega, om, sizeof(om), hipMemcpyHostToDevice));
   }
   const float cp = c->density * c->h / dt;
@@ -452,9 +307,10 @@ int multigrid_solve(Ctx* c, int numIters, float dt) {
     std::memcpy(&maxDiv, &bits, 4);
     if (maxDiv < 1e-5f) break;
     hipLaunchKernelGGL(k_mg_residual, fg, fb, 0, c->stream, c->grid, c->S, c->U, c->V, c->p, c->T0);
-    hipLaunchKernelGGL(k_mg_restrict, cg, fb, 0, c->stream, c->grid, cNX, cNY, c->S, c->T0, c->mg_R, c->mg_S,
-                       c->mg_P);
-    if ((rc = mg_coarse_solve(c, cNX, cNY))) return restore(), rc;
+    hipLaunchKernelGGL(k_mg_restrict, cg, fb, 0, c->stream, c->grid, cNX, cNY, c->S, c->T0, c->mg_R,
+                       c->mg_masks, c->mg_P);
+    if (cNX >= 3 && cNY >= 3 && (rc = gs_coarse_solve(c, cNX, cNY, MG_COARSE_ITERS, c->mg_R, c->mg_P, c->mg_masks)))
+      return restore(), rc;
     hipLaunchKernelGGL(k_mg_apply, fg, fb, 0, c->stream, c->grid, cNX, cNY, c->S, c->mg_P, cp, c->U, c->V, c->p);
     FL_HIP(hipGetLastError());
     c->d_omega = c->mg_omega + 3;

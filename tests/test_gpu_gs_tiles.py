@@ -1,7 +1,7 @@
 """The temporal-blocked solve at the edges of its tiles, bit for bit against the oracle: grids of
 one cell, one lane more or less than a 64-row tile and one column more or less than a block of
 columns; sweep counts that do not fill a tile or a wave's pair of sweeps; blocks of cells with all
-neighbours, walls only and scattered solids; the parameters that need the selecting update
+neighbours, walls only and scattered solids; the multigrid's coarse solve on the same tiles; the parameters that need the selecting update
 (damping, negative relaxation and dt); faces that are infinite or NaN. The tolerance is zero: the
 solve performs the oracle's float32 operations in the oracle's order (NaN compares by position)."""
 import numpy as np
@@ -53,3 +53,11 @@ def test_edges_of_tiles(w, h, sweeps, tk, blk):
                                   dict(special=True, steps=1)], ids=str)
 def test_cells_and_parameters(case, tk, blk):
     run(150, 41, 21, tk, blk, **case)
+
+
+@pytest.mark.parametrize("w,h", [(3, 3), (4, 130), (122, 12), (126, 30), (130, 31), (3300, 3900)])
+@pytest.mark.parametrize("solid", [0.0, 0.05])
+def test_multigrid_coarse_tiles(w, h, solid):
+    """Coarse interiors of one cell, one row more or less than a tile, and (the last) more than
+    256 tiles of four sweeps in flight, so tiles of eight."""
+    run(w, h, 1, 0, 0, solid=solid, steps=2 if w < 1000 else 1, UseMultigrid=True)
