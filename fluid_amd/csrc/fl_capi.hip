@@ -372,13 +372,13 @@ void free_ctx(Ctx* c) {
       if (*b) (void)hipFree(*b);
     if (c->flags) (void)hipFree(c->flags);
     if (c->masks) (void)hipFree(c->masks);
-    if (c->mg_masks) (void)hipFree(c->mg_masks);
     if (c->keep) (void)hipFree(c->keep);
     if (c->d_ctrl) (void)hipFree(c->d_ctrl);
     if (c->d_maxdiv) (void)hipFree(c->d_maxdiv);
   }
   for (float** b : {&c->d_omega, &c->d_edit_vals, &c->d_xy, &c->mg_omega, &c->mg_P, &c->mg_R})
     if (*b) (void)hipFree(*b);
+  if (c->mg_masks) (void)hipFree(c->mg_masks);
   if (c->d_red) (void)hipFree(c->d_red);
   if (c->rs_mem) (void)hipFree(c->rs_mem);
   if (c->stage) (void)hipHostFree(c->stage);
