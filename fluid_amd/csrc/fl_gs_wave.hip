@@ -753,8 +753,13 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
 }
 
 // The initial state in the solve's layout, and the result out of it. An item is 64 rows of words of
-// one row-tile; each of a workgroup's four waves moves 16 of the tile's 64 grid rows, 64 columns
-// each, through LDS, so that both sides read and write whole lines.
+// one row-tile; each of a workgroup's SKEW_WAVES waves moves SKEW_ROWS of the tile's 64 grid rows, 64
+// columns each, through LDS, so that both sides read and write whole lines. Bound by the latency of
+// its loads on small grids (30 items at 256^2) and by memory on large ones, so a wave has all of its
+// loads in flight at once: with 4, 8 and 16 waves k_gs_skew took 13.4, 8.4 and 6.3 us at 256^2, 277,
+// 199 and 166 us on an ensemble of 18.6 M cells, 165, 114 and 100 us (4.7 TB/s) at 4096^2; k_gs_unskew
+// 8.4, 6.4 and 5.2 us, 168, 135 and 133 us, 103 us.
+static constexpr int SKEW_WAVES = 16, SKEW_ROWS = LANES / SKEW_WAVES;
 __device__ __forceinline__ bool skew_item(const OneSim& m, int, const SimDesc*& D, int& g, int& t0) {
   D = &m.d;
   const int nt = (D->rows + 1 + LANES - 1) / LANES;
@@ -776,7 +781,7 @@ __device__ __forceinline__ bool skew_item(const OneSim& m, const SkewItem*, cons
 // Row t (stored at t + 1) of row-tile g holds, at lane a, U, V and p of cell (64 g + a + 1, t - a + 1):
 // what lane a of a sweep before the first would have left at step t.
 template <class M>
-__global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int tk, int rPin) {
+__global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int tk, int rPin) {
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
   int g, t0;
@@ -784,9 +789,9 @@ __global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, con
   const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY;
   const float* src[3] = {D->buf[B_U],  // (a coarse solve has none)
                          D->buf[B_V], rPin >= 0 ? D->buf[rPin] : nullptr};
-#pragma unroll 4
-  for (int x = 0; x < 16; x++) {
-    const int a = 16 * w + x, r = LANES * g + a + 1, j = t0 - a + lane;
+#pragma unroll
+  for (int x = 0; x < SKEW_ROWS; x++) {
+    const int a = SKEW_ROWS * w + x, r = LANES * g + a + 1, j = t0 - a + lane;
     const bool in = r < NX && j >= 0 && j < NY;
 #pragma unroll
     for (int f = 0; f < 3; f++) sh[f][a][lane] = in && src[f] ? src[f][(size_t)r * NY + j] : 0.0f;
@@ -796,9 +801,9 @@ __global__ __launch_bounds__(256) void k_gs_skew(M m, const SkewItem* items, con
   const __amdgpu_buffer_rsrc_t dst = word_buffer(D->kinit + (size_t)g * (D->rows + 1) * (16 * LANES));
   // lane 63's also as the last sweep's of the G stream's first column
   const __amdgpu_buffer_rsrc_t gdst = word_buffer(D->gout + (size_t)g * (D->KB + 1) * D->rows * (16 * tk));
-#pragma unroll 4
-  for (int x = 0; x < 16; x++) {
-    const int u = 16 * w + x;
+#pragma unroll
+  for (int x = 0; x < SKEW_ROWS; x++) {
+    const int u = SKEW_ROWS * w + x;
     if (t0 + u <= D->rows)
       st_word<CACHED>(dst, (uint32_t)(t0 + u) * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
     if (lane == LANES - 1 && t0 + u < D->rows)
@@ -821,7 +826,7 @@ __device__ __forceinline__ void next_solve(GsState* S) {
 // (ctrl[1] sweeps) takes the re-run's. A coarse solve has p alone. Also numbers the next solve and
 // zeroes its counters.
 template <class M>
-__global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, GsState* state, int N, int tk, int S,
+__global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const SkewItem* items, GsState* state, int N, int tk, int S,
                                                    int rPout, bool coarse) {
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
@@ -834,9 +839,9 @@ __global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, G
   const int r0 = LANES * g - k0 - b;  // row of lane 0
   if (r0 > NX - 1 || r0 + LANES - 1 < 1) return;
   const __amdgpu_buffer_rsrc_t src = word_buffer(D->kout + (size_t)(g * D->KB + kb) * rows * (16 * LANES));
-#pragma unroll 4
-  for (int x = 0; x < 16; x++) {
-    const int u = 16 * w + x;
+#pragma unroll
+  for (int x = 0; x < SKEW_ROWS; x++) {
+    const int u = SKEW_ROWS * w + x;
     const word4 v = ld_word(src, (uint32_t)min(t0 + u, rows - 1) * (16 * LANES) + 16 * lane);
     sh[0][lane][u] = word_u(v);
     sh[1][lane][u] = word_v(v);
@@ -844,9 +849,9 @@ __global__ __launch_bounds__(256) void k_gs_unskew(M m, const SkewItem* items, G
   }
   __syncthreads();
   float* const dst[3] = {D->buf[B_U2], D->buf[B_V2], D->buf[rPout]};
-#pragma unroll 4
-  for (int x = 0; x < 16; x++) {
-    const int a = 16 * w + x, r = r0 + a, j = t0 + lane - a - b;
+#pragma unroll
+  for (int x = 0; x < SKEW_ROWS; x++) {
+    const int a = SKEW_ROWS * w + x, r = r0 + a, j = t0 + lane - a - b;
     if (r < 1 || r > NX - 1 || j < 1 || j > NY - 1 || t0 + lane >= rows) continue;
     const size_t c = (size_t)r * NY + j;
     if (!coarse && j <= NY - 2) dst[0][c] = sh[0][a][lane];
@@ -1154,7 +1159,7 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   hipLaunchKernelGGL(k_gs_prep, dim3(std::max(4, (mr + 255) / 256)), dim3(256), 0, c->stream, m, rPin, (int)B_T3,
                      c->d_maxdiv, 2 * c->nmax, c->d_ctrl);
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
-  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, rPin);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
@@ -1178,7 +1183,7 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
                      tile_sweeps(W.tk), (int)B_T3, false);
   FL_HIP(hipGetLastError());
   std::swap(c->U, c->U2);
@@ -1218,7 +1223,7 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
   d.early_exit = 0;
   OneSim m{d};
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
-  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, -1);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, -1);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
@@ -1230,7 +1235,7 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
   auto fn = W.tk == 4 ? k_gs_wave<SOLVE_COARSE, 1, 4, 8, false, OneSim> : k_gs_wave<SOLVE_COARSE, 2, 4, 8, false, OneSim>;
   hipLaunchKernelGGL(fn, dim3(W.grid), dim3(tile_waves(W.tk) * LANES), 0, c->stream, m, R);
   FL_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(256), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
+  hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
                      tile_sweeps(W.tk), (int)B_T3, true);
   FL_HIP(hipGetLastError());
   return FL_OK;
@@ -1349,7 +1354,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   hipLaunchKernelGGL(k_gs_ring<ManySims>, dim3(B->nring_items), dim3(256), 0, B->stream, m, rPin, rPout);
   // per-sweep maxima and re-run requests of all members are contiguous
   hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E);
-  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, &B->state->solve, B->tk,
+  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(SKEW_WAVES * LANES), 0, B->stream, m, B->d_skews, &B->state->solve, B->tk,
                      rPin);
   FL_HIP(hipGetLastError());
   GsRun R{};
@@ -1376,7 +1381,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
       FL_HIP(hipGetLastError());
     }
   }
-  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(256), 0, B->stream, m, B->d_skews, B->state, N,
+  hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(SKEW_WAVES * LANES), 0, B->stream, m, B->d_skews, B->state, N,
                      B->tk, tile_sweeps(B->tk), rPout, false);
   FL_HIP(hipGetLastError());
   return FL_OK;
