@@ -90,7 +90,7 @@ struct GsRun {
   int which;          // 0 main run (K sweeps), 1 re-run (ctrl[1] sweeps of each simulation)
   int K;
   GsCounters* count;
-  const int32_t* rerun;  // re-run launch only: nonzero when some simulation asked for one
+  const int32_t* rerun;  // a batch's re-run launch only: nonzero when some simulation asked for one
   const int32_t* solve;
   const float* omega;
   float damping;
@@ -138,6 +138,21 @@ __device__ __forceinline__ int ld_err(const int32_t* p) {
 
 __device__ __forceinline__ const SimDesc& sim_desc(const OneSim& m, int) { return m.d; }
 __device__ __forceinline__ const SimDesc& sim_desc(const ManySims& m, int e) { return m.sims[e]; }
+
+// Early exit of solveSingleGrid (fluid.go:175-177): the sweeps to re-run of a main run of N, up to
+// the first whose max |div| is below 1e-5, or 0 if that is the last or none. By one wave: lane l scans
+// sweeps l, l+64, ...; the wave's minimum is the first such sweep.
+__device__ __forceinline__ int sweeps_to_rerun(const SimDesc& D, int N) {
+  int first = N;
+  if (D.early_exit)
+    for (int k = threadIdx.x & (LANES - 1); k < N; k += LANES)
+      if (__uint_as_float(D.maxdiv[k]) < 1e-5f) {
+        first = k;
+        break;
+      }
+  for (int o = LANES / 2; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, LANES));
+  return first + 1 < N ? first + 1 : 0;
+}
 
 // Lane a takes lane a-1's v; lane 0 takes its own `first`.
 __device__ __forceinline__ float from_lane_below(float first, float v) {
@@ -490,8 +505,18 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
   const int lane = threadIdx.x & (LANES - 1);
   // wave-uniform, and held in a scalar register so every test on it is a scalar branch
   const int w = uniform((int)(threadIdx.x / LANES));
-  // a re-run launch with nothing to re-run ends here, in every workgroup alike
-  if (R.rerun && *R.rerun == 0) return;
+  // a re-run launch with nothing to re-run ends here, in every workgroup alike. A single
+  // simulation's decides it here, in every wave (by a launch of its own, 4.5 us a solve).
+  int again = 0;
+  if constexpr (std::is_same<M, OneSim>::value) {
+    if (R.which) {
+      again = uniform(sweeps_to_rerun(m.d, R.K));
+      if (blockIdx.x == 0 && threadIdx.x == 0) m.d.ctrl[1] = again;
+      if (!again) return;
+    }
+  } else {
+    if (R.rerun && *R.rerun == 0) return;
+  }
   if (threadIdx.x < 16) {
     const CellW c = cell_weights(threadIdx.x);
     sh.tabw[threadIdx.x] = c.w;
@@ -520,7 +545,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const int NX = D.g.NX, NY = D.g.NY, rows = D.rows, KB = D.KB;
     const int nblk = rows / B;
     int32_t* err = D.ctrl + 3;
-    const int K = R.which ? D.ctrl[1] : R.K;
+    const int K = !R.which ? R.K : std::is_same<M, OneSim>::value ? again : D.ctrl[1];
     const int Kp = (K + S - 1) / S * S;  // with the sweeps that only fill the last wave
     if (tile_empty(g, kb, Kp, TK, NX)) continue;
     const float cp = D.cp, damping = R.damping;
@@ -760,32 +785,83 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
 // 199 and 166 us on an ensemble of 18.6 M cells, 165, 114 and 100 us (4.7 TB/s) at 4096^2; k_gs_unskew
 // 8.4, 6.4 and 5.2 us, 168, 135 and 133 us, 103 us.
 static constexpr int SKEW_WAVES = 16, SKEW_ROWS = LANES / SKEW_WAVES;
-__device__ __forceinline__ bool skew_item(const OneSim& m, int, const SimDesc*& D, int& g, int& t0) {
+__device__ __forceinline__ void skew_item(const OneSim& m, const SkewItem*, int item, const SimDesc*& D, int& g, int& t0) {
   D = &m.d;
   const int nt = (D->rows + 1 + LANES - 1) / LANES;
-  g = blockIdx.x / nt;
-  t0 = (blockIdx.x % nt) * LANES;
-  return true;
+  g = item / nt;
+  t0 = (item % nt) * LANES;
 }
-__device__ __forceinline__ bool skew_item(const ManySims& m, const SkewItem* items, const SimDesc*& D, int& g, int& t0) {
-  const SkewItem it = items[blockIdx.x];
+__device__ __forceinline__ void skew_item(const ManySims& m, const SkewItem* items, int item, const SimDesc*& D, int& g,
+                                          int& t0) {
+  const SkewItem it = items[item];
   D = &m.sims[it.sim];
   g = it.g;
   t0 = it.t0;
-  return true;
 }
-__device__ __forceinline__ bool skew_item(const OneSim& m, const SkewItem*, const SimDesc*& D, int& g, int& t0) {
-  return skew_item(m, 0, D, g, t0);
+
+// Faces and cells no interior cell touches keep their input values: U with i = 0 or
+// j in {0, NY-1}; V with i in {0, NX-1} or j = 0; p on the ring. All lie on the ring.
+__device__ __forceinline__ void ring_copy(const SimDesc& D, int i, int j, int rPin, int rPout) {
+  const int NX = D.g.NX, NY = D.g.NY;
+  const size_t c = (size_t)i * NY + j;
+  if (!(i >= 1 && j >= 1 && j <= NY - 2)) D.buf[B_U2][c] = D.buf[B_U][c];
+  if (!(i >= 1 && i <= NX - 2 && j >= 1)) D.buf[B_V2][c] = D.buf[B_V][c];
+  D.buf[rPout][c] = rPin >= 0 ? D.buf[rPin][c] : 0.0f;
+}
+// Ring item `item` of 256 cells of each side, by thread t of 256.
+__device__ __forceinline__ void ring_desc(const OneSim& m, int item, const SimDesc*& D, int& t) {
+  D = &m.d;
+  t += item * 256;
+}
+__device__ __forceinline__ void ring_desc(const ManySims& m, int item, const SimDesc*& D, int& t) {
+  const RingItem it = m.rings[item];
+  D = &m.sims[it.sim];
+  t += it.blk * 256;
+}
+// What precedes a solve besides its layout: the ring, and the per-sweep maxima and re-run sweeps of
+// every simulation set to zero. It only has to come before the solve, so it takes the first
+// workgroups of the layout's launch (a launch of its own took 4.7 us, two in a batch).
+struct GsPrep {
+  int groups, rings;  // workgroups, ring items
+  int rPout;
+  uint32_t* maxdiv;
+  int nmd;
+  int32_t* ctrl;
+  int nsim;
+};
+static constexpr int RINGS_PER_GROUP = SKEW_WAVES * LANES / 256;
+static int prep_groups(int rings) { return (rings + RINGS_PER_GROUP - 1) / RINGS_PER_GROUP; }
+template <class M> __device__ __forceinline__ void prepare_solve(const M& m, const GsPrep& P, int rPin) {
+  const int item = blockIdx.x * RINGS_PER_GROUP + threadIdx.x / 256;
+  if (item < P.rings) {
+    const SimDesc* D;
+    int t = threadIdx.x % 256;
+    ring_desc(m, item, D, t);
+    const int NX = D->g.NX, NY = D->g.NY;
+    if (t < NX) {
+      ring_copy(*D, t, 0, rPin, P.rPout);
+      ring_copy(*D, t, NY - 1, rPin, P.rPout);
+    }
+    if (t < NY) {
+      ring_copy(*D, 0, t, rPin, P.rPout);
+      ring_copy(*D, NX - 1, t, rPin, P.rPout);
+    }
+  }
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = P.groups * blockDim.x;
+  for (int t = t0; t < P.nmd; t += stride) P.maxdiv[t] = 0u;
+  for (int t = t0; t < P.nsim; t += stride) P.ctrl[4 * t] = P.ctrl[4 * t + 1] = 0;
 }
 
 // Row t (stored at t + 1) of row-tile g holds, at lane a, U, V and p of cell (64 g + a + 1, t - a + 1):
 // what lane a of a sweep before the first would have left at step t.
 template <class M>
-__global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int tk, int rPin) {
+__global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_skew(M m, const SkewItem* items, const int32_t* solve, int tk, int rPin,
+                                                                 GsPrep P) {
   __shared__ float sh[3][LANES][LANES + 1];
+  if (blockIdx.x < (unsigned)P.groups) return prepare_solve(m, P, rPin);
   const SimDesc* D;
   int g, t0;
-  skew_item(m, items, D, g, t0);
+  skew_item(m, items, blockIdx.x - P.groups, D, g, t0);
   const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY;
   const float* src[3] = {D->buf[B_U],  // (a coarse solve has none)
                          D->buf[B_V], rPin >= 0 ? D->buf[rPin] : nullptr};
@@ -831,7 +907,7 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const Ske
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
   int g, t0;
-  skew_item(m, items, D, g, t0);
+  skew_item(m, items, blockIdx.x, D, g, t0);
   if (blockIdx.x == 0) next_solve(state);
   const int lane = threadIdx.x & 63, w = threadIdx.x / 64, NX = D->g.NX, NY = D->g.NY, rows = D->rows;
   const int kept = D->early_exit ? D->ctrl[1] : 0, K = kept > 0 ? kept : N;
@@ -860,87 +936,16 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const Ske
   }
 }
 
-// Faces and cells no interior cell touches keep their input values: U with i = 0 or
-// j in {0, NY-1}; V with i in {0, NX-1} or j = 0; p on the ring. All lie on the ring.
-__device__ __forceinline__ void ring_copy(const SimDesc& D, int i, int j, int rPin, int rPout) {
-  const int NX = D.g.NX, NY = D.g.NY;
-  const size_t c = (size_t)i * NY + j;
-  if (!(i >= 1 && j >= 1 && j <= NY - 2)) D.buf[B_U2][c] = D.buf[B_U][c];
-  if (!(i >= 1 && i <= NX - 2 && j >= 1)) D.buf[B_V2][c] = D.buf[B_V][c];
-  D.buf[rPout][c] = rPin >= 0 ? D.buf[rPin][c] : 0.0f;
-}
-__device__ __forceinline__ void ring_desc(const OneSim& m, const SimDesc*& D, int& t) {
-  D = &m.d;
-  t = blockIdx.x * blockDim.x + threadIdx.x;
-}
-__device__ __forceinline__ void ring_desc(const ManySims& m, const SimDesc*& D, int& t) {
-  const RingItem it = m.rings[blockIdx.x];
-  D = &m.sims[it.sim];
-  t = it.blk * blockDim.x + threadIdx.x;
-}
-template <class M> __global__ void k_gs_ring(M m, int rPin, int rPout) {
-  const SimDesc* D;
-  int t;
-  ring_desc(m, D, t);
-  const int NX = D->g.NX, NY = D->g.NY;
-  if (t < NX) {
-    ring_copy(*D, t, 0, rPin, rPout);
-    ring_copy(*D, t, NY - 1, rPin, rPout);
-  }
-  if (t < NY) {
-    ring_copy(*D, 0, t, rPin, rPout);
-    ring_copy(*D, NX - 1, t, rPin, rPout);
-  }
-}
-
-// Zero the per-sweep maxima and the re-run sweeps of every simulation of the launch (graph-safe:
-// no memset).
-__global__ void k_gs_init(uint32_t* maxdiv, int nmd, int32_t* ctrl, int nsim) {
-  const int stride = blockDim.x * gridDim.x;
-  for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nmd; t += stride) maxdiv[t] = 0u;
-  for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < nsim; t += stride) ctrl[4 * t] = ctrl[4 * t + 1] = 0;
-}
-
-// k_gs_ring and k_gs_init of a single simulation in one launch (both only precede the solve).
-__global__ void k_gs_prep(OneSim m, int rPin, int rPout, uint32_t* maxdiv, int nmd, int32_t* ctrl) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const SimDesc& D = m.d;
-  const int NX = D.g.NX, NY = D.g.NY;
-  if (t < NX) {
-    ring_copy(D, t, 0, rPin, rPout);
-    ring_copy(D, t, NY - 1, rPin, rPout);
-  }
-  if (t < NY) {
-    ring_copy(D, 0, t, rPin, rPout);
-    ring_copy(D, NX - 1, t, rPin, rPout);
-  }
-  const int stride = blockDim.x * gridDim.x;
-  for (int i = t; i < nmd; i += stride) maxdiv[i] = 0u;
-  if (t == 0) ctrl[0] = ctrl[1] = 0;
-}
-
-// Early exit of solveSingleGrid (fluid.go:175-177), one wave per simulation: the first
-// sweep whose max |div| is below 1e-5 ends the solve; if that is not the last sweep,
-// request a re-run of k*+1 sweeps (ctrl[1]) and flag the launch (rerun[0]) for the re-run kernel.
-// Lane l scans sweeps l, l+64, ...; the wave's minimum is the first such sweep.
-template <class M>
-__global__ void k_gs_decide(M m, int nsim, int N, int32_t* rerun) {
+// Every member's early exit, one wave each: the sweeps to re-run to ctrl[1], and whether the re-run
+// launch has any. (A single simulation's re-run launch decides for itself.)
+__global__ void k_gs_decide(ManySims m, int nsim, int N, int32_t* rerun) {
   const int e = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES;
-  const int lane = threadIdx.x & (LANES - 1);
   if (e >= nsim) return;
-  const SimDesc& D = sim_desc(m, e);
-  int first = N;
-  if (D.early_exit)
-    for (int k = lane; k < N; k += LANES)
-      if (__uint_as_float(D.maxdiv[k]) < 1e-5f) {
-        first = k;
-        break;
-      }
-  for (int o = LANES / 2; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, LANES));
-  if (lane == 0) {
-    const int kept = first < N ? first + 1 : N;
-    D.ctrl[1] = kept < N ? kept : 0;
-    if (kept < N) atomicOr(rerun, 1);
+  const SimDesc& D = m.sims[e];
+  const int again = sweeps_to_rerun(D, N);
+  if ((threadIdx.x & (LANES - 1)) == 0) {
+    D.ctrl[1] = again;
+    if (again) atomicOr(rerun, 1);
   }
 }
 
@@ -1156,10 +1161,11 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   // Simulate's fill(p, 0) left to this solve: the initial p is zero and is not read
   const int rPin = c->gs_p_zero ? -1 : (int)B_P;
   c->gs_p_zero = false;
-  hipLaunchKernelGGL(k_gs_prep, dim3(std::max(4, (mr + 255) / 256)), dim3(256), 0, c->stream, m, rPin, (int)B_T3,
-                     c->d_maxdiv, 2 * c->nmax, c->d_ctrl);
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
-  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, rPin);
+  const int rings = (mr + 255) / 256;
+  const GsPrep P{prep_groups(rings), rings, (int)B_T3, c->d_maxdiv, 2 * c->nmax, c->d_ctrl, 1};
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(P.groups + nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr,
+                     &W.d_state->solve, W.tk, rPin, P);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
@@ -1171,17 +1177,12 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   R.damping = c->prm.pressure_damping;
   W.lag = c->prm.handoff_lag >= 1 && c->prm.handoff_lag <= 3 ? c->prm.handoff_lag : 1;
   const bool full = !regular(c->prm, cp);
-  // without the early exit no re-run can be requested: the decision and re-run are skipped
+  // without the early exit no re-run can be requested: it is skipped
   const int runs = c->prm.early_exit ? 2 : 1;
   for (int which = 0; which < runs; which++) {
     R.which = which;
     R.count = &W.d_state->run[which];
-    R.rerun = which ? &W.d_state->rerun : nullptr;
     if ((rc = launch_gs(W.tk, W.blk, W.grid, c->stream, m, R, full))) return rc;
-    if (which == 0 && runs > 1) {
-      hipLaunchKernelGGL(k_gs_decide<OneSim>, dim3(1), dim3(LANES), 0, c->stream, m, 1, N, &W.d_state->rerun);
-      FL_HIP(hipGetLastError());
-    }
   }
   hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
                      tile_sweeps(W.tk), (int)B_T3, false);
@@ -1223,7 +1224,8 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
   d.early_exit = 0;
   OneSim m{d};
   const int nskew = W.G * ((W.rows + 1 + LANES - 1) / LANES);
-  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, &W.d_state->solve, W.tk, -1);
+  hipLaunchKernelGGL(k_gs_skew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr,
+                     &W.d_state->solve, W.tk, -1, GsPrep{});
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = (const int2*)W.d_tile;
@@ -1351,11 +1353,10 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
 int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
   ManySims m{B->d_sims, B->d_cells, B->d_rings};
   const int E = (int)B->members.size();
-  hipLaunchKernelGGL(k_gs_ring<ManySims>, dim3(B->nring_items), dim3(256), 0, B->stream, m, rPin, rPout);
   // per-sweep maxima and re-run requests of all members are contiguous
-  hipLaunchKernelGGL(k_gs_init, dim3(256), dim3(256), 0, B->stream, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E);
-  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(B->nskew), dim3(SKEW_WAVES * LANES), 0, B->stream, m, B->d_skews, &B->state->solve, B->tk,
-                     rPin);
+  const GsPrep P{prep_groups(B->nring_items), B->nring_items, rPout, B->maxdiv_pool, 2 * B->nmax * E, B->ctrl_pool, E};
+  hipLaunchKernelGGL(k_gs_skew<ManySims>, dim3(P.groups + B->nskew), dim3(SKEW_WAVES * LANES), 0, B->stream, m,
+                     B->d_skews, &B->state->solve, B->tk, rPin, P);
   FL_HIP(hipGetLastError());
   GsRun R{};
   R.tiles = B->d_tiles;
@@ -1376,7 +1377,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
     if (rc) return rc;
     if (which == 0 && runs > 1) {
       // one wave per member, four per workgroup
-      hipLaunchKernelGGL(k_gs_decide<ManySims>, dim3((E + 3) / 4), dim3(4 * LANES), 0, B->stream, m, E, N,
+      hipLaunchKernelGGL(k_gs_decide, dim3((E + 3) / 4), dim3(4 * LANES), 0, B->stream, m, E, N,
                          &B->state->rerun);
       FL_HIP(hipGetLastError());
     }
