@@ -203,12 +203,15 @@ static int enqueue_step(Batch* B, float dt) {
   // there in place and the (first) velocity advection writes the step's result into (U, V).
   // Semi-Lagrangian smoke writes M2, which then trades roles with M (no copy).
   int cu = B_U, cv = B_V;
+  bool turb = P.turbulence_strength > 0.0f;
   if (P.pressure_iters > 0) {
-    if ((rc = batch_gs_solve(B, P.pressure_iters, -1, B_P))) return rc;
+    const float t = turb && P.confinement == 0.0f && B->ncells >= TURB_IN_SOLVE_CELLS ? P.turbulence_strength * dt : 0.0f;
+    if (t != 0.0f) turb = false;
+    if ((rc = batch_gs_solve(B, P.pressure_iters, -1, B_P, t))) return rc;
     cu = B_U2;
     cv = B_V2;
   }
-  if ((rc = batch_conf_turb(B, dt, cu, cv))) return rc;
+  if ((rc = batch_conf_turb(B, dt, cu, cv, turb))) return rc;
   if ((rc = batch_borders(B, cu, cv))) return rc;
   // forward (or only) pass: from the current velocity into the other pair of roles
   const int fu = cu == B_U ? B_U2 : B_U, fv = cv == B_V ? B_V2 : B_V;
@@ -552,7 +555,7 @@ int fl_batch_autotune(fl_batch* b, float dt, int* block_sweeps, float* ms) {
         B->prm.handoff_lag = sh.lag;
         return prepare_batch(B, dt);
       },
-      [&]() { return batch_gs_solve(B, N, -1, B_T2); }, &best, &best_ms);
+      [&]() { return batch_gs_solve(B, N, -1, B_T2, 0.0f); }, &best, &best_ms);
   B->prm = saved;
   if (rc) return rc;
   B->prm.block_sweeps = best.tk;

@@ -322,12 +322,16 @@ static int simulate_passes(Ctx* c, float dt) {
   if (!p_by_solve && (rc = launch_fill(c->p, 0.0f, c->N, c->stream))) return rc;         // fill(p,0)
   if (P.viscosity_diffusion > 0 && (rc = launch_viscosity(c, dt))) return rc;          // applyViscosity
   if ((rc = mark(c, 1))) return rc;
+  const bool conf = P.confinement != 0.0f;
+  bool turb = P.turbulence_strength > 0.0f;
   c->gs_p_zero = p_by_solve;
+  c->gs_turb = p_by_solve && turb && !conf && c->N >= TURB_IN_SOLVE_CELLS ? P.turbulence_strength * dt : 0.0f;
+  if (c->gs_turb != 0.0f) turb = false;
   rc = make_incompressible(c, P.pressure_iters, dt, false);                              // makeIncompressible
   c->gs_p_zero = false;
+  c->gs_turb = 0.0f;
   if (rc) return rc;
   if ((rc = mark(c, 2))) return rc;
-  const bool conf = P.confinement != 0.0f, turb = P.turbulence_strength > 0.0f;
   if (conf && (rc = launch_curl(c, c->T0))) return rc;
   if ((conf || turb) && (rc = launch_conf_turb(c, c->T0, dt, conf, turb))) return rc;  // confinement, turbulence
   if ((rc = launch_borders(c))) return rc;                                             // handleBorders

@@ -87,6 +87,18 @@ __device__ __forceinline__ float turb_noise(int k) {
   float seed = (float)k * 0.01f;
   return (float)go_sin((double)seed);
 }
+// applyTurbulence (fluid.go:496-526) of a fluid interior cell; whether it changed. The noise (two
+// float64 sines) is evaluated only where the speed gate lets it in.
+__device__ __forceinline__ bool add_turbulence(float& u, float& v, int i, int j, float turb) {
+  const float localVel = sqrtf(u * u + v * v);
+  if (!(localVel > 0.1f)) return false;
+  const float noiseU = turb_noise(i * 137 + j * 241) * turb;
+  const float noiseV = turb_noise(i * 157 + j * 263) * turb;
+  const float factor = go_minf(localVel * 0.5f, 1.0f);
+  u += noiseU * factor;
+  v += noiseV * factor;
+  return true;
+}
 
 // A field element at a 32-bit cell index from a kernel-uniform base. The byte offset stays a
 // 32-bit unsigned value, so the compiler addresses with the base in scalar registers instead of

@@ -899,11 +899,11 @@ __device__ __forceinline__ void next_solve(GsState* S) {
 
 // The rows of the last sweep's wave (its last sweep b, padded to the wave's S) to U2, V2 and role
 // rPout: row t of row-tile g holds cell (64 g + a - k0 - b, t - a - b) at lane a. An early exit
-// (ctrl[1] sweeps) takes the re-run's. A coarse solve has p alone. Also numbers the next solve and
-// zeroes its counters.
+// (ctrl[1] sweeps) takes the re-run's. A coarse solve has p alone. turb: the turbulence that follows
+// the solve (strength times dt; 0: none). Also numbers the next solve and zeroes its counters.
 template <class M>
 __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const SkewItem* items, GsState* state, int N, int tk, int S,
-                                                   int rPout, bool coarse) {
+                                                   int rPout, bool coarse, float turb) {
   __shared__ float sh[3][LANES][LANES + 1];
   const SimDesc* D;
   int g, t0;
@@ -923,6 +923,12 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const Ske
     sh[1][lane][u] = word_v(v);
     sh[2][lane][u] = word_p(v);
   }
+  uint32_t fluid[SKEW_ROWS] = {};  // the cells that take turbulence, loaded with the words
+#pragma unroll
+  for (int x = 0; x < SKEW_ROWS; x++) {
+    const int r = r0 + SKEW_ROWS * w + x, j = t0 + lane - SKEW_ROWS * w - x - b;
+    if (turb != 0.0f && r >= 1 && r <= NX - 2 && j >= 1 && j <= NY - 2) fluid[x] = D->flags[(size_t)r * NY + j] & CF_FLUID;
+  }
   __syncthreads();
   float* const dst[3] = {D->buf[B_U2], D->buf[B_V2], D->buf[rPout]};
 #pragma unroll
@@ -930,8 +936,10 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const Ske
     const int a = SKEW_ROWS * w + x, r = r0 + a, j = t0 + lane - a - b;
     if (r < 1 || r > NX - 1 || j < 1 || j > NY - 1 || t0 + lane >= rows) continue;
     const size_t c = (size_t)r * NY + j;
-    if (!coarse && j <= NY - 2) dst[0][c] = sh[0][a][lane];
-    if (!coarse && r <= NX - 2) dst[1][c] = sh[1][a][lane];
+    float u = sh[0][a][lane], v = sh[1][a][lane];
+    if (fluid[x]) add_turbulence(u, v, r, j, turb);
+    if (!coarse && j <= NY - 2) dst[0][c] = u;
+    if (!coarse && r <= NX - 2) dst[1][c] = v;
     if (r <= NX - 2 && j <= NY - 2) dst[2][c] = sh[2][a][lane];
   }
 }
@@ -1185,7 +1193,7 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
     if ((rc = launch_gs(W.tk, W.blk, W.grid, c->stream, m, R, full))) return rc;
   }
   hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
-                     tile_sweeps(W.tk), (int)B_T3, false);
+                     tile_sweeps(W.tk), (int)B_T3, false, c->gs_turb);
   FL_HIP(hipGetLastError());
   std::swap(c->U, c->U2);
   std::swap(c->V, c->V2);
@@ -1238,7 +1246,7 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
   hipLaunchKernelGGL(fn, dim3(W.grid), dim3(tile_waves(W.tk) * LANES), 0, c->stream, m, R);
   FL_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_gs_unskew<OneSim>, dim3(nskew), dim3(SKEW_WAVES * LANES), 0, c->stream, m, nullptr, W.d_state, N, W.tk,
-                     tile_sweeps(W.tk), (int)B_T3, true);
+                     tile_sweeps(W.tk), (int)B_T3, true, 0.0f);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -1350,7 +1358,7 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   return FL_OK;
 }
 
-int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
+int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb) {
   ManySims m{B->d_sims, B->d_cells, B->d_rings};
   const int E = (int)B->members.size();
   // per-sweep maxima and re-run requests of all members are contiguous
@@ -1383,7 +1391,7 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout) {
     }
   }
   hipLaunchKernelGGL(k_gs_unskew<ManySims>, dim3(B->nskew), dim3(SKEW_WAVES * LANES), 0, B->stream, m, B->d_skews, B->state, N,
-                     B->tk, tile_sweeps(B->tk), rPout, false);
+                     B->tk, tile_sweeps(B->tk), rPout, false, turb);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }

@@ -145,6 +145,8 @@ struct Ctx {
   // Simulate's fill(p, 0) is left to its temporal-blocked solve, which then starts from p = 0
   // without reading p (set by the step around its solve only)
   bool gs_p_zero = false;
+  // Simulate's turbulence (times dt) is left to the last kernel of its temporal-blocked solve; 0: none
+  float gs_turb = 0.0f;
 
   // Device state: the 8 reference buffers plus ping-pong partners and scratch.
   float *U = nullptr, *V = nullptr, *nU = nullptr, *nV = nullptr, *p = nullptr, *S = nullptr, *M = nullptr,
@@ -359,7 +361,7 @@ int batch_copy_role(Batch* B, int rdst, int rsrc);
 int batch_swap_roles(Batch* B, int a, int b);  // in every member's device descriptor
 int batch_flags(Batch* B);
 int batch_viscosity(Batch* B, float dt);
-int batch_conf_turb(Batch* B, float dt, int rU, int rV);
+int batch_conf_turb(Batch* B, float dt, int rU, int rV, bool turb);
 int batch_borders(Batch* B, int rU, int rV);
 int batch_advect_velocity(Batch* B, int rUt, int rVt, int rUo, int rVo, float dt, bool write_new = true);
 int batch_bfecc_velocity_corr(Batch* B, int rUo, int rVo, int rUf, int rVf, float dt);
@@ -373,7 +375,14 @@ int pick_tk(const fl_params& P, int NX, int NY, int N);
 bool gs_wave_supported(Ctx* c, int numIters);
 int pick_blk(const fl_params& P);
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs);
-int batch_gs_solve(Batch* B, int N, int rPin, int rPout);  // p from rPin (< 0: zero), to rPout
+// Without confinement, turbulence follows the solve cell by cell, and from this many cells the solve's
+// last kernel, which holds both faces of a cell, adds it: a launch and a pass over U and V less.
+// 4096^2 61 us + 104 -> 109, a batch of 18.6 M cells 83 us + 133 -> 148.
+// Smaller grids have too few waves to hide four cells' sines in a row: 256^2 4.6 us + 5.2 -> 8.3,
+// and the jet clip 1691 -> 1708 us.
+static constexpr size_t TURB_IN_SOLVE_CELLS = size_t(1) << 20;
+// p from rPin (< 0: zero), to rPout; then turbulence of strength times dt `turb` (0: none)
+int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb);
 
 // ---- pressure (fl_pressure.hip) -------------------------------------------------------
 // Runs the single-grid projection: sweeps with the reference order on (U,V,p).

@@ -292,20 +292,9 @@ __global__ void k_conf_turb(M m, int rU, int rV, int rcurl, float conf, float dt
     u += strength * gy * vort * dt;
     v -= strength * gx * vort * dt;
   }
-  // the update is in place: a face the passes leave alone is not written back, and the
-  // noise (two float64 sines) is evaluated only where the speed gate lets it in
+  // the update is in place: a face the passes leave alone is not written back
   bool changed = do_conf != 0;
-  if (do_turb) {
-    float localVel = sqrtf(u * u + v * v);
-    if (localVel > 0.1f) {
-      float noiseU = turb_noise(i * 137 + j * 241) * turb;
-      float noiseV = turb_noise(i * 157 + j * 263) * turb;
-      float factor = go_minf(localVel * 0.5f, 1.0f);
-      u += noiseU * factor;
-      v += noiseV * factor;
-      changed = true;
-    }
-  }
+  if (do_turb && add_turbulence(u, v, i, j, turb)) changed = true;
   if (changed) {
     U[c] = u;
     V[c] = v;
@@ -1000,9 +989,9 @@ int batch_viscosity(Batch* B, float dt) {
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
-int batch_conf_turb(Batch* B, float dt, int rU, int rV) {
+int batch_conf_turb(Batch* B, float dt, int rU, int rV, bool turb) {
   const fl_params& P = B->prm;
-  const bool conf = P.confinement != 0.0f, turb = P.turbulence_strength > 0.0f;
+  const bool conf = P.confinement != 0.0f;
   if (conf) hipLaunchKernelGGL(k_curl<ManySims>, FL_BATCH_CELLS(B), many(B), (int)B_T0, rU, rV);
   if (conf || turb)
     hipLaunchKernelGGL(k_conf_turb<ManySims>, FL_BATCH_CELLS(B), many(B), rU, rV, (int)B_T0, P.confinement, dt,

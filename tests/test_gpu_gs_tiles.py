@@ -7,7 +7,7 @@ solve performs the oracle's float32 operations in the oracle's order (NaN compar
 import numpy as np
 import pytest
 
-from fluid_amd import Fluid
+from fluid_amd import Fluid, FluidBatch
 from oracle.pyoracle import OracleFluid
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +61,36 @@ def test_multigrid_coarse_tiles(w, h, solid):
     """Coarse interiors of one cell, one row more or less than a tile, and (the last) more than
     256 tiles of four sweeps in flight, so tiles of eight."""
     run(w, h, 1, 0, 0, solid=solid, steps=2 if w < 1000 else 1, UseMultigrid=True)
+
+
+@pytest.mark.parametrize("w,h,early", [(1022, 1021, False), (1022, 1022, False), (1022, 1022, True), (4094, 255, False),
+                                       (90, 12001, False)])
+def test_turbulence_with_the_solve(w, h, early):
+    """From 2^20 cells the solve's last kernel adds the turbulence; (1022, 1021) is the largest below.
+    early: with a tolerance met after some sweeps the result is the re-run's."""
+    run(w, h, 5, 0, 0, early=early, solid=0.9 if early else 0.05)
+
+
+def test_turbulence_with_a_batch_solve():
+    """Members that alone stay below 2^20 cells, together above; and each on its own."""
+    sizes = [(800, 798), (631, 700), (5, 7)]
+    b = FluidBatch(1000.0, sizes, 0.01)
+    alone = [Fluid(1000.0, w, h, 0.01) for w, h in sizes]
+    for e, (m, f) in enumerate(zip(b.members, alone)):
+        rng = np.random.default_rng(e)
+        shape = (sizes[e][0] + 2, sizes[e][1] + 2)
+        st = {"S": (rng.random(shape) >= 0.05).astype(np.float32)}
+        for k in ("U", "V", "newU", "newV"):
+            st[k] = (0.5 * rng.standard_normal(shape)).astype(np.float32)
+        m.load_state(st)
+        f.load_state(st)
+        f.PressureIters = 9
+    b.PressureIters = 9
+    for step in range(2):
+        b.update(0.1)
+        for f in alone:
+            f.update(0.1)
+        for e, (m, f) in enumerate(zip(b.members, alone)):
+            for k in ("U", "V", "p", "M"):
+                assert np.array_equal(m.get(k).view(np.uint32), f.get(k).view(np.uint32)), (step, e, k)
+    b.close()
