@@ -334,7 +334,8 @@ enum { OUT_LDS, OUT_WORDS };
 // go: lane 63's U, V, p of each sweep after step u, at lane 64 - B + u: every step shifts them down
 // a lane and lets lane 63 in, one instruction a value into the register that the value leaves (a
 // store of lane 63 to LDS took two exec changes and two writes, 44 cycles a step for one sweep).
-template <int SOLVE, int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL>
+// ROW63: without the last sweep's V and p, which the caller takes from the LDS rows.
+template <int SOLVE, int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL, bool ROW63>
 __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST ? B : 1], float (&k)[3],
                                           const uint32_t (&mk)[S], const float* gi, const float4* Kin, float4* Kout,
                                           float (&go)[S][3], const char* tab, __amdgpu_buffer_rsrc_t kbuf,
@@ -377,6 +378,7 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
 #pragma unroll
     for (int c = 0; c < S; c++) {
       if (SOLVE == SOLVE_GS) go[c][0] = from_lane_above(Q.UrO[c], go[c][0]);
+      if (ROW63 && c == S - 1) continue;
       go[c][1] = from_lane_above(Q.VbO[c], go[c][1]);
       go[c][2] = from_lane_above(Q.pO[c], go[c][2]);
     }
@@ -693,6 +695,16 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         }
       };
       float go[S][3];
+      // The last sweep's V and p of lane 63 are in the rows that the wave left in LDS: the last B lanes
+      // read them there after the block, two shifts a step less (256^2 a solve 123 -> 120 us, 512^2 200
+      // sweeps 444 -> 436, 2048x1024 861 -> 842). Not in tiles of 16 sweeps, which lose (4096^2 4.74 ->
+      // 4.79 ms).
+      constexpr bool ROW63 = OUT == OUT_LDS && !NEAR;
+      const float4* krow63[2] = {};
+      if constexpr (ROW63) {
+        krow63[0] = &sh.K[w][0][max(lane - (LANES - B), 0)][LANES - 1];
+        krow63[1] = &sh.K[w][1][max(lane - (LANES - B), 0)][LANES - 1];
+      }
       auto run = [&](const Block& x, int n) __attribute__((always_inline)) {
         const float4* Kin = FIRST ? nullptr : &sh.K[w - 1][n & 1][0][lane];
         float4* Kout = OUT == OUT_WORDS ? nullptr : &sh.K[w][n & 1][0][lane];
@@ -704,7 +716,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
+  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
         if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
         } else if (every_lane(same)) {
@@ -713,6 +725,11 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           FL_RUN(BLOCK_ANY);
         }
 #undef FL_RUN
+        if constexpr (ROW63) {
+          const float4 v = *krow63[n & 1];
+          go[S - 1][1] = v.y;
+          go[S - 1][2] = v.z;
+        }
       };
       for (int p = 0; p < w; p++) __syncthreads();
       // Block n runs while the words of block n + 1 are on their way (the last block's once more
