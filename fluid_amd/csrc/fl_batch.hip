@@ -114,11 +114,7 @@ static int flush_batch_edits(Batch* B) {
   for (size_t e = 0; e < B->members.size(); e++) {
     Ctx* c = B->members[e];
     if (c->edits.empty()) continue;
-    std::vector<uint32_t> order(c->edits.size());
-    for (size_t k = 0; k < order.size(); k++) order[k] = (uint32_t)k;
-    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
-      return (c->edits[a].key & 0x7fffffffu) < (c->edits[b].key & 0x7fffffffu);
-    });
+    const std::vector<uint32_t> order = edit_order(c);
     uint32_t prev = 0xffffffffu;
     for (uint32_t k : order) {
       const WordOp& op = c->edits[k];

@@ -157,14 +157,32 @@ int copy_to_device(Ctx* c, void* dst, const void* src, size_t bytes) {
   return FL_OK;
 }
 
+// Words are field-major, and programs mostly edit a field's cells in ascending order, two fields at a
+// time: so the edits are dealt out to their fields, and only a field that is not in order by then is
+// sorted (a sort of all 230,000 edits of an ensemble's impulses took 5 ms).
+std::vector<uint32_t> edit_order(const Ctx* c) {
+  constexpr int FIELDS = 8;
+  const std::vector<WordOp>& ops = c->edits;
+  auto word = [&](uint32_t k) { return ops[k].key & 0x7fffffffu; };
+  auto field = [&](uint32_t k) { return word(k) / (uint32_t)c->N; };
+  size_t at[FIELDS + 1] = {};
+  for (uint32_t k = 0; k < ops.size(); k++) at[field(k) + 1]++;
+  for (int f = 0; f < FIELDS; f++) at[f + 1] += at[f];
+  std::vector<uint32_t> order(ops.size());
+  size_t to[FIELDS];
+  std::copy(at, at + FIELDS, to);
+  for (uint32_t k = 0; k < ops.size(); k++) order[to[field(k)]++] = k;
+  auto before = [&](uint32_t a, uint32_t b) { return word(a) < word(b); };
+  for (int f = 0; f < FIELDS; f++)
+    if (!std::is_sorted(order.begin() + at[f], order.begin() + at[f + 1], before))
+      std::stable_sort(order.begin() + at[f], order.begin() + at[f + 1], before);
+  return order;
+}
+
 int flush_edits(Ctx* c) {
   if (c->edits.empty()) return FL_OK;
   const size_t n = c->edits.size();
-  std::vector<uint32_t> order(n);
-  std::iota(order.begin(), order.end(), 0u);
-  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
-    return (c->edits[a].key & 0x7fffffffu) < (c->edits[b].key & 0x7fffffffu);
-  });
+  const std::vector<uint32_t> order = edit_order(c);
   std::vector<uint32_t> keys(n);
   std::vector<float> vals(n);
   std::vector<int32_t> seg;

@@ -40,8 +40,8 @@
 // initial state out as K-stream words and k_gs_unskew takes the last sweep's back, so tiles
 // read and write nothing but words, whole lines at a time.
 //
-// What it measured, one sweep a wave with a barrier a step -> now: 256^2 40 sweeps 0.49 -> 0.154 ms,
-// 300x251 8 sweeps 0.42 -> 0.110, 512^2 200 sweeps 1.32 -> 0.473, 4096^2 200 sweeps 10.5 -> 5.04.
+// What a solve measured, one sweep a wave with a barrier a step -> now: 256^2 40 sweeps 0.49 -> 0.136 ms,
+// 300x251 8 sweeps 0.42 -> 0.095, 512^2 200 sweeps 1.32 -> 0.454, 4096^2 200 sweeps 10.5 -> 4.96.
 // At 4096^2 the two waves of a SIMD are bound by their issue: 43 instructions a step of two
 // sweeps, 34 of them the shifts and updates.
 //

@@ -315,6 +315,8 @@ struct CtxErrScope {
 
 // ---- host runtime shared by single contexts and batches (fl_capi.hip) ------------------
 int flush_edits(Ctx* c);
+// The context's queued edits in the order of their target words, those of a word in call order.
+std::vector<uint32_t> edit_order(const Ctx* c);
 // Device-to-host copy on the context's stream that returns when `dst` holds the data.
 int copy_to_host(Ctx* c, void* dst, const void* src, size_t bytes);
 int copy_to_device(Ctx* c, void* dst, const void* src, size_t bytes);
