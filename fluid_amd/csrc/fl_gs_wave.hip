@@ -109,7 +109,8 @@ __device__ __forceinline__ bool tile_empty(int g, int kb, int K, int TK, int NX)
 // while it is being written sees for each half whether it is this solve's; only the 8-byte halves
 // have to arrive whole. Words are written once per solve, so the tag they hold before is that of one of the
 // last solves. Device-coherent accesses (sc1), so that neither side needs a cache writeback or
-// invalidate.
+// invalidate. The intrinsics' offsets are 32 bits and a tile's K rows 1 KB each, so a buffer begins
+// at the rows of a block (or of a layout item), and its offsets stay within those.
 typedef uint32_t word4 __attribute__((ext_vector_type(4)));
 static constexpr int CACHED = 0, SC1 = 16, VOLATILE_OP = (int)0x80000000;  // cache policy of the buffer intrinsics
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t word_buffer(const void* p) {
@@ -565,12 +566,12 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     // The G stream has a column of tiles before the first for the initial state (k_gs_skew), so the
     // corner's words lie a tile before the G stream's.
     const size_t gtile = (size_t)rows * GROW, ktile = (size_t)rows * KROW, itile = (size_t)(rows + 1) * KROW;
-    const __amdgpu_buffer_rsrc_t kmine = word_buffer(D.kout + (size_t)(g * KB + kb) * ktile);
-    const __amdgpu_buffer_rsrc_t gmine = word_buffer(D.gout + (size_t)(g * (KB + 1) + kb + 1) * gtile);
-    const __amdgpu_buffer_rsrc_t gprod = word_buffer(D.gout + (g > 0 ? (size_t)((g - 1) * (KB + 1) + kb) * gtile : 0));
+    uint8_t* const kmine = D.kout + (size_t)(g * KB + kb) * ktile;
+    uint8_t* const gmine = D.gout + (size_t)(g * (KB + 1) + kb + 1) * gtile;
+    const uint8_t* const gprod = D.gout + (g > 0 ? (size_t)((g - 1) * (KB + 1) + kb) * gtile : 0);
     const uint8_t* ksrc = kb ? D.kout + (size_t)(kb - 1) * ktile : D.kinit;  // of row-tile 0
     const size_t kstep = kb ? KB * ktile : itile;                            // to the next row-tile
-    const __amdgpu_buffer_rsrc_t kprod = word_buffer(ksrc + (hK ? g * kstep : 0));
+    const uint8_t* const kprod = ksrc + (hK ? g * kstep : 0);
     const uint32_t ktag = kb ? tag : tag0;
     const int kfirst = kb ? TK - 1 : 0, klast = kb ? rows - 1 : rows;  // row of step 0, last row
 
@@ -601,9 +602,8 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     // last sweep of the corner tile instead. need: all ones in the lanes that wait for a producer.
     const int gu = lane / (S + 1), gx = lane - gu * (S + 1);
     const bool gcorner = w == 0 && gx == 0, gstage = gu < B;
-    const uint32_t gat = gcorner ? 16 * (TK - 1) : (uint32_t)gtile + 16 * (b0 - 1 + gx);
-    const uint32_t goff = gat + (gcorner ? gu + LANES + kfirst : gu + LANES - 1) * GROW;
-    const uint32_t glast = gat + (rows - 1) * GROW;
+    const uint32_t gat = gcorner ? 16 * (TK - 1) : (uint32_t)gtile + 16 * (b0 - 1 + gx);  // (words_fit)
+    const int grow = gcorner ? gu + LANES + kfirst : gu + LANES - 1;  // row of a block's word, from the block's first
     const uint32_t gtag = gcorner ? ktag : tag, gneed = gstage && (gcorner ? hC : hG) ? ~0u : 0u, kneed = hK ? ~0u : 0u;
     lds_float* const gdst = (lds_float*)&sh.Gi[w][min(gu, B - 1) + 1][3 * gx];
     const bool gout = g_wave && lane >= LANES - B;  // stores lane 63's words of step lane - (64 - B)
@@ -632,11 +632,12 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         word4 gw, kw[FIRST ? B : 1];
       };
       auto load_g = [&](Block& x, int n) __attribute__((always_inline)) {
-        x.gw = ld_word(gprod, min(goff + n * (B * GROW), glast));
+        x.gw = ld_word(word_buffer(gprod + (size_t)n * (B * GROW)), gat + (uint32_t)min(grow, rows - 1 - n * B) * GROW);
       };
       auto load_k = [&](Block& x, int n, int u) __attribute__((always_inline)) {
-        x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(kprod, 16 * lane, min(n * B + u + kfirst, klast) * KROW,
-                                                        SC1 | VOLATILE_OP);
+        const int r = min(n * B + kfirst, klast);  // the block's first row, or the last of all
+        x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(word_buffer(kprod + (size_t)r * KROW), 16 * lane,
+                                                        min(u, klast - r) * KROW, SC1 | VOLATILE_OP);
       };
       auto load = [&](Block& x, int n) __attribute__((always_inline)) {
 #pragma unroll
@@ -708,7 +709,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       auto run = [&](const Block& x, int n) __attribute__((always_inline)) {
         const float4* Kin = FIRST ? nullptr : &sh.K[w - 1][n & 1][0][lane];
         float4* Kout = OUT == OUT_WORDS ? nullptr : &sh.K[w][n & 1][0][lane];
-        const uint32_t kbyte = (uint32_t)n * (B * KROW) + 16 * lane;
+        const __amdgpu_buffer_rsrc_t kbuf = word_buffer(kmine + (size_t)n * (B * KROW));
         bool plain = true, same = true;
 #pragma unroll
         for (int c = 0; c < S; c++) {
@@ -716,7 +717,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
+  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kbuf, 16 * lane, tag, damping, cp)
         if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
         } else if (every_lane(same)) {
@@ -742,9 +743,10 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         run(x, n);
         stage(next, n1);
         if (gout) {
+          const __amdgpu_buffer_rsrc_t gbuf = word_buffer(gmine + (size_t)n * (B * GROW));
 #pragma unroll
           for (int c = 0; c < S; c++)
-            st_word<SC1>(gmine, goword + n * (B * GROW) + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
+            st_word<SC1>(gbuf, goword + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
         }
         if (NEAR && OUT == OUT_WORDS && far) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
@@ -891,16 +893,16 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_skew(M m, const SkewI
   }
   __syncthreads();
   const uint32_t tag = 2u * (uint32_t)*solve & 0xffffu;
-  const __amdgpu_buffer_rsrc_t dst = word_buffer(D->kinit + (size_t)g * (D->rows + 1) * (16 * LANES));
+  const __amdgpu_buffer_rsrc_t dst = word_buffer(D->kinit + ((size_t)g * (D->rows + 1) + t0) * (16 * LANES));
   // lane 63's also as the last sweep's of the G stream's first column
-  const __amdgpu_buffer_rsrc_t gdst = word_buffer(D->gout + (size_t)g * (D->KB + 1) * D->rows * (16 * tk));
+  const __amdgpu_buffer_rsrc_t gdst = word_buffer(D->gout + ((size_t)g * (D->KB + 1) * D->rows + t0) * (16 * tk));
 #pragma unroll
   for (int x = 0; x < SKEW_ROWS; x++) {
     const int u = SKEW_ROWS * w + x;
     if (t0 + u <= D->rows)
-      st_word<CACHED>(dst, (uint32_t)(t0 + u) * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
+      st_word<CACHED>(dst, (uint32_t)u * (16 * LANES) + 16 * lane, sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
     if (lane == LANES - 1 && t0 + u < D->rows)
-      st_word<CACHED>(gdst, (uint32_t)(t0 + u) * (16 * tk) + 16 * (tk - 1), sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
+      st_word<CACHED>(gdst, (uint32_t)u * (16 * tk) + 16 * (tk - 1), sh[0][lane][u], sh[1][lane][u], sh[2][lane][u], tag);
   }
 }
 
@@ -931,11 +933,12 @@ __global__ __launch_bounds__(SKEW_WAVES * LANES) void k_gs_unskew(M m, const Ske
   const int kb = (K - 1) / tk, k0 = kb * tk, b = (K - 1 - k0) / S * S + S - 1;
   const int r0 = LANES * g - k0 - b;  // row of lane 0
   if (r0 > NX - 1 || r0 + LANES - 1 < 1) return;
-  const __amdgpu_buffer_rsrc_t src = word_buffer(D->kout + (size_t)(g * D->KB + kb) * rows * (16 * LANES));
+  const int first = min(t0, rows - 1);  // (the item past the last row of words has no cells)
+  const __amdgpu_buffer_rsrc_t src = word_buffer(D->kout + ((size_t)(g * D->KB + kb) * rows + first) * (16 * LANES));
 #pragma unroll
   for (int x = 0; x < SKEW_ROWS; x++) {
     const int u = SKEW_ROWS * w + x;
-    const word4 v = ld_word(src, (uint32_t)min(t0 + u, rows - 1) * (16 * LANES) + 16 * lane);
+    const word4 v = ld_word(src, (uint32_t)min(u, rows - 1 - first) * (16 * LANES) + 16 * lane);
     sh[0][lane][u] = word_u(v);
     sh[1][lane][u] = word_v(v);
     sh[2][lane][u] = word_p(v);
@@ -1006,6 +1009,18 @@ static TileGeom geom(int NX, int NY, int N, int tk, int blk) {
   const int steps = NY + LANES - 1 + tk - 1;
   t.rows = (steps + blk - 1) / blk * blk;
   return t;
+}
+// A wave loads its G words from its producer's tile and the corner tile before it in one instruction,
+// so their offset from a block's row of the corner tile spans one tile of `rows` rows and the 64 + tk +
+// blk rows that a tile lags, and has to stay below 2^32. With one row-tile the words are not used.
+static bool words_fit(const TileGeom& t, int tk) {
+  return t.G == 1 || ((uint64_t)t.rows + 2 * LANES) * (16 * tk) < (uint64_t)1 << 32;
+}
+// The depth to use where tiles of tk sweeps are too long for that (16.7 million columns with 16):
+// shallower ones, whose G rows are smaller.
+static int shallow_enough(int NX, int NY, int N, int tk, int blk) {
+  while (tk > 2 && !words_fit(geom(NX, NY, N, tk, blk), tk)) tk /= 2;
+  return tk;
 }
 // Tiles are handed out in the order their producers let them start: a consumer loads a block
 // ahead, so it runs 64 + 2 BLK columns behind the tile one row-tile up, and TK + 2 BLK plus the
@@ -1082,8 +1097,8 @@ static bool tk_knob(const fl_params& P) {
   return P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16;
 }
 int pick_tk(const fl_params& P, int NX, int NY, int N) {
-  if (tk_knob(P)) return P.block_sweeps;
-  return depth_for([&](int tk) { return tiles_in_flight(NX, NY, N, tk); });
+  const int tk = tk_knob(P) ? P.block_sweeps : depth_for([&](int tk) { return tiles_in_flight(NX, NY, N, tk); });
+  return shallow_enough(NX, NY, N, tk, pick_blk(P));
 }
 // Columns per block: 4 with the knob, else 8, which won at every size (4096^2 200 sweeps 5.0 ms
 // against 7.1, 256^2 0.154 against 0.163). 16, which the knob also takes, would not fit in LDS.
@@ -1275,12 +1290,15 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
 // velocity to U2, V2.
 // A batch's sweeps per tile: as for one grid, by the tiles of all members.
 static int batch_tk(const fl_params& P, const std::vector<SimDesc>& descs, int N) {
-  if (tk_knob(P)) return P.block_sweeps;
-  return depth_for([&](int tk) {
-    long long n = 0;
-    for (const SimDesc& d : descs) n += tiles_in_flight(d.g.NX, d.g.NY, N, tk);
-    return n;
-  });
+  int tk = P.block_sweeps;
+  if (!tk_knob(P))
+    tk = depth_for([&](int tk) {
+      long long n = 0;
+      for (const SimDesc& d : descs) n += tiles_in_flight(d.g.NX, d.g.NY, N, tk);
+      return n;
+    });
+  for (const SimDesc& d : descs) tk = shallow_enough(d.g.NX, d.g.NY, N, tk, pick_blk(P));
+  return tk;
 }
 int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   const int tk = batch_tk(B->prm, descs, N);
