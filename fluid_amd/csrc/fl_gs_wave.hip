@@ -84,7 +84,7 @@ enum { MODE_NEAR = 1, MODE_FAR = 2 };
 
 // One launch of the solve (main run or early-exit re-run).
 struct GsRun {
-  const int2* tiles;  // (simulation, (g << 16) | kb): each queue's tiles in ticket order, then all of them
+  const SolveTile* tiles;  // each queue's tiles in ticket order, then all of them
   const int* first;   // [nq + 2] where each queue's tiles begin, then all tiles, and the end
   int nq;             // 0: all tiles from one queue
   int which;          // 0 main run (K sweeps), 1 re-run (ctrl[1] sweeps of each simulation)
@@ -542,8 +542,8 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const int t = uniform(sh.tile), far = uniform(sh.far);
     __syncthreads();
     if (t < 0) break;
-    const int2 te = R.tiles[t];
-    const int sim = te.x, g = te.y >> 16, kb = te.y & 0xffff;
+    const SolveTile te = R.tiles[t];
+    const int sim = te.sim, g = te.g, kb = te.kb;
     const SimDesc& D = sim_desc(m, sim);
     const int NX = D.g.NX, NY = D.g.NY, rows = D.rows, KB = D.KB;
     const int nblk = rows / B;
@@ -1030,26 +1030,26 @@ static int shallow_enough(int NX, int NY, int N, int tk, int blk) {
 struct GsTile {
   long long key;
   int row;  // of all simulations' row-tiles
-  int2 t;
+  SolveTile t;
 };
 static void append_tiles(std::vector<GsTile>& out, int sim, int row0, int NX, int N, int tk, int blk, const TileGeom& t) {
   for (int g = 0; g < t.G; g++)
     for (int kb = 0; kb < t.KB; kb++)
       if (!tile_empty_h(g, kb, padded(N, tk), tk, NX)) {
         const long long start = (long long)(LANES + 2 * blk) * g + (long long)(tk + (tile_waves(tk) + 1) * blk) * kb;
-        out.push_back({(start << 32) | ((long long)sim << 12) | kb, row0 + g, make_int2(sim, (g << 16) | kb)});
+        out.push_back({(start << 32) | ((long long)sim << 12) | kb, row0 + g, SolveTile{sim, g, kb, 0}});
       }
 }
 // The tiles of nq queues, each in ticket order, then all in ticket order; first[q]: where they begin.
 // Row-tiles go to the queue that has the fewest steps so far, in the order of their first tiles.
 // Returns the tiles of the longest queue.
-static int queue_tiles(std::vector<GsTile>& tiles, const std::vector<int>& row_steps, int nq, std::vector<int2>& out,
+static int queue_tiles(std::vector<GsTile>& tiles, const std::vector<int>& row_steps, int nq, std::vector<SolveTile>& out,
                        std::vector<int>& first) {
   std::sort(tiles.begin(), tiles.end(), [](const GsTile& a, const GsTile& b) { return a.key < b.key; });
   std::vector<long long> load(row_steps.size(), 0), total(nq, 0);
   std::vector<int> queue(row_steps.size(), -1);
   for (const GsTile& t : tiles) load[t.row] += row_steps[t.row];
-  std::vector<std::vector<int2>> lists(nq);
+  std::vector<std::vector<SolveTile>> lists(nq);
   for (const GsTile& t : tiles) {
     int& q = queue[t.row];
     if (q < 0 && nq > 0) {
@@ -1162,14 +1162,14 @@ static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   W.rows = t.rows;
   std::vector<GsTile> order;
   append_tiles(order, 0, 0, NX, N, tk, blk, t);
-  std::vector<int2> tiles;
+  std::vector<SolveTile> tiles;
   std::vector<int> first;
   W.nq = device_queues(c->dev, tk);
   const int longest = queue_tiles(order, std::vector<int>(t.G, t.rows), W.nq, tiles, first);
   W.ntiles = (int)order.size();
   const size_t nt = (size_t)W.G * W.KB;
   const size_t kbytes = 16 * nt * W.rows * LANES, gbytes = 16 * (nt + W.G) * W.rows * tk;
-  FL_HIP(hipMalloc(&W.d_tile, sizeof(int2) * std::max<size_t>(1, tiles.size())));
+  FL_HIP(hipMalloc(&W.d_tile, sizeof(SolveTile) * std::max<size_t>(1, tiles.size())));
   FL_HIP(hipMalloc(&W.d_first, sizeof(int) * first.size()));
   FL_HIP(hipMalloc(&W.d_kout, kbytes));
   FL_HIP(hipMalloc(&W.d_gout, gbytes));
@@ -1181,7 +1181,7 @@ static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   GsState state{};
   state.solve = 1;
   FL_HIP(hipMemcpy(W.d_state, &state, sizeof(state), hipMemcpyHostToDevice));
-  FL_HIP(hipMemcpy(W.d_tile, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(W.d_tile, tiles.data(), sizeof(SolveTile) * tiles.size(), hipMemcpyHostToDevice));
   FL_HIP(hipMemcpy(W.d_first, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice));
   W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, std::max(W.ntiles, W.nq * longest));
   return FL_OK;
@@ -1208,7 +1208,7 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
                      &W.d_state->solve, W.tk, rPin, P);
   FL_HIP(hipGetLastError());
   GsRun R{};
-  R.tiles = (const int2*)W.d_tile;
+  R.tiles = W.d_tile;
   R.first = W.d_first;
   R.nq = W.nq;
   R.K = N;
@@ -1268,7 +1268,7 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
                      &W.d_state->solve, W.tk, -1, GsPrep{});
   FL_HIP(hipGetLastError());
   GsRun R{};
-  R.tiles = (const int2*)W.d_tile;
+  R.tiles = W.d_tile;
   R.first = W.d_first;
   R.nq = W.nq;
   R.K = N;
@@ -1348,12 +1348,12 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
     for (int g = 0; g < tg[e].G; g++)
       for (int t0 = 0; t0 <= tg[e].rows; t0 += LANES) skews.push_back(SkewItem{(int)e, g, t0, 0});
   }
-  std::vector<int2> tiles;
+  std::vector<SolveTile> tiles;
   std::vector<int> first;
   B->nq = device_queues(B->dev, tk);
   const int longest = queue_tiles(order, row_steps, B->nq, tiles, first);
   B->ntiles = (int)order.size();
-  FL_HIP(hipMalloc(&B->d_tiles, sizeof(int2) * std::max<size_t>(1, tiles.size())));
+  FL_HIP(hipMalloc(&B->d_tiles, sizeof(SolveTile) * std::max<size_t>(1, tiles.size())));
   FL_HIP(hipMalloc(&B->d_first, sizeof(int) * first.size()));
   FL_HIP(hipMalloc(&B->kout, std::max<size_t>(kbytes, 16)));
   FL_HIP(hipMalloc(&B->gout, std::max<size_t>(gbytes, 16)));
@@ -1368,7 +1368,7 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   GsState state{};
   state.solve = 1;
   FL_HIP(hipMemcpy(B->state, &state, sizeof(state), hipMemcpyHostToDevice));
-  FL_HIP(hipMemcpy(B->d_tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
+  FL_HIP(hipMemcpy(B->d_tiles, tiles.data(), sizeof(SolveTile) * tiles.size(), hipMemcpyHostToDevice));
   FL_HIP(hipMemcpy(B->d_first, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice));
   size_t ko = 0, go = 0, io = 0;
   B->gs_fields.assign(descs.size(), SimDesc{});

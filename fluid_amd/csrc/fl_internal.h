@@ -110,6 +110,10 @@ struct ManySims {
   const RingItem* rings;
 };
 
+// Row-tile g, sweep block kb of one simulation.
+struct SolveTile {
+  int sim, g, kb, pad;
+};
 // Pressure workspace of the temporal-blocked Gauss-Seidel kernel.
 struct GsState;  // counters of a solve's launches, on the device (fl_gs_wave.hip)
 struct GsWork {
@@ -122,7 +126,7 @@ struct GsWork {
   int nq = 0;              // queues they are handed out from
   int grid = 0;            // persistent workgroups launched
   int lag = 0;             // handoff_lag of the last solve (0: none yet)
-  int32_t* d_tile = nullptr;    // [2 ntiles] packed (g << 16 | kb), in ticket order by queue and of all
+  SolveTile* d_tile = nullptr;    // [2 ntiles] in ticket order by queue and of all
   uint8_t* d_kout = nullptr;    // [G*KB][rows][64] K-stream handoff words
   uint8_t* d_gout = nullptr;    // [G*KB][rows][tk] G-stream handoff words
   uint8_t* d_kinit = nullptr;   // [G][rows + 1][64] the initial state as K-stream words
@@ -270,7 +274,7 @@ struct Batch {
   int tk = 0, blk = 0, gs_n = -1;
   int ntiles = 0, grid = 0;
   std::vector<SimDesc> gs_fields;  // per member: G, KB, rows and its handoff slices
-  int2* d_tiles = nullptr;
+  SolveTile* d_tiles = nullptr;
   int* d_first = nullptr;
   int nq = 0;
   uint8_t* kout = nullptr;
