@@ -1147,16 +1147,13 @@ static int launch_gs(int tk, int blk, int grid, hipStream_t stream, const M& m, 
 static void free_work(GsWork& W) {
   for (void* p : {(void*)W.d_tile, (void*)W.d_first, (void*)W.d_state, (void*)W.d_kout, (void*)W.d_gout, (void*)W.d_kinit})
     if (p) (void)hipFree(p);
+  (void)hipGetLastError();  // of a failed allocation: the next launch's check is not to report it
   W = GsWork{};
 }
-static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
-  if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
-  FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
-  free_work(W);
+static int plan(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   const TileGeom t = geom(NX, NY, N, tk, blk);
   W.tk = tk;
   W.blk = blk;
-  W.n_alloc = N;
   W.G = t.G;
   W.KB = t.KB;
   W.rows = t.rows;
@@ -1186,10 +1183,21 @@ static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, std::max(W.ntiles, W.nq * longest));
   return FL_OK;
 }
+static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
+  if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
+  FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
+  free_work(W);
+  if (int rc = plan(W, c, NX, NY, N, tk, blk)) {
+    free_work(W);  // a layout is whole or none: the next solve plans again
+    return rc;
+  }
+  W.n_alloc = N;
+  return FL_OK;
+}
 
 bool gs_wave_supported(Ctx* c, int numIters) { return numIters >= 1 && c->NX >= 3 && c->NY >= 3; }
 
-int gs_wave_solve(Ctx* c, int N, float cp) {
+static int enqueue_solve(Ctx* c, int N, float cp) {
   GsWork& W = c->gs;
   int rc = layout(W, c, c->NX, c->NY, N, pick_tk(c->prm, c->NX, c->NY, N), pick_blk(c->prm));
   if (rc) return rc;
@@ -1233,6 +1241,13 @@ int gs_wave_solve(Ctx* c, int N, float cp) {
   c->host_sweeps = -1;
   return FL_OK;
 }
+// A solve's last kernel resets the counters for the next, so one that was not enqueued whole leaves
+// a layout that must not be used again.
+int gs_wave_solve(Ctx* c, int N, float cp) {
+  const int rc = enqueue_solve(c, N, cp);
+  if (rc) c->gs.n_alloc = -1;
+  return rc;
+}
 
 int pressure_free(Ctx* c) {
   free_work(c->gs);
@@ -1243,7 +1258,7 @@ int pressure_free(Ctx* c) {
 // solveCoarseGrid's sweeps (fluid.go:686-716) from p = 0 by the same tiles. It
 // replaces one launch per diagonal of 32 x 64 tiles and sweep, 89 launches of 24 us at 257^2:
 // 2.16 ms -> 0.16.
-int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks) {
+static int enqueue_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks) {
   GsWork& W = c->mg_gs;
   const int blk = 8;
   int rc = layout(W, c, cNX, cNY, N, std::min(8, pick_tk(fl_params{}, cNX, cNY, N)), blk);
@@ -1282,6 +1297,11 @@ int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p,
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
+int gs_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks) {
+  const int rc = enqueue_coarse_solve(c, cNX, cNY, N, rhs, p, masks);
+  if (rc) c->mg_gs.n_alloc = -1;
+  return rc;
+}
 
 // ---- batched solve ------------------------------------------------------------------------
 // All members' tiles in one ticket list, merged by hyperplane start; one persistent launch
@@ -1300,38 +1320,20 @@ static int batch_tk(const fl_params& P, const std::vector<SimDesc>& descs, int N
   for (const SimDesc& d : descs) tk = shallow_enough(d.g.NX, d.g.NY, N, tk, pick_blk(P));
   return tk;
 }
-int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
-  const int tk = batch_tk(B->prm, descs, N);
-  const int blk = pick_blk(B->prm);
-  auto fill = [&]() {
-    for (size_t e = 0; e < descs.size(); e++) {
-      const SimDesc& f = B->gs_fields[e];
-      SimDesc& d = descs[e];
-      d.G = f.G;
-      d.KB = f.KB;
-      d.rows = f.rows;
-      d.kout = f.kout;
-      d.gout = f.gout;
-      d.kinit = f.kinit;
-    }
-  };
-  if (B->gs_n == N && B->tk == tk && B->blk == blk && B->gs_fields.size() == descs.size()) {
-    fill();
-    return FL_OK;
-  }
-  FL_HIP(hipStreamSynchronize(B->stream));  // earlier solves may still use the old layout
-  if (B->d_tiles) (void)hipFree(B->d_tiles);
-  if (B->kout) (void)hipFree(B->kout);
-  if (B->gout) (void)hipFree(B->gout);
-  if (B->kinit) (void)hipFree(B->kinit);
-  if (B->d_skews) (void)hipFree(B->d_skews);
-  if (B->d_first) (void)hipFree(B->d_first);
-  if (B->state) (void)hipFree(B->state);
+static void batch_free_layout(Batch* B) {
+  for (void* p : {(void*)B->d_tiles, (void*)B->d_first, (void*)B->kout, (void*)B->gout, (void*)B->kinit, (void*)B->d_skews,
+                  (void*)B->state})
+    if (p) (void)hipFree(p);
+  (void)hipGetLastError();  // as in free_work
   B->d_tiles = nullptr;
+  B->d_first = nullptr;
   B->kout = B->gout = B->kinit = nullptr;
   B->d_skews = nullptr;
-  B->d_first = nullptr;
   B->state = nullptr;
+  B->gs_fields.clear();
+  B->gs_n = -1;
+}
+static int batch_plan(Batch* B, int N, int tk, int blk, const std::vector<SimDesc>& descs) {
   std::vector<GsTile> order;
   std::vector<int> row_steps;
   size_t kbytes = 0, gbytes = 0, ibytes = 0;
@@ -1387,13 +1389,40 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   }
   B->tk = tk;
   B->blk = blk;
-  B->gs_n = N;
   B->grid = occupancy_grid<ManySims>(B->dev, tk, blk, std::max(B->ntiles, B->nq * longest));
+  return FL_OK;
+}
+int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
+  const int tk = batch_tk(B->prm, descs, N);
+  const int blk = pick_blk(B->prm);
+  auto fill = [&]() {
+    for (size_t e = 0; e < descs.size(); e++) {
+      const SimDesc& f = B->gs_fields[e];
+      SimDesc& d = descs[e];
+      d.G = f.G;
+      d.KB = f.KB;
+      d.rows = f.rows;
+      d.kout = f.kout;
+      d.gout = f.gout;
+      d.kinit = f.kinit;
+    }
+  };
+  if (B->gs_n == N && B->tk == tk && B->blk == blk && B->gs_fields.size() == descs.size()) {
+    fill();
+    return FL_OK;
+  }
+  FL_HIP(hipStreamSynchronize(B->stream));  // earlier solves may still use the old layout
+  batch_free_layout(B);
+  if (int rc = batch_plan(B, N, tk, blk, descs)) {
+    batch_free_layout(B);
+    return rc;
+  }
+  B->gs_n = N;
   fill();
   return FL_OK;
 }
 
-int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb) {
+static int enqueue_batch_solve(Batch* B, int N, int rPin, int rPout, float turb) {
   ManySims m{B->d_sims, B->d_cells, B->d_rings};
   const int E = (int)B->members.size();
   // per-sweep maxima and re-run requests of all members are contiguous
@@ -1429,6 +1458,11 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb) {
                      B->tk, tile_sweeps(B->tk), rPout, false, turb);
   FL_HIP(hipGetLastError());
   return FL_OK;
+}
+int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb) {
+  const int rc = enqueue_batch_solve(B, N, rPin, rPout, turb);
+  if (rc) B->gs_n = -1;
+  return rc;
 }
 
 }  // namespace fl
