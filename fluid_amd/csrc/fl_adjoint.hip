@@ -74,7 +74,8 @@ struct Vjp {
   double* d_loss = nullptr;
   float dt = 0.0f;
   bool have_forward = false;
-  int mir_K = -1;
+  int mir_K = -1, mir_N = -1;  // what its relaxation table holds (mirror_omega)
+  float mir_relax = 0.0f;
   std::vector<int> sweeps;
 };
 
@@ -829,15 +830,20 @@ static int vjp_step(Vjp* J, float dt, float* tp, int* kept) {
   return FL_OK;
 }
 
-// Relaxation of the mirror run: sweep k' of the transposed solve is forward sweep K-1-k'.
+// Relaxation of the mirror run: sweep k' of the transposed solve is forward sweep K-1-k'. The table
+// is of K kept sweeps of Nf at a relaxation, all of which a program may change between passes.
 static int mirror_omega(Vjp* J, int K) {
-  if (J->mir_K == K) return FL_OK;
   Ctx* m = J->mir;
   const fl_params& P = J->c->prm;
   const int Nf = P.pressure_iters;
+  if (J->mir_K == K && J->mir_N == Nf && J->mir_relax == P.relaxation) return FL_OK;
+  J->mir_K = -1;
   if (m->nmax < K) {
     if (m->d_omega) FL_HIP(hipFree(m->d_omega));
     if (m->d_maxdiv) FL_HIP(hipFree(m->d_maxdiv));
+    m->d_omega = nullptr;
+    m->d_maxdiv = nullptr;
+    m->nmax = 0;
     const int cap = std::max(K, 64);
     FL_HIP(hipMalloc(&m->d_omega, sizeof(float) * cap));
     FL_HIP(hipMalloc(&m->d_maxdiv, sizeof(uint32_t) * 2 * cap));
@@ -853,6 +859,8 @@ static int mirror_omega(Vjp* J, int K) {
   FL_HIP(hipMemcpy(m->d_omega, om.data(), sizeof(float) * K, hipMemcpyHostToDevice));
   m->omega_n = -1;  // the table is not the forward schedule
   J->mir_K = K;
+  J->mir_N = Nf;
+  J->mir_relax = P.relaxation;
   return FL_OK;
 }
 

@@ -195,3 +195,35 @@ def test_gradient_through_multigrid_exit_matches_oracle():
     G, G32 = np.stack([gu, gv]), np.stack([u32, v32])
     assert np.abs(G32).max() > 0
     assert rel(G, G32) < 1e-4, rel(G, G32)
+
+
+@pytest.mark.parametrize("change", ["relaxation", "sweeps"])
+def test_gradient_follows_changed_knobs(change):
+    """The transposed solve's relaxation follows the knobs from one pass of a live rollout to the
+    next: a changed Relaxation, and a changed PressureIters where the early exit keeps as many
+    sweeps as before (5, of a jet of 1e-5). Against the oracle's rollout with the same knobs."""
+    w, h = 40, 32
+    u = 1.0 if change == "relaxation" else 1e-5
+    g, o = (C.jet_scene(lambda *a: cls(*a), w, h, 24, jet_u=u, jet_rows=8) for cls in (Fluid, OracleFluid))
+    for f in (g, o):
+        f.UseBFECC, f.TurbulenceStrength, f.EarlyExit = True, 0.0, change == "sweeps"
+    z = np.zeros((g.NumX, g.NumY), np.float32)
+    T = C.gaussian_blobs(g.NumX, g.NumY, sigma=4.0)
+    start = o.state()
+    r = Rollout(g, 1 if change == "sweeps" else 3, checkpoint_every=2)
+    for k in range(3):
+        if k:
+            for f in (g, o):
+                if change == "relaxation":
+                    f.Relaxation = (1.9, 1.4, -0.5)[k]
+                else:
+                    f.PressureIters = (24, 40, 30)[k]
+        loss = r.forward(C.DT, z, z, T)
+        G = np.stack(r.backward())
+        o.load_state(start)
+        l32, u32, v32 = o.rollout(r.steps, C.DT, z, z, T)
+        if change == "sweeps":
+            assert o.last_sweeps() == 5
+        assert abs(loss - l32) <= 1e-9 * abs(l32)
+        assert rel(G, np.stack([u32, v32])) < 1e-4, k
+    r.close()
