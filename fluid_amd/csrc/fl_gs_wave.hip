@@ -87,6 +87,7 @@ struct GsRun {
   const SolveTile* tiles;  // each queue's tiles in ticket order, then all of them
   const int* first;   // [nq + 2] where each queue's tiles begin, then all tiles, and the end
   int nq;             // 0: all tiles from one queue
+  int mode;           // 0, or MODE_FAR asked for by a test
   int which;          // 0 main run (K sweeps), 1 re-run (ctrl[1] sweeps of each simulation)
   int K;
   GsCounters* count;
@@ -477,6 +478,7 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
 // else, or kept from this stream) the launch takes all tiles from one queue instead and writes
 // its L2 back after every block, slowly.
 static __device__ int queue_of_tiles(const GsRun& R) {
+  if (R.mode == MODE_FAR) return R.nq;
   const int q = __builtin_amdgcn_s_getreg(20 | (3 << 11)) % R.nq;  // HW_REG_XCC_ID, 4 bits
   GsCounters* C = R.count;
   int seen = atomicOr(&C->here, 1 << q) | 1 << q;
@@ -1219,6 +1221,7 @@ static int enqueue_solve(Ctx* c, int N, float cp) {
   R.tiles = W.d_tile;
   R.first = W.d_first;
   R.nq = W.nq;
+  R.mode = c->gs_far ? MODE_FAR : 0;
   R.K = N;
   R.solve = &W.d_state->solve;
   R.omega = c->d_omega;
@@ -1434,6 +1437,7 @@ static int enqueue_batch_solve(Batch* B, int N, int rPin, int rPout, float turb)
   R.tiles = B->d_tiles;
   R.first = B->d_first;
   R.nq = B->nq;
+  R.mode = B->gs_far ? MODE_FAR : 0;
   R.K = N;
   R.solve = &B->state->solve;
   R.omega = B->d_omega;
@@ -1466,3 +1470,29 @@ int batch_gs_solve(Batch* B, int N, int rPin, int rPout, float turb) {
 }
 
 }  // namespace fl
+
+// For the tests, and in no header: puts a solve into states that a program reaches by chance or after
+// hours. far: the launches of 16-sweep tiles take MODE_FAR, as if an XCD had not started; number (if
+// positive): the number of the next solve (the tags repeat after 32768), of an existing layout.
+using namespace fl;
+static int set_solve_number(hipStream_t stream, GsState* state, int number) {
+  if (number <= 0) return FL_OK;
+  if (!state) {
+    set_error("no solve has run");
+    return FL_ERR_INVALID_ARG;
+  }
+  FL_HIP(hipStreamSynchronize(stream));
+  FL_HIP(hipMemcpy(&state->solve, &number, sizeof(number), hipMemcpyHostToDevice));
+  return FL_OK;
+}
+extern "C" int fl_test_solve(fl_ctx* ctx, int far, int number) {
+  Ctx* c = reinterpret_cast<Ctx*>(ctx);
+  c->gs_far = far != 0;
+  return set_solve_number(c->stream, c->gs.d_state, number);
+}
+extern "C" int fl_test_batch_solve(fl_batch* b, int far, int number) {
+  Batch* B = reinterpret_cast<Batch*>(b);
+  B->gs_far = far != 0;
+  B->graph_gen++;
+  return set_solve_number(B->stream, B->state, number);
+}

@@ -151,6 +151,7 @@ struct Ctx {
   bool gs_p_zero = false;
   // Simulate's turbulence (times dt) is left to the last kernel of its temporal-blocked solve; 0: none
   float gs_turb = 0.0f;
+  bool gs_far = false;  // fl_test_solve
 
   // Device state: the 8 reference buffers plus ping-pong partners and scratch.
   float *U = nullptr, *V = nullptr, *nU = nullptr, *nV = nullptr, *p = nullptr, *S = nullptr, *M = nullptr,
@@ -283,6 +284,7 @@ struct Batch {
   SkewItem* d_skews = nullptr;
   int nskew = 0;
   GsState* state = nullptr;
+  bool gs_far = false;  // fl_test_batch_solve
   float* d_omega = nullptr;
   int omega_n = -1;
   float omega_relax = 0.0f;
