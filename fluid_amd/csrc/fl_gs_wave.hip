@@ -324,8 +324,9 @@ template <int S> __device__ __forceinline__ void coarse_any(CoarseCells<S>& x, c
 // How a block's cells are updated: all plain; with weights looked up once (along a wall, say: every
 // lane's cells of a sweep have the same mask); or with weights looked up per cell.
 enum { BLOCK_PLAIN, BLOCK_SAME, BLOCK_ANY };
-// Where a wave's rows go: to the next wave's LDS rows, or to memory as handoff words.
-enum { OUT_LDS, OUT_WORDS };
+// Where a wave's rows go: to the next wave's LDS rows, or to memory as handoff words, written through
+// to where every XCD reads them or (OUT_CACHED) left in this XCD's L2.
+enum { OUT_LDS, OUT_WORDS, OUT_CACHED };
 
 // One block of B steps of a wave. gi, Kin: this block's boundary rows in LDS (Kin, Kout at this
 // lane); k: the first step's K row; mk: the masks. A FIRST wave's rows are the words kw instead,
@@ -337,7 +338,7 @@ enum { OUT_LDS, OUT_WORDS };
 // a lane and lets lane 63 in, one instruction a value into the register that the value leaves (a
 // store of lane 63 to LDS took two exec changes and two writes, 44 cycles a step for one sweep).
 // ROW63: without the last sweep's V and p, which the caller takes from the LDS rows.
-template <int SOLVE, int S, int B, int GP, int MODE, bool FIRST, int OUT, int POLICY, bool FULL, bool ROW63>
+template <int SOLVE, int S, int B, int GP, int MODE, bool FIRST, int OUT, bool FULL, bool ROW63>
 __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST ? B : 1], float (&k)[3],
                                           const uint32_t (&mk)[S], const float* gi, const float4* Kin, float4* Kout,
                                           float (&go)[S][3], const char* tab, __amdgpu_buffer_rsrc_t kbuf,
@@ -376,7 +377,7 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
     if constexpr (OUT == OUT_LDS)
       Kout[u * LANES] = make_float4(ul, Q.VbO[S - 1], Q.pO[S - 1], 0.0f);
     else
-      st_word<POLICY>(kbuf, kbyte + u * (LANES * 16), ul, Q.VbO[S - 1], Q.pO[S - 1], tag);
+      st_word<OUT == OUT_CACHED ? CACHED : SC1>(kbuf, kbyte + u * (LANES * 16), ul, Q.VbO[S - 1], Q.pO[S - 1], tag);
 #pragma unroll
     for (int c = 0; c < S; c++) {
       if (SOLVE == SOLVE_GS) go[c][0] = from_lane_above(Q.UrO[c], go[c][0]);
@@ -470,13 +471,15 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
 
 // The queue a workgroup takes its tiles from (called by one thread of it). A row-tile's tiles are
 // all in the queue of one XCD, so that their K streams, one 1 KB row a step each, stay in that XCD's
-// L2 (written through to memory, the 4096^2 solve took 5.81 ms
-// against 5.04, 2048^2 1.99 against 1.72). Only for tiles of 16 sweeps, which make
-// more rows than XCDs: on small grids whole rows divide unevenly (512^2 0.530 ms against 0.475): a workgroup serves the XCD that it runs on. Each queue needs a workgroup, or tiles
-// would wait for ever for those of a queue without one, so the first workgroups wait until one has
-// started on every XCD (a few microseconds). If that fails (an XCD that is busy with something
-// else, or kept from this stream) the launch takes all tiles from one queue instead and writes
-// its L2 back after every block, slowly.
+// L2 (OUT_CACHED; written through to memory the 4096^2 solve of 200 sweeps takes 5.70 ms against 4.98,
+// 2048^2 1.96 against 1.71). Only for tiles of 16 sweeps, which make more rows than XCDs: on small
+// grids whole rows divide unevenly (512^2 0.530 ms against 0.475). A workgroup serves the XCD that it
+// runs on. Each queue needs a workgroup, or tiles would wait for ever for those of a queue without
+// one, so the first workgroups wait until one has started on every XCD (a few microseconds). If that
+// fails (an XCD that is busy with something else, or kept from this stream) the launch takes all
+// tiles from one queue instead and writes its K streams through. Solves on two streams at once do
+// so now and then: two of 4096^2 4.7 ms a step each, of 2048^2 1.42 (with the L2 written back after
+// every block instead 6.2 and 1.43, and 22 ms a step where a solve alone took that way).
 static __device__ int queue_of_tiles(const GsRun& R) {
   if (R.mode == MODE_FAR) return R.nq;
   const int q = __builtin_amdgcn_s_getreg(20 | (3 << 11)) % R.nq;  // HW_REG_XCC_ID, 4 bits
@@ -672,7 +675,6 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         // that reload whole blocks would take the bandwidth their producers need.
         if (!arrived()) {
           for (int it = 0; !expired(it); it++) {
-            if (NEAR && far) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             load_g(x, n);
             if constexpr (FIRST) {
               load_k(x, n, B - 1);
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       }
       auto run = [&](const Block& x, int n) __attribute__((always_inline)) {
         const float4* Kin = FIRST ? nullptr : &sh.K[w - 1][n & 1][0][lane];
-        float4* Kout = OUT == OUT_WORDS ? nullptr : &sh.K[w][n & 1][0][lane];
+        float4* Kout = OUT != OUT_LDS ? nullptr : &sh.K[w][n & 1][0][lane];
         const __amdgpu_buffer_rsrc_t kbuf = word_buffer(kmine + (size_t)n * (B * KROW));
         bool plain = true, same = true;
 #pragma unroll
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, NEAR ? CACHED : SC1, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kbuf, 16 * lane, tag, damping, cp)
+  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kbuf, 16 * lane, tag, damping, cp)
         if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
         } else if (every_lane(same)) {
@@ -750,7 +752,6 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           for (int c = 0; c < S; c++)
             st_word<SC1>(gbuf, goword + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
         }
-        if (NEAR && OUT == OUT_WORDS && far) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
       };
       Block x, y;
@@ -773,16 +774,23 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     using later_t = std::false_type;
     using lds_t = std::integral_constant<int, OUT_LDS>;
     using words_t = std::integral_constant<int, OUT_WORDS>;
+    using cached_t = std::integral_constant<int, OUT_CACHED>;
+    auto run_words = [&](auto first_c) __attribute__((always_inline)) {
+      if constexpr (NEAR) {
+        if (!far) return run_wave(first_c, cached_t{});
+      }
+      run_wave(first_c, words_t{});
+    };
     if (!wave_on) {
       for (int p = 0; p < nblk + W; p++) __syncthreads();
     } else if (w == 0) {
       if (words)
-        run_wave(first_t{}, words_t{});
+        run_words(first_t{});
       else if constexpr (W > 1)
         run_wave(first_t{}, lds_t{});
     } else if constexpr (W > 1) {
       if (words)
-        run_wave(later_t{}, words_t{});
+        run_words(later_t{});
       else
         run_wave(later_t{}, lds_t{});
     }
