@@ -1193,23 +1193,30 @@ static int plan(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
   W.grid = occupancy_grid<OneSim>(c->dev, tk, blk, std::max(W.ntiles, W.nq * longest));
   return FL_OK;
 }
-static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int blk) {
-  if (W.n_alloc == N && W.tk == tk && W.blk == blk) return FL_OK;
+// The layout for N sweeps in tiles of tk, or of up to `deepest` if the words of those do not fit the
+// device: deeper tiles hand over less (a column of 40 sweeps takes 12 KB a row-tile in tiles of 4, 7 of
+// 8, 5 of 16).
+static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int deepest, int blk) {
+  if (W.n_alloc == N && W.asked == tk && W.blk == blk) return FL_OK;
   FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
-  free_work(W);
-  if (int rc = plan(W, c, NX, NY, N, tk, blk)) {
-    free_work(W);  // a layout is whole or none: the next solve plans again
-    return rc;
+  int rc = FL_OK;
+  for (int t = tk; t == tk || (t <= deepest && words_fit(geom(NX, NY, N, t, blk), t)); t *= 2) {
+    free_work(W);
+    if ((rc = plan(W, c, NX, NY, N, t, blk)) == FL_OK) {
+      W.n_alloc = N;
+      W.asked = tk;
+      return FL_OK;
+    }
   }
-  W.n_alloc = N;
-  return FL_OK;
+  free_work(W);  // a layout is whole or none: the next solve plans again
+  return rc;
 }
 
 bool gs_wave_supported(Ctx* c, int numIters) { return numIters >= 1 && c->NX >= 3 && c->NY >= 3; }
 
 static int enqueue_solve(Ctx* c, int N, float cp) {
   GsWork& W = c->gs;
-  int rc = layout(W, c, c->NX, c->NY, N, pick_tk(c->prm, c->NX, c->NY, N), pick_blk(c->prm));
+  int rc = layout(W, c, c->NX, c->NY, N, pick_tk(c->prm, c->NX, c->NY, N), tk_knob(c->prm) ? 0 : 16, pick_blk(c->prm));
   if (rc) return rc;
   if (c->flags_dirty && (rc = launch_flags(c))) return rc;
   SimDesc d = c->desc();
@@ -1272,7 +1279,7 @@ int pressure_free(Ctx* c) {
 static int enqueue_coarse_solve(Ctx* c, int cNX, int cNY, int N, const float* rhs, float* p, uint8_t* masks) {
   GsWork& W = c->mg_gs;
   const int blk = 8;
-  int rc = layout(W, c, cNX, cNY, N, std::min(8, pick_tk(fl_params{}, cNX, cNY, N)), blk);
+  int rc = layout(W, c, cNX, cNY, N, std::min(8, pick_tk(fl_params{}, cNX, cNY, N)), 8, blk);
   if (rc) return rc;
   SimDesc d = c->desc();
   d.g.NX = cNX;
@@ -1418,19 +1425,28 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
       d.kinit = f.kinit;
     }
   };
-  if (B->gs_n == N && B->tk == tk && B->blk == blk && B->gs_fields.size() == descs.size()) {
+  if (B->gs_n == N && B->asked == tk && B->blk == blk && B->gs_fields.size() == descs.size()) {
     fill();
     return FL_OK;
   }
   FL_HIP(hipStreamSynchronize(B->stream));  // earlier solves may still use the old layout
-  batch_free_layout(B);
-  if (int rc = batch_plan(B, N, tk, blk, descs)) {
+  int rc = FL_OK;
+  auto fits = [&](int t) {
+    for (const SimDesc& d : descs)
+      if (!words_fit(geom(d.g.NX, d.g.NY, N, t, blk), t)) return false;
+    return true;
+  };
+  for (int t = tk; t == tk || (t <= (tk_knob(B->prm) ? 0 : 16) && fits(t)); t *= 2) {  // as in layout()
     batch_free_layout(B);
-    return rc;
+    if ((rc = batch_plan(B, N, t, blk, descs)) == FL_OK) {
+      B->gs_n = N;
+      B->asked = tk;
+      fill();
+      return FL_OK;
+    }
   }
-  B->gs_n = N;
-  fill();
-  return FL_OK;
+  batch_free_layout(B);
+  return rc;
 }
 
 static int enqueue_batch_solve(Batch* B, int N, int rPin, int rPout, float turb) {

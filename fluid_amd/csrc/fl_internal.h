@@ -118,6 +118,7 @@ struct SolveTile {
 struct GsState;  // counters of a solve's launches, on the device (fl_gs_wave.hip)
 struct GsWork {
   int tk = 0;              // sweeps per tile
+  int asked = 0;           // sweeps per tile asked for (tiles are deeper where those did not fit)
   int blk = 0;             // columns per block
   int n_alloc = -1;        // sweep count the layout was built for
   int G = 0, KB = 0;       // tiles along skewed rows and along sweeps
@@ -272,7 +273,7 @@ struct Batch {
   int ncell_items = 0, nring_items = 0;
   std::vector<SimDesc> descs;  // what d_sims holds
   // batched Gauss-Seidel layout
-  int tk = 0, blk = 0, gs_n = -1;
+  int tk = 0, asked = 0, blk = 0, gs_n = -1;
   int ntiles = 0, grid = 0;
   std::vector<SimDesc> gs_fields;  // per member: G, KB, rows and its handoff slices
   SolveTile* d_tiles = nullptr;

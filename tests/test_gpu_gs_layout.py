@@ -1,9 +1,12 @@
 """The temporal-blocked solve's layout (its handoff buffers and tile lists) from solve to solve: a
 layout that does not fit the device is an error each time it is asked for, and leaves nothing
 behind: the sweep counts before it run again, bit for bit the oracle's (zero tolerance: the same
-float32 operations in the same order)."""
+float32 operations in the same order). Where only deeper tiles fit, the solve takes those."""
+import contextlib
+
 import numpy as np
 import pytest
+import torch
 
 from fluid_amd import Fluid, FluidBatch
 from oracle.pyoracle import OracleFluid
@@ -65,4 +68,42 @@ def test_batch_layout_that_does_not_fit(graph):
             o.PressureIters = sweeps
             o.update(0.1)
             same(m, o)
+    b.close()
+
+
+@contextlib.contextmanager
+def device_memory_left(bytes_left):
+    """The rest of the device's memory is taken while the block runs."""
+    torch.cuda.empty_cache()
+    hog = [torch.empty(max(0, torch.cuda.mem_get_info()[0] - bytes_left), dtype=torch.uint8, device="cuda")]
+    try:
+        yield
+    finally:
+        hog.clear()
+        torch.cuda.empty_cache()
+
+
+def test_deeper_tiles_where_shallow_ones_do_not_fit():
+    """40 sweeps of a million columns: 12 GB of words in the tiles of 4 sweeps that the size picks,
+    6.9 GB in tiles of 8, 5.1 GB in tiles of 16."""
+    g, o = pair(1, 1000000)
+    b = FluidBatch(1000.0, [(1, 1000000)], 0.01)
+    m, ob = pair(1, 1000000, b.members[0])
+    b.EarlyExit = False
+    g.PressureIters = o.PressureIters = b.PressureIters = ob.PressureIters = 40
+    with device_memory_left(6 << 30):
+        for _ in range(2):
+            g.Simulate(0.1)
+        assert g.gs_layout()["sweeps_per_tile"] > 4
+    for _ in range(2):
+        o.Simulate(0.1)
+    same(g, o)
+    g.close()
+    with device_memory_left(6 << 30):
+        for _ in range(2):
+            b.update(0.1)
+        b.sync()
+    for _ in range(2):
+        ob.update(0.1)
+    same(m, ob)
     b.close()
