@@ -63,7 +63,10 @@
 namespace fl {
 
 static constexpr int LANES = 64;
-static constexpr int SPIN_LIMIT = 1 << 20;     // bounded wait (about a second); then error and continue
+// Bounded wait, in tries of a microsecond or more (several seconds); then error and continue. A wait is
+// short where a tile's producers were handed out before it; with a queue to an XCD it can last as long as the
+// tiles before its producer's take an XCD that other work holds all but a workgroup of (up to 0.1 s at 4096^2).
+static constexpr int SPIN_LIMIT = 1 << 22;
 
 // Tiles whose K streams stay in one XCD's L2 (queue_of_tiles).
 __host__ __device__ constexpr bool near_tiles(int tk) { return tk == 16; }
@@ -615,7 +618,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const uint32_t goword = max(lane - (LANES - B), 0) * GROW + 16 * b0;
     // Ends a wait for words that all carry this solve's tag. Bounded: after SPIN_LIMIT tries, or
     // once another wait of this simulation has expired (err set), err is set and the solve goes
-    // on, so one whose producers stall ends within about a second with FL_ERR_INTERNAL.
+    // on, so one whose producers stall ends within seconds with FL_ERR_INTERNAL.
     auto expired = [&](int it) __attribute__((always_inline)) {
       if (it > SPIN_LIMIT || ((it & 255) == 255 && ld_err(err) != 0)) {
         if (lane == 0) atomicOr(err, 1);
