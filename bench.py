@@ -52,13 +52,14 @@ def build(kind, make, size, iters):
 
 
 def measured_traffic(kind, size, iters):
-    """HBM bytes per GS launch measured with rocprofv3 FETCH_SIZE/WRITE_SIZE for this
-    workload (profiles/hbm_traffic_cavity4096.txt), or None when not measured."""
+    """HBM bytes of one pressure solve (its layout, tile and result kernels) measured with rocprofv3
+    FETCH_SIZE/WRITE_SIZE for this workload (profiles/hbm_traffic_cavity4096.txt), or None when not
+    measured."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic_%s%d.txt" % (kind, size))
     if iters != 200 or not os.path.exists(path):
         return None
     for line in open(path):
-        if line.startswith("k_gs_wave traffic_bytes_per_launch:"):
+        if line.startswith("solve traffic_bytes:"):
             return float(line.split(":")[1])
     return None
 
@@ -517,8 +518,8 @@ def main():
             "traffic": measured_traffic(args.config, args.size, args.iters),
             "kernel": "pressure solve (%d sweeps x 28 B x %d cells per launch)" % (sweeps, cells),
             "note": "achieved counts the algorithmic bytes of a sweep-by-sweep solve; the temporal-blocked "
-                    "kernel moves `traffic` bytes of HBM per launch (rate in hbm_measured) and is bound by its "
-                    "critical path of column steps and tile handoffs, not by HBM"},
+                    "solve moves `traffic` bytes of HBM (rate in hbm_measured) and is bound by its waves' instruction "
+                    "issue and its critical path of column steps and tile handoffs, not by HBM"},
         "early_exit": bool(f.EarlyExit),
         "step_alg_bytes_per_cell": b_alg,
         "step_achieved_GBs": step_gbs,
@@ -539,7 +540,7 @@ def main():
         out["latency_roof"] = latency_roof(f, solve_ms)
     traffic = out["roofline"]["traffic"] if out["roofline"] else None
     if traffic:
-        # the solve's physical HBM traffic (rocprof FETCH_SIZE + WRITE_SIZE per launch, calibrated
+        # the solve's physical HBM traffic (rocprof FETCH_SIZE + WRITE_SIZE per solve, calibrated
         # against a copy kernel) over its live device time: temporal blocking keeps most of the
         # 28 B per cell-sweep on chip, so this is far below the algorithmic rate above
         phys = traffic / (solve_ms * 1e-3) / 1e9
@@ -555,15 +556,32 @@ def main():
     print(json.dumps(out), flush=True)
 
 
-def critical_path_steps(L):
+def tile_waves(tk):
+    """Waves of a tile of tk sweeps: one sweep a wave up to 4, two above."""
+    return tk if tk <= 4 else tk // 2
+
+
+def longest_chain_steps(L):
     """Column steps on the solve's longest chain of dependent tiles, from its tiling (a dict of
-    fl_get_gs_layout). The kernel's wait rule: before running block b a tile stages block b + 1,
-    so it needs its G producer (the tile one row-tile up) to have published row s1 + 64 and its
-    K producer (the tile one sweep-block back) row s1 + TK, s1 being block b + 1's last step.
-    Rows are published in whole blocks (on time: when the next block starts; halfway: BLK/2 steps
-    later; one block late: BLK steps later), which puts a consumer 2 + ceil((L - 1) / BLK) blocks
-    plus that delay behind its producer, L = 64 along the rows and TK along the sweeps. The last
-    tile starts after G - 1 row hops and KB - 1 sweep hops, then runs its own steps."""
+    fl_get_gs_layout), if words arrived as soon as they are stored. Wave w of a tile's W runs its
+    block n (BLK steps) in phase w + n, and at that phase's end has to hold the words of block n + 1:
+    rows up to 62 + 2 BLK of the tile one row-tile up, whose wave w stores a block's rows at the end
+    of its phase, and for wave 0 rows up to TK - 2 + 2 BLK of the tile one sweep block back, whose
+    last wave stores them as it runs. So a tile starts 2 + floor(62 / BLK) blocks behind the first and
+    W + 1 + floor((TK - 2) / BLK) behind the second. The last tile starts after G - 1 row hops and
+    KB - 1 sweep hops and runs its own steps and the W - 1 blocks to its last wave."""
+    tk, blk = L["sweeps_per_tile"], L["cols_per_block"]
+    w = tile_waves(tk)
+    row_hop, sweep_hop = (2 + 62 // blk) * blk, (w + 1 + (tk - 2) // blk) * blk
+    return ((L["row_tiles"] - 1) * row_hop + (L["sweep_blocks"] - 1) * sweep_hop + L["steps_per_tile"] +
+            (w - 1) * blk)
+
+
+def critical_path_steps(L):
+    """The same chain for handoff rows that are published by progress counters, block by block: a tile
+    stages block b + 1 before it runs block b, so it needs row s1 + 64 of the tile one row-tile up and
+    row s1 + TK of the tile one sweep block back, s1 being block b + 1's last step, and rows are
+    published when the next block starts (handoff_lag 1), half a block (3) or a block (2) later."""
     tk, blk, lag = L["sweeps_per_tile"], L["cols_per_block"], L["handoff_lag"]
     delay = {1: 0, 2: blk, 3: blk // 2}[lag]
 
@@ -574,7 +592,8 @@ def critical_path_steps(L):
 
 def column_step_us(L, dt):
     """Wall time of one column step of a tile running alone (no producer to wait for): a 40-row
-    strip 4000 columns long, one tile of the same shape and publication, solved 5 times."""
+    strip 4000 columns long, one tile of the same shape, solved 5 times (with the layout and result
+    kernels, a few percent of it)."""
     import numpy as np
     from fluid_amd import Fluid
     f = Fluid(1000.0, 40, 4000, 0.01)
@@ -585,7 +604,7 @@ def column_step_us(L, dt):
     st["S"] = S
     f.load_state(st)
     f.EarlyExit = False
-    f.BlockSweeps, f.BlockCols, f.HandoffLag = L["sweeps_per_tile"], L["cols_per_block"], L["handoff_lag"]
+    f.BlockSweeps, f.BlockCols = L["sweeps_per_tile"], L["cols_per_block"]
     tk = L["sweeps_per_tile"]
     for _ in range(2):
         f.run_pass("makeIncompressible", dt, tk)
@@ -598,11 +617,11 @@ def column_step_us(L, dt):
     one = f.gs_layout()
     f.close()
     assert one["tiles"] == 1, one
-    return 1e6 * per_solve / one["steps_per_tile"]
+    return 1e6 * per_solve / longest_chain_steps(one)
 
 
 def latency_roof(f, solve_ms):
-    """The temporal-blocked solve's latency bound: its critical path of column steps times the
+    """The temporal-blocked solve's latency bound: its longest chain of column steps times the
     measured cost of one column step of a lone tile. `frac` is that bound over the solve's
     measured time (how far the solve is from running at the speed of its longest chain)."""
     from fluid_amd import configs as C
@@ -610,16 +629,15 @@ def latency_roof(f, solve_ms):
         L = f.gs_layout()
     except Exception:
         return None
-    steps = critical_path_steps(L)
+    steps = longest_chain_steps(L)
     us = column_step_us(L, C.DT)
     ms = steps * us * 1e-3
     return {"critical_path_steps": steps, "column_step_us": us, "ms": ms, "frac": ms / solve_ms,
-            "shape": "%d sweeps x %d columns per tile block, %s publication, %d tiles on %d workgroups" % (
-                L["sweeps_per_tile"], L["cols_per_block"], {1: "on-time", 2: "one-block-late", 3: "halfway"}[
-                    L["handoff_lag"]], L["tiles"], L["workgroups"]),
+            "shape": "%d sweeps x %d columns per tile block, %d tiles on %d workgroups" % (
+                L["sweeps_per_tile"], L["cols_per_block"], L["tiles"], L["workgroups"]),
             "note": "column_step_us is measured on a single tile (a 40x4000 strip, whose edge waves take "
-                    "the general update); the rest of frac is time tiles spend in the pipeline's fill and "
-                    "drain, waiting on producers and sharing CUs"}
+                    "the general update); the rest of frac is the words' way through memory, more tiles than "
+                    "workgroups, and the layout and result kernels"}
 
 
 def metric_extras(args):
