@@ -71,6 +71,10 @@ static constexpr int SPIN_LIMIT = 1 << 22;
 // Tiles whose K streams stay in one XCD's L2 (queue_of_tiles).
 __host__ __device__ constexpr bool near_tiles(int tk) { return tk == 16; }
 static constexpr int MAXQ = 16;  // queues of tiles, one per XCD
+// Blocks after which a tile's buffers begin anew (even: the waves take two blocks a turn). Beginning them anew for
+// every block cost 0.5% to 1% on small grids (a step of 256^2 0.1516 -> 0.1523 ms, 300x251 0.1140 -> 0.1152).
+static constexpr int SEGMENT = 1 << 16;
+__host__ __device__ constexpr int segment_rows(int blk) { return SEGMENT * blk + 4 * LANES; }  // with those read ahead
 // The counters of one launch (main run or re-run), zero before it.
 struct GsCounters {
   int32_t ticket[MAXQ + 1];  // of each XCD's queue, and of all tiles in one
@@ -114,7 +118,7 @@ __device__ __forceinline__ bool tile_empty(int g, int kb, int K, int TK, int NX)
 // have to arrive whole. Words are written once per solve, so the tag they hold before is that of one of the
 // last solves. Device-coherent accesses (sc1), so that neither side needs a cache writeback or
 // invalidate. The intrinsics' offsets are 32 bits and a tile's K rows 1 KB each, so a buffer begins
-// at the rows of a block (or of a layout item), and its offsets stay within those.
+// at the rows of a stretch of SEGMENT blocks (or of a layout item), and its offsets stay within those.
 typedef uint32_t word4 __attribute__((ext_vector_type(4)));
 static constexpr int CACHED = 0, SC1 = 16, VOLATILE_OP = (int)0x80000000;  // cache policy of the buffer intrinsics
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t word_buffer(const void* p) {
@@ -171,6 +175,11 @@ __device__ __forceinline__ float from_lane_above(float last, float v) {
 }
 __device__ __forceinline__ bool every_lane(bool v) { return __builtin_amdgcn_ballot_w64(!v) == 0; }
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T> __device__ __forceinline__ T* uniform(T* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = uniform((int)v), hi = uniform((int)(v >> 32));
+  return reinterpret_cast<T*>((uint64_t)hi << 32 | lo);
+}
 __device__ __forceinline__ float uniform(float v) { return __int_as_float(uniform(__float_as_int(v))); }
 
 typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // four floats at any word address
@@ -553,7 +562,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const SolveTile te = R.tiles[t];
     const int sim = te.sim, g = te.g, kb = te.kb;
     const SimDesc& D = sim_desc(m, sim);
-    const int NX = D.g.NX, NY = D.g.NY, rows = D.rows, KB = D.KB;
+    const int NX = D.g.NX, NY = D.g.NY, rows = D.rows;
     const int nblk = rows / B;
     int32_t* err = D.ctrl + 3;
     const int K = !R.which ? R.K : std::is_same<M, OneSim>::value ? again : D.ctrl[1];
@@ -571,15 +580,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const bool hG = g > 0 && !tile_empty(g - 1, kb, Kp, TK, NX);
     const bool hK = kb == 0 || !tile_empty(g, kb - 1, Kp, TK, NX);
     const bool hC = g > 0 && (kb == 0 || !tile_empty(g - 1, kb - 1, Kp, TK, NX));
-    // The G stream has a column of tiles before the first for the initial state (k_gs_skew), so the
-    // corner's words lie a tile before the G stream's.
-    const size_t gtile = (size_t)rows * GROW, ktile = (size_t)rows * KROW, itile = (size_t)(rows + 1) * KROW;
-    uint8_t* const kmine = D.kout + (size_t)(g * KB + kb) * ktile;
-    uint8_t* const gmine = D.gout + (size_t)(g * (KB + 1) + kb + 1) * gtile;
-    const uint8_t* const gprod = D.gout + (g > 0 ? (size_t)((g - 1) * (KB + 1) + kb) * gtile : 0);
-    const uint8_t* ksrc = kb ? D.kout + (size_t)(kb - 1) * ktile : D.kinit;  // of row-tile 0
-    const size_t kstep = kb ? KB * ktile : itile;                            // to the next row-tile
-    const uint8_t* const kprod = ksrc + (hK ? g * kstep : 0);
+    const size_t gtile = (size_t)rows * GROW;
     const uint32_t ktag = kb ? tag : tag0;
     const int kfirst = kb ? TK - 1 : 0, klast = kb ? rows - 1 : rows;  // row of step 0, last row
 
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
     const int gu = lane / (S + 1), gx = lane - gu * (S + 1);
     const bool gcorner = w == 0 && gx == 0, gstage = gu < B;
     const uint32_t gat = gcorner ? 16 * (TK - 1) : (uint32_t)gtile + 16 * (b0 - 1 + gx);  // (words_fit)
-    const int grow = gcorner ? gu + LANES + kfirst : gu + LANES - 1;  // row of a block's word, from the block's first
+    const uint32_t goff = gat + (gcorner ? gu + LANES + kfirst : gu + LANES - 1) * GROW;
     const uint32_t gtag = gcorner ? ktag : tag, gneed = gstage && (gcorner ? hC : hG) ? ~0u : 0u, kneed = hK ? ~0u : 0u;
     lds_float* const gdst = (lds_float*)&sh.Gi[w][min(gu, B - 1) + 1][3 * gx];
     const bool gout = g_wave && lane >= LANES - B;  // stores lane 63's words of step lane - (64 - B)
@@ -639,13 +640,36 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
         uint32_t mw[S];
         word4 gw, kw[FIRST ? B : 1];
       };
+      // The buffers of a stretch of blocks that begins with block `from`. Below, n counts from there. (The
+      // tile is looked up again, so that no base takes scalar registers from the blocks: they spilled, 256^2
+      // 0.1516 -> 0.1535 ms. In a batch the addresses come from vector loads: uniform() spares a loop over the lanes
+      // at every access, a step of 6 grids 0.329 -> 0.246 ms, of 48 2.92 -> 2.58.)
+      // The G stream has a column of tiles before the first for the initial state (k_gs_skew), so the
+      // corner's words lie a tile before the G stream's.
+      __amdgpu_buffer_rsrc_t kmine, gmine, gprod, kprod;
+      int nleft, klastn;  // blocks from there to the tile's end, last K row
+      uint32_t glast;
+      auto begin_at = [&](int from) __attribute__((always_inline)) {
+        const SolveTile te = R.tiles[uniform(sh.tile)];
+        const SimDesc& D = sim_desc(m, te.sim);
+        const int KB = D.KB, g = te.g, kb = te.kb, row = from * B;
+        const size_t ktile = (size_t)rows * KROW, itile = (size_t)(rows + 1) * KROW;
+        const uint8_t* ksrc = kb ? D.kout + (size_t)(kb - 1) * ktile : D.kinit;  // of row-tile 0
+        const size_t kstep = kb ? KB * ktile : itile;                            // to the next row-tile
+        kmine = word_buffer(uniform(D.kout + (size_t)(g * KB + kb) * ktile + (size_t)row * KROW));
+        gmine = word_buffer(uniform(D.gout + (size_t)(g * (KB + 1) + kb + 1) * gtile + (size_t)row * GROW));
+        gprod = word_buffer(uniform(D.gout + (size_t)(max(g - 1, 0) * (KB + 1) + (g > 0 ? kb : 0)) * gtile + (size_t)row * GROW));
+        kprod = word_buffer(uniform(ksrc + g * kstep + (size_t)row * KROW));
+        nleft = nblk - from;
+        klastn = min(klast - row, segment_rows(B));
+        glast = gat + min(rows - 1 - row, segment_rows(B)) * GROW;
+      };
       auto load_g = [&](Block& x, int n) __attribute__((always_inline)) {
-        x.gw = ld_word(word_buffer(gprod + (size_t)n * (B * GROW)), gat + (uint32_t)min(grow, rows - 1 - n * B) * GROW);
+        x.gw = ld_word(gprod, min(goff + n * (B * GROW), glast));
       };
       auto load_k = [&](Block& x, int n, int u) __attribute__((always_inline)) {
-        const int r = min(n * B + kfirst, klast);  // the block's first row, or the last of all
-        x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(word_buffer(kprod + (size_t)r * KROW), 16 * lane,
-                                                        min(u, klast - r) * KROW, SC1 | VOLATILE_OP);
+        x.kw[u] = __builtin_amdgcn_raw_buffer_load_b128(kprod, 16 * lane, min(n * B + u + kfirst, klastn) * KROW,
+                                                        SC1 | VOLATILE_OP);
       };
       auto load = [&](Block& x, int n) __attribute__((always_inline)) {
 #pragma unroll
@@ -716,7 +740,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       auto run = [&](const Block& x, int n) __attribute__((always_inline)) {
         const float4* Kin = FIRST ? nullptr : &sh.K[w - 1][n & 1][0][lane];
         float4* Kout = OUT != OUT_LDS ? nullptr : &sh.K[w][n & 1][0][lane];
-        const __amdgpu_buffer_rsrc_t kbuf = word_buffer(kmine + (size_t)n * (B * KROW));
+        const uint32_t kbyte = (uint32_t)n * (B * KROW) + 16 * lane;
         bool plain = true, same = true;
 #pragma unroll
         for (int c = 0; c < S; c++) {
@@ -724,7 +748,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
           same = same && mk[c] == (mk[c] & 0xFu) * (BITS / 0xFu);
         }
 #define FL_RUN(MODE) \
-  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kbuf, 16 * lane, tag, damping, cp)
+  run_block<SOLVE, S, B, GP, MODE, FIRST, OUT, FULL, ROW63>(Q, x.kw, k, mk, gi, Kin, Kout, go, tab, kmine, kbyte, tag, damping, cp)
         if (!FULL && every_lane(plain)) {
           FL_RUN(BLOCK_PLAIN);
         } else if (every_lane(same)) {
@@ -745,31 +769,38 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       // memory operations complete in order, and a wait behind a store would last as long as the
       // store's way to memory.
       auto phase = [&](const Block& x, Block& next, int n) __attribute__((always_inline)) {
-        const int n1 = min(n + 1, nblk - 1);
+        const int n1 = min(n + 1, nleft - 1);
         load(next, n1);
         run(x, n);
         stage(next, n1);
         if (gout) {
-          const __amdgpu_buffer_rsrc_t gbuf = word_buffer(gmine + (size_t)n * (B * GROW));
 #pragma unroll
           for (int c = 0; c < S; c++)
-            st_word<SC1>(gbuf, goword + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
+            st_word<SC1>(gmine, goword + n * (B * GROW) + 16 * c, go[c][SOLVE == SOLVE_GS ? 0 : 2], go[c][1], go[c][2], tag);
         }
         __syncthreads();
       };
       Block x, y;
+      begin_at(0);
       load(x, 0);
       stage(x, 0);
       __syncthreads();
-      if constexpr (FIRST) {  // two blocks to a turn, so that their words stay where they were loaded
-        for (int n = 0;;) {
-          phase(x, y, n);
-          if (++n == nblk) break;
-          phase(y, x, n);
-          if (++n == nblk) break;
+      for (int from = 0;;) {
+        const int end = min(nleft, SEGMENT);
+        if constexpr (FIRST) {  // two blocks to a turn, so that their words stay where they were loaded
+          for (int n = 0;;) {
+            phase(x, y, n);
+            if (++n == end) break;
+            phase(y, x, n);
+            if (++n == end) break;
+          }
+        } else {
+          for (int n = 0; n < end; n++) phase(x, x, n);
         }
-      } else {
-        for (int n = 0; n < nblk; n++) phase(x, x, n);
+        if ((from += SEGMENT) >= nblk) break;
+        begin_at(from);
+#pragma unroll
+        for (int c = 0; c < S; c++) mcol[c] += SEGMENT * B / 2;
       }
       for (int p = w + 1; p < W; p++) __syncthreads();
     };
@@ -1024,15 +1055,15 @@ static TileGeom geom(int NX, int NY, int N, int tk, int blk) {
   return t;
 }
 // A wave loads its G words from its producer's tile and the corner tile before it in one instruction,
-// so their offset from a block's row of the corner tile spans one tile of `rows` rows and the 64 + tk +
-// blk rows that a tile lags, and has to stay below 2^32. With one row-tile the words are not used.
-static bool words_fit(const TileGeom& t, int tk) {
-  return t.G == 1 || ((uint64_t)t.rows + 2 * LANES) * (16 * tk) < (uint64_t)1 << 32;
+// so their offsets span one tile of `rows` rows and a stretch of SEGMENT blocks, and have to stay
+// below 2^32. With one row-tile the words are not used.
+static bool words_fit(const TileGeom& t, int tk, int blk) {
+  return t.G == 1 || ((uint64_t)t.rows + segment_rows(blk)) * (16 * tk) < (uint64_t)1 << 32;
 }
-// The depth to use where tiles of tk sweeps are too long for that (16.7 million columns with 16):
+// The depth to use where tiles of tk sweeps are too long for that (16.2 million columns with 16):
 // shallower ones, whose G rows are smaller.
 static int shallow_enough(int NX, int NY, int N, int tk, int blk) {
-  while (tk > 2 && !words_fit(geom(NX, NY, N, tk, blk), tk)) tk /= 2;
+  while (tk > 2 && !words_fit(geom(NX, NY, N, tk, blk), tk, blk)) tk /= 2;
   return tk;
 }
 // Tiles are handed out in the order their producers let them start: a consumer loads a block
@@ -1203,7 +1234,7 @@ static int layout(GsWork& W, Ctx* c, int NX, int NY, int N, int tk, int deepest,
   if (W.n_alloc == N && W.asked == tk && W.blk == blk) return FL_OK;
   FL_HIP(hipStreamSynchronize(c->stream));  // earlier solves may still use the old layout
   int rc = FL_OK;
-  for (int t = tk; t == tk || (t <= deepest && words_fit(geom(NX, NY, N, t, blk), t)); t *= 2) {
+  for (int t = tk; t == tk || (t <= deepest && words_fit(geom(NX, NY, N, t, blk), t, blk)); t *= 2) {
     free_work(W);
     if ((rc = plan(W, c, NX, NY, N, t, blk)) == FL_OK) {
       W.n_alloc = N;
@@ -1436,7 +1467,7 @@ int batch_gs_layout(Batch* B, int N, std::vector<SimDesc>& descs) {
   int rc = FL_OK;
   auto fits = [&](int t) {
     for (const SimDesc& d : descs)
-      if (!words_fit(geom(d.g.NX, d.g.NY, N, t, blk), t)) return false;
+      if (!words_fit(geom(d.g.NX, d.g.NY, N, t, blk), t, blk)) return false;
     return true;
   };
   for (int t = tk; t == tk || (t <= (tk_knob(B->prm) ? 0 : 16) && fits(t)); t *= 2) {  // as in layout()

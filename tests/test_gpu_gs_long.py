@@ -1,6 +1,6 @@
 """The temporal-blocked solve on grids at the lengths where its handoff words pass 4 GB, bit for bit
 against the oracle. A tile of 64 rows writes 1 KB of words a column, so its words lie beyond
-32-bit byte offsets from column 2^22 on: one row-tile with three blocks of sweeps, two row-tiles
+32-bit byte offsets from column 2^22 on, and its buffers begin anew after every 2^16 blocks of columns: one row-tile with three blocks of sweeps, two row-tiles
 (63 sweeps on one interior row), a batch member, and the other way round a grid of more than
 2^15 row-tiles. The tolerance is zero: the oracle's float32 operations in the oracle's order."""
 import numpy as np
@@ -31,11 +31,12 @@ def compare(g, o):
         assert not bad.any(), "%s differs at %d cells, first %s" % (k, int(bad.sum()), np.argwhere(bad)[0])
 
 
-@pytest.mark.parametrize("w,h,sweeps,tk", [(1, LONG, 5, 2), (1, LONG, 63, 16), (64 * ((1 << 15) + 3), 1, 5, 0)])
-def test_long_grids_bit_exact(w, h, sweeps, tk):
+@pytest.mark.parametrize("w,h,sweeps,tk,blk", [(1, LONG, 5, 2, 8), (1, LONG, 63, 16, 8), (64 * ((1 << 15) + 3), 1, 5, 0, 8),
+                                               (63, (1 << 18) - 70, 21, 8, 4), (3, (1 << 19) + 1, 64, 4, 8)])
+def test_long_grids_bit_exact(w, h, sweeps, tk, blk):
     st = state(w, h)
     g, o = Fluid(1000.0, w, h, 0.01), OracleFluid(1000.0, w, h, 0.01, threads=8)
-    g.Solver, g.BlockSweeps = 2, tk
+    g.Solver, g.BlockSweeps, g.BlockCols = 2, tk, blk
     for f in (g, o):
         f.load_state(st)
         f.PressureIters, f.EarlyExit = sweeps, False
