@@ -411,7 +411,7 @@ def main():
     ap.add_argument("--iters", type=int, default=200)
     ap.add_argument("--solver", type=int, default=0)
     ap.add_argument("--block-sweeps", type=int, default=0)
-    ap.add_argument("--handoff-lag", type=int, default=0, help="0 auto, 1 on time, 2 one block late")
+    ap.add_argument("--handoff-lag", type=int, default=0, help="accepted (0 to 3); all values run alike")
     ap.add_argument("--precise", action="store_true",
                     help="PreciseAdvection: back-trace in cell units (an addition; default is the reference's arithmetic)")
     ap.add_argument("--multigrid", action="store_true",

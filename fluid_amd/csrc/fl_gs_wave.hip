@@ -32,18 +32,19 @@
 // of the solve, in each half, and the consumer loads the words until they carry the tag of this
 // solve. So a handoff costs one trip of the data: no wait for stores, no progress counters, no
 // polls beside the loads themselves. A block's words are loaded while the block before it runs.
-// The compiler has to know
-// how many stores were issued since a load to wait for the load alone, so every path of a block issues
-// the same loads and stores, under branches that it sees are uniform
-// (with a wait for the stores 256^2 took 0.180 ms, 512^2 0.540). Tiles run as a persistent kernel in ticket order (a topological order of the tile graph), so
-// whatever a workgroup waits for was taken earlier by a workgroup that runs. k_gs_skew lays the
-// initial state out as K-stream words and k_gs_unskew takes the last sweep's back, so tiles
-// read and write nothing but words, whole lines at a time.
+// The compiler has to know how many stores were issued since a load to wait for the load alone, so
+// every path of a block issues the same loads and stores, under branches that it sees are uniform
+// (with a wait for the stores 256^2 took 0.180 ms a solve, 512^2 0.540). Tiles run as a persistent
+// kernel in ticket order (a topological order of the tile graph), so whatever a workgroup waits for was
+// taken earlier by a workgroup that runs, or (queue_of_tiles) will be by one that has started.
+// k_gs_skew lays the initial state out as K-stream words and k_gs_unskew takes the last sweep's back,
+// so tiles read and write nothing but words, whole lines at a time.
 //
-// What a solve measured, one sweep a wave with a barrier a step -> now: 256^2 40 sweeps 0.49 -> 0.136 ms,
-// 300x251 8 sweeps 0.42 -> 0.095, 512^2 200 sweeps 1.32 -> 0.454, 4096^2 200 sweeps 10.5 -> 4.96.
-// At 4096^2 the two waves of a SIMD are bound by their issue: 43 instructions a step of two
-// sweeps, 34 of them the shifts and updates.
+// What a solve with these two kernels measured (events around it), one sweep a wave with a barrier a
+// step -> now: 256^2 40 sweeps 0.49 -> 0.140 ms, 300x251 8 sweeps 0.42 -> 0.097, 512^2 200 sweeps 1.32 ->
+// 0.451, 4096^2 200 sweeps 10.5 -> 4.97 (k_gs_wave alone 0.122, 0.078, 0.437, 4.73). At 4096^2 the two
+// waves of a SIMD are bound by their issue: 53 issue slots of 4 cycles a step of two sweeps, 40 of them
+// vector instructions (34 the shifts and updates).
 //
 // Cells outside the interior or solid pass their faces through unchanged, exactly like
 // the skipped cells of the serial loop. Faces no interior cell touches keep their input
@@ -483,8 +484,8 @@ __device__ __forceinline__ void run_block(Sweeps<S>& Q, const word4 (&kw)[FIRST 
 
 // The queue a workgroup takes its tiles from (called by one thread of it). A row-tile's tiles are
 // all in the queue of one XCD, so that their K streams, one 1 KB row a step each, stay in that XCD's
-// L2 (OUT_CACHED; written through to memory the 4096^2 solve of 200 sweeps takes 5.70 ms against 4.98,
-// 2048^2 1.96 against 1.71). Only for tiles of 16 sweeps, which make more rows than XCDs: on small
+// L2 (OUT_CACHED; written through to memory the 4096^2 solve of 200 sweeps takes 5.74 ms against 4.97,
+// 2048^2 2.04 against 1.70). Only for tiles of 16 sweeps, which make more rows than XCDs: on small
 // grids whole rows divide unevenly (512^2 0.530 ms against 0.475). A workgroup serves the XCD that it
 // runs on. Each queue needs a workgroup, or tiles would wait for ever for those of a queue without
 // one, so the first workgroups wait until one has started on every XCD (a few microseconds). If that
@@ -728,7 +729,7 @@ __global__ __launch_bounds__(W* LANES, W > 4 ? 2 : 1) void k_gs_wave(M m, GsRun 
       };
       float go[S][3];
       // The last sweep's V and p of lane 63 are in the rows that the wave left in LDS: the last B lanes
-      // read them there after the block, two shifts a step less (256^2 a solve 123 -> 120 us, 512^2 200
+      // read them there after the block, two shifts a step less (256^2 the kernel 123 -> 120 us, 512^2 200
       // sweeps 444 -> 436, 2048x1024 861 -> 842). Not in tiles of 16 sweeps, which lose (4096^2 4.74 ->
       // 4.79 ms).
       constexpr bool ROW63 = OUT == OUT_LDS && !NEAR;
@@ -1030,8 +1031,8 @@ static bool tile_empty_h(int g, int kb, int K, int TK, int NX) {
 }
 
 // Waves per workgroup of a tile of tk sweeps: two sweeps to a wave; one in the small tiles, whose
-// few waves leave the CU's issue slots free (4 sweeps, 256^2 jet: 0.154 ms against 0.175 with two
-// waves of two; 300x251 0.110 against 0.136). Four to a wave lost everywhere (2048^2 2.35 ms
+// few waves leave the CU's issue slots free (measured before the layout kernels were shortened: 4
+// sweeps, 256^2 jet 0.154 ms a solve against 0.175 with two waves of two; 300x251 0.110 against 0.136). Four to a wave lost everywhere (2048^2 2.35 ms
 // against 1.72 at 16 sweeps, 2048x1024 1.55 against 1.09 at 8).
 static int tile_waves(int tk) { return tk <= 4 ? tk : tk / 2; }
 static int tile_sweeps(int tk) { return tk / tile_waves(tk); }  // sweeps per wave
@@ -1130,12 +1131,13 @@ static long long tiles_in_flight(int NX, int NY, int N, int tk) {
 // Sweeps per tile for the number of tiles in flight by their depth: the smallest tile of which
 // there is no more than one per CU. Small tiles spread a small grid over the CUs and
 // step faster; once there are more of them than CUs, large ones hand over less and take fewer
-// turns. Solve times in ms with 4, 8, 16 sweeps: 300x251 8 sweeps 0.110 0.142 0.146; 256^2 40 sweeps
-// 0.154 0.174 0.227; 777x391 33 sweeps 0.239 0.307 0.415; 1024^2 40 sweeps (140 in flight with 4)
-// 0.366 0.457 0.625; 1024^2 100 sweeps (350 with 4, 182 with 8) 0.633 0.585 0.734; 512^2 200 sweeps
-// (400, 200) 0.510 0.473 0.636; 2048x1024 100 sweeps (350, 182) 1.012 0.928 1.054; 4096^2 40 sweeps
-// (265 with 8) 3.12 2.90 2.51; 2048^2 200 sweeps (675) 2.83 2.10 1.72; 4096^2 200 sweeps 10.2 6.6 5.0.
-// Two sweeps (the knob takes them) gain nothing on 4: 300x251 0.111, 256^2 0.161.
+// turns. Solve times in ms with 4, 8, 16 sweeps: 300x251 8 sweeps 0.097 0.127 0.132; 256^2 40 sweeps
+// 0.140 0.158 0.207; 777x391 33 sweeps 0.224 0.285 0.389; 1024^2 40 sweeps (140 in flight with 4)
+// 0.363 0.444 0.615; 1024^2 100 sweeps (350 with 4, 182 with 8) 0.618 0.599 0.717; 512^2 200 sweeps
+// (400, 200) 0.474 0.451 0.598; 2048x1024 100 sweeps (350, 182) 1.010 0.945 1.033; 4096^2 40 sweeps
+// (265 with 8) 3.20 2.77 2.43; 2048^2 200 sweeps (675) 2.79 2.05 1.68; 4096^2 200 sweeps 10.2 6.5 5.0.
+// Two sweeps (the knob takes them) gain at most 0.004 ms on 4 and lose from 1024^2 on: 300x251 0.093, 256^2
+// 0.142, 777x391 0.218, 1024^2 40 sweeps 0.432.
 template <class F> static int depth_for(F in_flight) { return in_flight(4) <= 256 ? 4 : in_flight(8) <= 256 ? 8 : 16; }
 static bool tk_knob(const fl_params& P) {
   return P.block_sweeps == 2 || P.block_sweeps == 4 || P.block_sweeps == 8 || P.block_sweeps == 16;
@@ -1145,7 +1147,7 @@ int pick_tk(const fl_params& P, int NX, int NY, int N) {
   return shallow_enough(NX, NY, N, tk, pick_blk(P));
 }
 // Columns per block: 4 with the knob, else 8, which won at every size (4096^2 200 sweeps 5.0 ms
-// against 7.1, 256^2 0.154 against 0.163). 16, which the knob also takes, would not fit in LDS.
+// against 7.0, 256^2 0.140 against 0.151). 16, which the knob also takes, would not fit in LDS.
 int pick_blk(const fl_params& P) { return P.block_cols == 4 ? 4 : 8; }
 // The update that leaves inactive cells alone by the signs of zeros needs these; any other
 // parameters take the FULL kernels.

@@ -126,10 +126,10 @@ struct GsWork {
   int ntiles = 0;          // non-empty tiles
   int nq = 0;              // queues they are handed out from
   int grid = 0;            // persistent workgroups launched
-  int lag = 0;             // handoff_lag of the last solve (0: none yet)
+  int lag = 0;             // handoff_lag of the last solve (reported only; 0: none yet)
   SolveTile* d_tile = nullptr;    // [2 ntiles] in ticket order by queue and of all
   uint8_t* d_kout = nullptr;    // [G*KB][rows][64] K-stream handoff words
-  uint8_t* d_gout = nullptr;    // [G*KB][rows][tk] G-stream handoff words
+  uint8_t* d_gout = nullptr;    // [G*(KB + 1)][rows][tk] G-stream handoff words (the first column: the initial state)
   uint8_t* d_kinit = nullptr;   // [G][rows + 1][64] the initial state as K-stream words
   int* d_first = nullptr;       // where each queue's tiles begin
   GsState* d_state = nullptr;

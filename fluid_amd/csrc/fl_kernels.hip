@@ -117,8 +117,6 @@ template <class M> __global__ void k_copy_role(M m, int rdst, int rsrc) {
 }
 
 // ---- cell flags (from S, which holds exactly 0.0 or 1.0) ------------------------------
-// The anti-diagonal copy is written only at grid cells; its other entries stay zero from
-// allocation.
 template <class M> __global__ void k_flags(M m) {
   const SimDesc* d;
   int i, j;

@@ -155,8 +155,8 @@ class Fluid:
         check(self._L.fl_set_params(self._ctx, ctypes.byref(p)))
 
     def autotune(self, dt):
-        """Time the candidate Gauss-Seidel tile shapes (sweeps per tile, columns per block,
-        handoff lag) on the current state; keep the fastest. Returns (sweeps per tile, ms)."""
+        """Time the candidate Gauss-Seidel tile shapes (sweeps per tile, columns per block)
+        on the current state; keep the fastest. Returns (sweeps per tile, ms)."""
         self._push()
         tk, ms = ctypes.c_int(), ctypes.c_float()
         check(self._L.fl_autotune(self._ctx, dt, ctypes.byref(tk), ctypes.byref(ms)))

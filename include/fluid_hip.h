@@ -137,7 +137,7 @@ int fl_sweep_maxdiv(fl_ctx* ctx, float* out, int cap, int* count);
  * the critical-path model of the solve's time. FL_ERR_INVALID_ARG before the first such solve. */
 typedef struct fl_gs_layout {
   int32_t sweeps_per_tile;  /* TK */
-  int32_t cols_per_block;   /* BLK: columns per staging and publication block */
+  int32_t cols_per_block;   /* BLK: columns between two barriers of a workgroup */
   int32_t handoff_lag;      /* params.handoff_lag of the last solve, 1 if auto */
   int32_t row_tiles;        /* G: tiles along the skewed rows (64 rows each) */
   int32_t sweep_blocks;     /* KB: tiles along the sweeps */
