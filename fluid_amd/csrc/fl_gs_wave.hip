@@ -1547,11 +1547,13 @@ static int set_solve_number(hipStream_t stream, GsState* state, int number) {
 }
 extern "C" int fl_test_solve(fl_ctx* ctx, int far, int number) {
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
+  if (!c) return FL_ERR_INVALID_ARG;
   c->gs_far = far != 0;
   return set_solve_number(c->stream, c->gs.d_state, number);
 }
 extern "C" int fl_test_batch_solve(fl_batch* b, int far, int number) {
   Batch* B = reinterpret_cast<Batch*>(b);
+  if (!B) return FL_ERR_INVALID_ARG;
   B->gs_far = far != 0;
   B->graph_gen++;
   return set_solve_number(B->stream, B->state, number);
