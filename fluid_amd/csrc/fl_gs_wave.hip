@@ -1032,8 +1032,9 @@ static bool tile_empty_h(int g, int kb, int K, int TK, int NX) {
 
 // Waves per workgroup of a tile of tk sweeps: two sweeps to a wave; one in the small tiles, whose
 // few waves leave the CU's issue slots free (measured before the layout kernels were shortened: 4
-// sweeps, 256^2 jet 0.154 ms a solve against 0.175 with two waves of two; 300x251 0.110 against 0.136). Four to a wave lost everywhere (2048^2 2.35 ms
-// against 1.72 at 16 sweeps, 2048x1024 1.55 against 1.09 at 8).
+// sweeps, 256^2 jet 0.154 ms a solve against 0.175 with two waves of two; 300x251 0.110 against
+// 0.136). Four to a wave lost everywhere (2048^2 2.35 ms against 1.72 at 16 sweeps, 2048x1024 1.55
+// against 1.09 at 8).
 static int tile_waves(int tk) { return tk <= 4 ? tk : tk / 2; }
 static int tile_sweeps(int tk) { return tk / tile_waves(tk); }  // sweeps per wave
 // N sweeps with those that only fill the last wave: their cells pass their faces on.
